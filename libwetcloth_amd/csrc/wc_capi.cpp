@@ -135,6 +135,7 @@ void release_all(wc_ctx* c) {
   c->b.release();
   c->p.release();
   c->dof_level.release();
+  c->dof_live.release();
   c->pcg.release();
   c->amg.release();
   c->dof_ijk.release();
@@ -192,6 +193,7 @@ bool solve_system(wc_ctx* c, double tol, int maxit, double* res, int* it) {
   gs.dofscan = c->dofscan.p;
   gs.rowlen = c->rowlen.p;
   gs.col = c->col.p;
+  gs.live = c->dof_live.p;
   bool ok;
   if (c->solver == 1 && A.n > 0) {
     wc::pcg_prepare_vectors(c->stream, c->pcg, A.n);
@@ -940,6 +942,8 @@ wc_status wc_apply_preconditioner(wc_ctx* c, const double* r, double* z) {
     if (P.valid) {
       wc::box_gather(c->stream, P, dr.p, P.rb.p);
       wc::sweep_apply(c->stream, P, P.rb.p, nullptr, n);
+      // DOFs outside the box have empty rows: zero
+      WC_HIP(hipMemsetAsync(dz.p, 0, sizeof(double) * n, c->stream));
       wc::box_scatter(c->stream, P, P.zb.p, dz.p);
     } else {
       wc::pcg_apply(c->stream, c->pcg, system_csr(c), dr.p, dz.p);
@@ -970,6 +974,7 @@ wc_status wc_system_multiply(wc_ctx* c, const double* x, double* y) {
     if (P.valid) {
       wc::box_gather(c->stream, P, dx.p, P.sb.p);
       wc::box_spmv(c->stream, P, P.sb.p, P.zb.p);
+      WC_HIP(hipMemsetAsync(dy.p, 0, sizeof(double) * n, c->stream));
       wc::box_scatter(c->stream, P, P.zb.p, dy.p);
     } else {
       wc::pcg_spmv(c->stream, system_csr(c), dx.p, dy.p);

@@ -134,6 +134,10 @@ struct SweepPlan {
   DevBuf<double> bb;
   DevBuf<int> progress, flags;
   DevBuf<double> tdot;              // per-unit z . r partials of the last apply
+  // the sub-tile sweeps' exchange records, forward then backward; mail_word:
+  // size of the value type they stand ready for (0: to be filled first)
+  DevBuf<double> mail;
+  int mail_word = 0;
   int ndot = 0;                     // how many (tiles, or sub-tiles)
   // Sub-tile sweeps (one wave per 8x8 quarter of a tile, k_sweep_sub) or
   // the tile sweeps (k_sweep); both give the same values bit for bit

@@ -229,6 +229,7 @@ struct AsmArgs {
   double* val;
   double* b;
   int32_t* level;
+  uint8_t* live;  // the row holds a nonzero value
   int32_t level_min;
   double dt;
   FrozenView F;
@@ -326,10 +327,13 @@ __global__ void k_assemble(AsmArgs A) {
   }
   A.b[me] = rhs;
   A.rowlen[me] = (uint32_t)len;
+  bool live = false;
   for (int t = 0; t < len; ++t) {
     A.col[7 * (int64_t)me + t] = cols[t];
     A.val[7 * (int64_t)me + t] = vals[t];
+    live = live || vals[t] != 0;
   }
+  A.live[me] = live;
   A.level[me] = i + j + k - A.level_min;
 }
 
@@ -555,6 +559,7 @@ int64_t grid_assemble(wc_ctx* ctx, double dt) {
   ctx->b.ensure(ndof);
   ctx->p.ensure(ndof);
   ctx->dof_level.ensure(ndof);
+  ctx->dof_live.ensure(ndof);
   ctx->level_min = 0;
   ctx->level_max = g.nx[0] + g.nx[1] + g.nx[2];
   if (ndof > 0) {
@@ -576,6 +581,7 @@ int64_t grid_assemble(wc_ctx* ctx, double dt) {
     A.val = ctx->val.p;
     A.b = ctx->b.p;
     A.level = ctx->dof_level.p;
+    A.live = ctx->dof_live.p;
     A.level_min = ctx->level_min;
     A.dt = dt;
     A.F = frozen_view(ctx);

@@ -352,9 +352,9 @@ __global__ void k_update_s(V* s, const V* z, int64_t n, const double* scal) {
 
 // x += s alpha, r -= z alpha (FP64 r and z, or FP32 formed in FP64), |r|_inf
 // block partials into rpart (mapped host memory, which the host polls; the
-// sweeps' abort flag rides in block 0's entry); and the next forward
-// sweep's output set to the all-ones sentinel (reset, the same slots),
-// which saves the sweep's own fill launch.
+// sweeps' abort flag rides in block 0's entry); and with reset the next
+// forward sweep's output set to the all-ones sentinel (the same slots),
+// which saves the tile sweep's own fill launch.
 // N values of T, aligned to their size (N defaults to 16 bytes' worth):
 // one vector access per lane instead of N scalar ones
 template <class T, int NN = 16 / (int)sizeof(T)>
@@ -409,15 +409,17 @@ __global__ __launch_bounds__(kRedThreads) void k_update_xr_fused(
     for (int k = 0; k < N; ++k) one(xv.v[k], rv.v[k], sv.v[k], zv.v[k]);
     reinterpret_cast<Pack<double, N>*>(x)[i] = xv;
     reinterpret_cast<PV*>(r)[i] = rv;
-    PV ones;
+    if (reset) {
+      PV ones;
 #pragma unroll
-    for (int k = 0; k < N; ++k) set_all_ones(&ones.v[k]);
-    reinterpret_cast<PV*>(reset)[i] = ones;
+      for (int k = 0; k < N; ++k) set_all_ones(&ones.v[k]);
+      reinterpret_cast<PV*>(reset)[i] = ones;
+    }
   }
   for (int64_t i = nv * N + blockIdx.x * (int64_t)kRedThreads + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * kRedThreads) {
     one(x[i], r[i], s[i], z[i]);
-    set_all_ones(&reset[i]);
+    if (reset) set_all_ones(&reset[i]);
   }
   const double mm = block_max(m, sh);
   if (threadIdx.x == 0) {
@@ -848,10 +850,10 @@ static bool pcg_loop_box(hipStream_t st, PcgWork& w, int64_t ndof, const double*
     if (e0) ti->add(KTimer::SPMV, ndof, e0, ti->mark(st));
     hipLaunchKernelGGL(k_update_xr_fused<double>, dim3(nb), dim3(kRedThreads), 0, st, x, r, s,
                        z, nc, dp.p, dp.n, w.scal.p, rho_slot, w.host_part_dev,
-                       P.progress.p + 2, P.zf.p);
+                       P.progress.p + 2, P.sub ? nullptr : P.zf.p);
     WC_LAUNCH_CHECK();
     if (it + 1 < maxit) {
-      sweep_apply(st, P, r, ti, ndof, true);  // the update has set zf to the sentinel
+      sweep_apply(st, P, r, ti, ndof, true);  // (tile sweeps: the update has set zf to the sentinel)
       const int rho_next = rho_slot == S_RHO ? S_RHO2 : S_RHO;
       hipLaunchKernelGGL(k_update_s_fused<double>, dim3(nb), dim3(kRedThreads), 0, st, s, z,
                          nc, P.tdot.p, P.ndot, w.scal.p, rho_slot, rho_next,
@@ -950,11 +952,11 @@ static bool pcg_loop_box_mixed(hipStream_t st, PcgWork& w, int64_t ndof, const d
       if (e0) ti->add(KTimer::SPMV, ndof, e0, ti->mark(st));
       hipLaunchKernelGGL(k_update_xr_fused<float>, dim3(nb), dim3(kRedThreads), 0, st, x, r,
                          s, z, nc, dp.p, dp.n, w.scal.p, rho_slot, w.host_part_dev,
-                         P.progress.p + 2, P.zf32.p);
+                         P.progress.p + 2, P.sub ? nullptr : P.zf32.p);
       WC_LAUNCH_CHECK();
       ++total;
       if (total < maxit) {
-        sweep_apply32(st, P, r, ti, ndof, true);  // the update has set zf32 to the sentinel
+        sweep_apply32(st, P, r, ti, ndof, true);  // (as in pcg_loop_box)
         const int rho_next = rho_slot == S_RHO ? S_RHO2 : S_RHO;
         hipLaunchKernelGGL(k_update_s_fused<float>, dim3(nb), dim3(kRedThreads), 0, st, s, z,
                            nc, P.tdot.p, P.ndot, w.scal.p, rho_slot, rho_next,

@@ -899,7 +899,9 @@ struct SweepArgs {
   const uint32_t* code;
   const V* in;             // forward: r; backward: the forward result
   V* out;                  // the sweep result, or the factor's invdiag
-  V* reset;                // forward sweep: set to the sentinel step by step
+  V* reset;                // forward tile sweep: set to the sentinel step by step
+  V* mail;                 // sub-tile sweeps: the records units exchange ...
+  V* mail_reset;           // ... and the other pass's, set to the sentinel
   const V* dot_r;          // backward sweep: r (the forward sweep's input) ...
   double* dot_out;         // ... and its per-tile partials of z . r
   int* ticket;
@@ -1448,25 +1450,37 @@ __global__ __launch_bounds__(SweepBlock<KIND>::value) void k_sweep(SweepArgs<V> 
 // each step's values through LDS without a workgroup barrier (the LDS
 // processes one wave's operations in order, so a read issued after a write
 // sees it), and the only barriers are those that hand over a batch of kNB
-// steps of records and face values from the loader and face waves.  There
-// are twice as many hops between units as between tiles, each costing the
-// face read-ahead and a round trip; the shorter step is what the change
-// buys.
+// steps of records and face values from the loader and face waves.
 //
 // A sub-tile (sa, sb) of tile (a, b) runs every step w of the tile, 0 ..
 // nsteps - 1, for its 64 pencils (li, lj) = (8 sa + ui, 8 sb + uj): the
 // steps outside its pencils' cells are padding, which it writes as +0 like
 // every other slot, so each slot of the box is still written once per pass.
 // Units are claimed by ticket in (A + B, A) order over the sub-tile grid
-// (A, B) = (2 a + sa, 2 b + sb), and a unit waits only for the units at
-// (A - 1, B) and (A, B - 1): inside a tile through the slot offsets -257 and
-// -272 (one step back and one pencil over), across tiles through K.dx and
-// K.dy, mirrored in the backward pass.
+// (A, B) = (2 a + sa, 2 b + sb), one unit per workgroup, and a unit waits
+// only for the units at (A - 1, B) and (A, B - 1).
+//
+// What bounds the pass is the exchange between units, so it has memory of
+// its own, the mail: per unit and step one record of kMail values, the 15
+// values its downstream neighbours read (0..7 the column ui = 7 by uj, 8..14
+// the row uj = 7 by ui; the corner is entry 7).  The compute wave stores a
+// step's record with agent-scope stores as soon as it has the step, and the
+// neighbours' face waves read a batch's 8 + 8 values per step from 2 or 4
+// records that lie together.  The output itself is written by a store wave,
+// from the exchange planes, with plain 16-byte stores.  A record holds the
+// all-ones sentinel until it is written; the forward pass resets the
+// backward pass's mail and the other way round.  (With every output stored
+// agent-scope and the face values read out of it, a batch's faces lay in 20
+// cache lines instead of 4.)
+// Forward / backward sweep, us: 256^3 FP32 159 / 169 -> 128 / 129, FP64
+// 212 / 199 -> 162 / 171; 128^3 FP32 63 / 70 -> 56 / 58; 32^3 FP64 30 / 32 ->
+// 25 / 27.  A unit without upstream runs a step in 0.072 us (0.117 before the
+// records were read a batch ahead); a hop between units costs 1.8-2.4 us.
 constexpr int kS = 8;             // sub-tile edge (pencils)
 constexpr int kNB = 4;            // steps per batch
-constexpr int kSubPlanes = 16;    // exchange planes (step % 16), > 2 kNB - 1
-constexpr int kFaceWaves = 1;     // face waves (one read in flight each)
-constexpr int kSubThreads = 64 * (2 + kFaceWaves);  // compute, face(s), loader
+constexpr int kSubPlanes = 8;     // exchange planes (step % 8), two batches
+constexpr int kSubThreads = 256;  // compute, face, loader and store waves
+constexpr int kMail = 2 * kS;     // values of a mail record (the last unused)
 
 template <class V>
 struct SubRing {
@@ -1480,7 +1494,7 @@ struct SubRing {
   // batches loaded ahead: as many as the 6-bit load counter and the ring allow
   static constexpr int ahead() {
     int a = kBatches - 1;
-    while ((a - 1) * kFwdLoads + a * kRhsOps > 63 || (a - 1) * kBwdLoads > 63) --a;
+    while ((a - 1) * kBwdLoads > 63) --a;
     return a;
   }
   static constexpr int kAhead = ahead();
@@ -1492,6 +1506,18 @@ __device__ inline void wait_lgkmcnt0() {
   __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (3 << 14));
 }
 
+// agent-scope (sc1) store of one value at a byte offset of a buffer
+constexpr int kSc1 = 16;
+__device__ inline void store_mail(float v, __amdgpu_buffer_rsrc_t b, uint32_t off, int step) {
+  __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), b, (int)off, step, kSc1);
+}
+__device__ inline void store_mail(double v, __amdgpu_buffer_rsrc_t b, uint32_t off, int step) {
+  typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  __builtin_amdgcn_raw_buffer_store_b64(U2{(unsigned)u, (unsigned)(u >> 32)}, b, (int)off, step,
+                                        kSc1);
+}
+
 template <int KIND, class V>
 __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   static_assert(KIND == K_FWD || KIND == K_BWD, "sweeps only");
@@ -1499,15 +1525,24 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   using Ring = SubRing<V>;
   constexpr int kRB = Ring::kBatches;
   constexpr int kLA = Ring::kAhead;
-  // exchange planes in the tile's 17 x 17 geometry (the operand words'),
-  // each with a +0 at [0][0] that no unit writes
-  __shared__ V pl[kSubPlanes * kPlane];
-  // record rings [batch % kRB][step in batch][physical position in the unit]
-  __shared__ CellT<V> rc[kRB][kNB][64];
-  __shared__ V rr[kRB][kNB][64];
-  __shared__ uint32_t rk[kRB][kNB][64];
-  __shared__ V rq[BWD ? kRB : 1][kNB][64];
-  __shared__ int s_unit;
+  // (one object, the planes first: a plane's cells are then reached with the
+  // LDS instructions' immediate offsets)
+  __shared__ struct {
+    // exchange planes in the tile's 17 x 17 geometry (the operand words'),
+    // each with a +0 at [0][0] that no unit writes
+    V pl[kSubPlanes * kPlane];
+    // record rings [batch % kRB][step in batch][physical position in the unit]
+    CellT<V> rc[kRB][kNB][64];
+    V rr[kRB][kNB][64];
+    uint32_t rk[kRB][kNB][64];
+    V rq[BWD ? kRB : 1][kNB][64];
+    int unit;
+  } sh;
+  auto& pl = sh.pl;
+  auto& rc = sh.rc;
+  auto& rr = sh.rr;
+  auto& rk = sh.rk;
+  auto& rq = sh.rq;
   if (threadIdx.x < kSubPlanes) pl[threadIdx.x * kPlane] = (V)0;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
@@ -1517,326 +1552,304 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   const int nsa = 2 * S.K.ntile_a;
   auto PL = [](int w) -> uint32_t { return (uint32_t)(w & (kSubPlanes - 1)) * kPlane; };
   const int sgn = BWD ? -kThreads : kThreads;
-  // The next unit (A, B), counted from the sweep's start corner, or -1.
-  // Each role runs its own loop over the units (so the compute wave's code
-  // holds none of the loader's direct-to-LDS loads, and the compiler adds
-  // no wait for them there); the loops meet at the same barriers.
-  auto claim = [&]() -> int {
-    if (threadIdx.x == 0) {
-      const int t = atomicAdd(S.ticket, 1);
-      s_unit = t < S.ntiles ? (int)S.order[t] : -1;
-      if (t == 0) *S.next_ticket = 0;  // the other pass's counter
-    }
-    __syncthreads();
-    return __builtin_amdgcn_readfirstlane(s_unit);
+  // The unit (A, B), counted from the sweep's start corner.  The grid has
+  // one workgroup per ticket.
+  if (threadIdx.x == 0) {
+    const int t = atomicAdd(S.ticket, 1);
+    sh.unit = (int)S.order[t];
+    if (t == 0) *S.next_ticket = 0;  // the other pass's counter
+  }
+  __syncthreads();
+  const int unit = __builtin_amdgcn_readfirstlane(sh.unit);
+  // its tile and quarter in the sweep's frame and the physical ones
+  const int A = unit & 0xFFFF, B = unit >> 16;
+  const int sa = A & 1, sb = B & 1;
+  const int a = BWD ? S.K.ntile_a - 1 - (A >> 1) : A >> 1;
+  const int b = BWD ? S.K.ntile_b - 1 - (B >> 1) : B >> 1;
+  const int psa = BWD ? 1 - sa : sa, psb = BWD ? 1 - sb : sb;
+  // the unit's 64 slots of step w are 8 rows of 8 consecutive slots
+  // (physical order p = row * 8 + column); steps past the end give the last
+  const uint32_t tile0 = (uint32_t)skew_slot(S.K, a, b, 0, 0, 0);
+  auto slot = [&](int w, int p) -> uint32_t {
+    const int wc = w < nsteps ? w : nsteps - 1;
+    const int wp = BWD ? nsteps - 1 - wc : wc;
+    return tile0 + (uint32_t)wp * kThreads +
+           (uint32_t)((kS * psb + (p >> 3)) * kT + kS * psa + (p & 7));
   };
-  // a unit's tile and quarter in the sweep's frame and the physical ones
-  struct Unit {
-    int A, B, sa, sb, a, b, psa, psb;
-  };
-  auto decode = [&](int unit) -> Unit {
-    Unit u;
-    u.A = unit & 0xFFFF;
-    u.B = unit >> 16;
-    u.sa = u.A & 1;
-    u.sb = u.B & 1;
-    u.a = BWD ? S.K.ntile_a - 1 - (u.A >> 1) : u.A >> 1;
-    u.b = BWD ? S.K.ntile_b - 1 - (u.B >> 1) : u.B >> 1;
-    u.psa = BWD ? 1 - u.sa : u.sa;
-    u.psb = BWD ? 1 - u.sb : u.sb;
-    return u;
-  };
-  auto base_of = [&](const Unit& u, int li, int lj) -> uint32_t {
-    const int lip = BWD ? kT - 1 - li : li, ljp = BWD ? kT - 1 - lj : lj;
-    return (uint32_t)skew_slot(S.K, u.a, u.b, lip, ljp, BWD ? nsteps - 1 : 0);
+  // a unit's mail records: (step * kMail) from here
+  auto mail_of = [&](int UA, int UB) -> uint32_t {
+    return (uint32_t)((UB * nsa + UA) * nb * kNB) * kMail;
   };
   if (wave == 2) {
-    // loader: the unit's 64 slots of step w are 8 rows of 8 consecutive
-    // slots (physical order p = row * 8 + column); steps past the end
-    // reload the last one, so every batch issues the same operations and
-    // the counter waits stay exact
+    // loader; every batch issues the same operations, so the counter waits
+    // stay exact
     typedef __attribute__((address_space(3))) void* LdsPtr;
-    typedef unsigned int U4 __attribute__((ext_vector_type(4)));
-    U4 ones = {~0u, ~0u, ~0u, ~0u};
-    asm volatile("" : "+v"(ones));
-    for (;;) {
-      const int unit = claim();
-      if (unit < 0) return;
-      const Unit u = decode(unit);
-      const uint32_t tile0 = (uint32_t)skew_slot(S.K, u.a, u.b, 0, 0, 0);
-      auto slot = [&](int w, int p) -> uint32_t {
-        const int wc = w < nsteps ? w : nsteps - 1;
-        const int wp = BWD ? nsteps - 1 - wc : wc;
-        return tile0 + (uint32_t)wp * kThreads +
-               (uint32_t)((kS * u.psb + (p >> 3)) * kT + kS * u.psa + (p & 7));
-      };
-      // 16 bytes per lane from 'src' (element size E) into 'dst' for the
-      // kNB steps of batch n: each wave-wide load covers 1024 / (64 E) steps
-      auto stream = [&](const void* src, void* dst, int n, auto E) {
-        constexpr int per = 1024 / (64 * (int)decltype(E)::value);  // steps per load
-        constexpr int lanes = 64 / per;                              // lanes per step
+    // 16 bytes per lane from 'src' (element size E) into 'dst' for the
+    // kNB steps of batch n: each wave-wide load covers 1024 / (64 E) steps
+    auto stream = [&](const void* src, void* dst, int n, auto E) {
+      constexpr int per = 1024 / (64 * (int)decltype(E)::value);  // steps per load
+      constexpr int lanes = 64 / per;                              // lanes per step
 #pragma unroll
-        for (int j = 0; j < kNB / per; ++j) {
-          const int st = j * per + lane / lanes;
-          const int p = (lane % lanes) * (16 / (int)decltype(E)::value);
-          const char* g = reinterpret_cast<const char*>(src) +
-                          (size_t)slot(n * kNB + st, p) * decltype(E)::value;
-          __builtin_amdgcn_global_load_lds(g, (LdsPtr)(reinterpret_cast<char*>(dst) + j * 1024),
-                                           16, 0, 0);
-        }
-      };
-      using EV = std::integral_constant<int, (int)sizeof(V)>;
-      using E4 = std::integral_constant<int, 4>;
-      auto issue = [&](int n) {
-        const int r = n & (kRB - 1);
-        // records: 16 bytes per lane, sizeof(CellT) / 16 pieces per slot
-        constexpr int kPieces = (int)sizeof(CellT<V>) / 16;
-#pragma unroll
-        for (int st = 0; st < kNB; ++st)
-#pragma unroll
-          for (int h = 0; h < kPieces; ++h) {
-            const int p = h * (64 / kPieces) + lane / kPieces;
-            const char* g = reinterpret_cast<const char*>(S.cells) +
-                            (size_t)slot(n * kNB + st, p) * sizeof(CellT<V>) +
-                            (lane % kPieces) * 16;
-            __builtin_amdgcn_global_load_lds(
-                g, (LdsPtr)(reinterpret_cast<char*>(&rc[r][st][0]) + h * 1024), 16, 0, 0);
-          }
-        stream(S.in, &rr[r][0][0], n, EV{});
-        stream(S.code, &rk[r][0][0], n, E4{});
-        if constexpr (BWD) stream(S.dot_r, &rq[r][0][0], n, EV{});
-      };
-      // forward pass: the backward output's slots of batch n to the sentinel
-      auto clear = [&](int n) {
-        constexpr int per = 1024 / (64 * (int)sizeof(V));
-        constexpr int lanes = 64 / per;
-#pragma unroll
-        for (int j = 0; j < kNB / per; ++j) {
-          const int st = j * per + lane / lanes;
-          const int p = (lane % lanes) * (16 / (int)sizeof(V));
-          *reinterpret_cast<U4*>(reinterpret_cast<char*>(S.reset) +
-                                 (size_t)slot(n * kNB + st, p) * sizeof(V)) = ones;
-        }
-      };
-      for (int n = 0; n < kLA; ++n) issue(n);
-      for (int n = 0; n < nb; ++n) {
-        // batch n complete; the loads of the kLA - 1 batches after it (and
-        // in the forward pass the clears of the kLA batches before it,
-        // issued after its loads) may still be in flight
-        if (BWD)
-          wait_vmcnt<(kLA - 1) * Ring::kBwdLoads>();
-        else if (n < kLA)
-          wait_vmcnt<(kLA - 1) * Ring::kFwdLoads>();
-        else
-          wait_vmcnt<(kLA - 1) * Ring::kFwdLoads + kLA * Ring::kRhsOps>();
-        __builtin_amdgcn_s_barrier();
-        issue(n + kLA);
-        if constexpr (!BWD) clear(n);
+      for (int j = 0; j < kNB / per; ++j) {
+        const int st = j * per + lane / lanes;
+        const int p = (lane % lanes) * (16 / (int)decltype(E)::value);
+        const char* g = reinterpret_cast<const char*>(src) +
+                        (size_t)slot(n * kNB + st, p) * decltype(E)::value;
+        __builtin_amdgcn_global_load_lds(g, (LdsPtr)(reinterpret_cast<char*>(dst) + j * 1024),
+                                         16, 0, 0);
       }
-      wait_vmcnt<0>();
+    };
+    using EV = std::integral_constant<int, (int)sizeof(V)>;
+    using E4 = std::integral_constant<int, 4>;
+    auto issue = [&](int n) {
+      const int r = n & (kRB - 1);
+      // records: 16 bytes per lane, sizeof(CellT) / 16 pieces per slot
+      constexpr int kPieces = (int)sizeof(CellT<V>) / 16;
+#pragma unroll
+      for (int st = 0; st < kNB; ++st)
+#pragma unroll
+        for (int h = 0; h < kPieces; ++h) {
+          const int p = h * (64 / kPieces) + lane / kPieces;
+          const char* g = reinterpret_cast<const char*>(S.cells) +
+                          (size_t)slot(n * kNB + st, p) * sizeof(CellT<V>) +
+                          (lane % kPieces) * 16;
+          __builtin_amdgcn_global_load_lds(
+              g, (LdsPtr)(reinterpret_cast<char*>(&rc[r][st][0]) + h * 1024), 16, 0, 0);
+        }
+      stream(S.in, &rr[r][0][0], n, EV{});
+      stream(S.code, &rk[r][0][0], n, E4{});
+      if constexpr (BWD) stream(S.dot_r, &rq[r][0][0], n, EV{});
+    };
+    constexpr int kLoads = BWD ? Ring::kBwdLoads : Ring::kFwdLoads;
+    for (int n = 0; n < kLA; ++n) issue(n);
+    wait_vmcnt<(kLA - 1) * kLoads>();
+    __builtin_amdgcn_s_barrier();  // batch 0's records
+    for (int n = 0; n < nb; ++n) {
+      // batch n + 1 complete; the loads of the kLA - 2 batches after it may
+      // still be in flight
+      wait_vmcnt<(kLA - 2) * kLoads>();
       __builtin_amdgcn_s_barrier();
+      issue(n + kLA);
     }
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    return;
   }
-  if (wave == 1 || wave >= 3) {
-    // face waves (wave 1, and waves 3 .. with kFaceWaves > 1): face wave p
-    // publishes the batches n = p (mod kFaceWaves), each read with one
-    // read in flight on the wave's own counter, issued when the wave
-    // publishes its previous batch, so a read has kFaceWaves batches to
-    // return.  A batch's face values are the x face of rows m (pencils
-    // (8 sa, 8 sb + m)) and the y face of columns m (pencils (8 sa + m,
-    // 8 sb)) at each of its steps; upstream values come from the unit
-    // before in x (y): the other quarter of this tile, one step back and
-    // one pencil over, or the tile before.
-    const int par = wave == 1 ? 0 : wave - 2;
-    // item k of a lane is value g = 64 k + lane of the batch: face g /
-    // (kNB kS) (x, then y), step (g / kS) % kNB, row or column g % kS
-    constexpr int kPer = kNB * kS;
-    constexpr int kItems = 2 * kPer / 64;
-    static_assert(2 * kPer % 64 == 0, "a batch's face values fill whole waves");
-    for (;;) {
-      const int unit = claim();
-      if (unit < 0) return;
-      const Unit u = decode(unit);
-      const int64_t dxs =
-          u.sa ? (BWD ? kThreads + 1 : -(kThreads + 1)) : (BWD ? -S.K.dx : S.K.dx);
-      const int64_t dys =
-          u.sb ? (BWD ? kThreads + kT : -(kThreads + kT)) : (BWD ? -S.K.dy : S.K.dy);
-      uint32_t ibase[kItems], idel[kItems], ihalo[kItems];
-      int ioff[kItems], istep[kItems];
-      bool iup[kItems];
-#pragma unroll
-      for (int k = 0; k < kItems; ++k) {
-        const int g = 64 * k + lane;
-        const bool xf = g < kPer;
-        const int m = g % kS;
-        istep[k] = (g / kS) % kNB;
-        const int li = xf ? kS * u.sa : kS * u.sa + m, lj = xf ? kS * u.sb + m : kS * u.sb;
-        iup[k] = xf ? u.A > 0 : u.B > 0;
-        ibase[k] = base_of(u, li, lj);
-        ioff[k] = li + lj;
-        idel[k] = iup[k] ? (uint32_t)(xf ? dxs : dys) : 0u;
-        // the halo cell beside the pencil in the exchange plane
-        ihalo[k] = (uint32_t)(xf ? (lj + 1) * (kT + 1) + li : lj * (kT + 1) + li + 1);
-      }
-      // the pencil's cell of step w (clamped into the pencil, so the
-      // address is always a slot of the box) and the upstream slot beside it
-      auto addr = [&](int k, int w) -> uint32_t {
-        const int kk = w - ioff[k];
-        const int kc = kk < 0 ? 0 : (kk >= Bz ? Bz - 1 : kk);
-        return ibase[k] + (uint32_t)(sgn * (kc + ioff[k])) + idel[k];
-      };
-      auto need = [&](int k, int w) -> bool {
-        const int kk = w - ioff[k];
-        return iup[k] && w < nsteps && kk >= 0 && kk < Bz;
-      };
-      V fv[kItems];
-#pragma unroll
-      for (int k = 0; k < kItems; ++k) fv[k] = (V)0;
-      // (only where the value is needed: a unit's face reads are a fair
-      // share of the sweep's coherent traffic)
-      auto fetch = [&](int n) {
-#pragma unroll
-        for (int k = 0; k < kItems; ++k)
-          fv[k] = need(k, n * kNB + istep[k]) ? load_coherent(at(S.out, addr(k, n * kNB + istep[k])))
-                                              : (V)0;
-      };
-      // batch n's values into the halos of the planes its steps read;
-      // a value still the sentinel is read again (bounded wait)
-      auto publish = [&](int n) {
-        bool nd[kItems];
-        bool bad = false;
-#pragma unroll
-        for (int k = 0; k < kItems; ++k) {
-          nd[k] = need(k, n * kNB + istep[k]);
-          bad = bad || (nd[k] && is_sentinel(fv[k]));
-        }
-        // (the first check stays outside the retry loop: with the loop's
-        // reloads on its path the compiler waits for every read in flight)
-        if (__any(bad)) {
-          long long spins = 0;
-          for (;;) {
-            if (++spins > kSpinLimit || load_flag(S.abort_flag)) {
-              store_flag(S.abort_flag, 1);
-#pragma unroll
-              for (int k = 0; k < kItems; ++k) fv[k] = (V)0;
-              break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-            bool again = false;
-#pragma unroll
-            for (int k = 0; k < kItems; ++k) {
-              if (nd[k] && is_sentinel(fv[k]))
-                fv[k] = load_coherent(at(S.out, addr(k, n * kNB + istep[k])));
-              again = again || (nd[k] && is_sentinel(fv[k]));
-            }
-            if (!__any(again)) break;
+  if (wave == 1) {
+    // face wave: lane (face, step, row) takes one value of the batch, from
+    // the x-upstream unit's record entry m (row m's pencil) or the
+    // y-upstream unit's entry of column m.  Both upstream pencils lie one
+    // step back inside a tile and, the steps of a tile being counted from
+    // its own corner, kT - 1 steps on across tiles.  The read of batch n + 2
+    // is issued when batch n + 1 is published, during batch n.
+    static_assert(2 * kNB * kS == 64, "a batch's face values fill the wave");
+    const bool xf = lane < kNB * kS;
+    const int st = (lane / kS) % kNB, m = lane % kS;
+    const int li = xf ? kS * sa : kS * sa + m, lj = xf ? kS * sb + m : kS * sb;
+    const bool up = xf ? A > 0 : B > 0;
+    const int ahead = (xf ? sa : sb) ? -1 : kT - 1;
+    const V* const src = S.mail + (up ? mail_of(xf ? A - 1 : A, xf ? B : B - 1) +
+                                            (uint32_t)(xf || m == kS - 1 ? m % kS : kS + m)
+                                      : 0u);
+    const int off = li + lj;
+    // the halo cell beside the pencil in the exchange plane
+    const uint32_t halo = (uint32_t)(xf ? (lj + 1) * (kT + 1) + li : lj * (kT + 1) + li + 1);
+    // the pencil has a cell at step w and an upstream value beside it
+    auto need = [&](int w) -> bool { return up && w < nsteps && w >= off && w - off < Bz; };
+    V fv = (V)0;
+    auto fetch = [&](int n) {
+      const int w = n * kNB + st;
+      fv = need(w) ? load_coherent(at(src, (uint32_t)((w + ahead) * kMail))) : (V)0;
+    };
+    // batch n's values into the halos of the planes its steps read;
+    // a value still the sentinel is read again (bounded wait)
+    auto publish = [&](int n) {
+      const int w = n * kNB + st;
+      const bool nd = need(w);
+      // (the first check stays outside the retry loop: with the loop's
+      // reloads on its path the compiler waits for every read in flight)
+      if (__any(nd && is_sentinel(fv))) {
+        long long spins = 0;
+        for (;;) {
+          if (++spins > kSpinLimit || load_flag(S.abort_flag)) {
+            store_flag(S.abort_flag, 1);
+            fv = (V)0;
+            break;
           }
-        }
-#pragma unroll
-        for (int k = 0; k < kItems; ++k) {
-          const int w = n * kNB + istep[k];
-          if (w < nsteps) pl[PL(w - 1) + ihalo[k]] = nd[k] ? fv[k] : (V)0;
-        }
-      };
-      // backward pass: the z . r partial of compute lane 'lane', summed
-      // here so the compute wave's steps stay short: r of batch n is copied
-      // from the ring during batch n, and z of batch n read from the
-      // exchange planes during batch n + 1 (the planes keep a step for 16
-      // steps), in step order, as the compute lane would sum them
-      const int cli = kS * u.sa + (lane & 7), clj = kS * u.sb + (lane >> 3);
-      const uint32_t cown = (uint32_t)((clj + 1) * (kT + 1) + cli + 1);
-      const int cpos = BWD ? 63 - lane : lane;
-      double dot = 0.0;
-      V rsave[kNB];
-      auto take_r = [&](int n) {
-#pragma unroll
-        for (int st = 0; st < kNB; ++st) rsave[st] = rq[n & (kRB - 1)][st][cpos];
-      };
-      auto add_z = [&](int n) {
-#pragma unroll
-        for (int st = 0; st < kNB; ++st) {
-          const int w = n * kNB + st;
-          if (w < nsteps) dot += (double)pl[PL(w) + cown] * (double)rsave[st];
-        }
-      };
-      // batch 0 is due at the first barrier: face wave 0 reads and
-      // publishes it now; then each face wave has its next batch in flight
-      if (par == 0) {
-        fetch(0);
-        publish(0);
-      }
-      {
-        const int first = par == 0 ? kFaceWaves : par;
-        if (first < nb) fetch(first);
-      }
-      for (int n = 0; n < nb; ++n) {
-        __syncthreads();  // batch n handed over
-        const int due = n + 1;  // published during batch n
-        if (due < nb && due % kFaceWaves == par) {
-          publish(due);
-          if (due + kFaceWaves < nb) fetch(due + kFaceWaves);
-        }
-        if constexpr (BWD) {
-          if (par == 0) {
-            if (n > 0) add_z(n - 1);
-            take_r(n);
-          }
+          if (nd && is_sentinel(fv)) fv = load_coherent(at(src, (uint32_t)((w + ahead) * kMail)));
+          if (!__any(nd && is_sentinel(fv))) break;
         }
       }
-      __syncthreads();
-      if (BWD && par == 0) {
-        add_z(nb - 1);
-        // the unit's partial: a fixed tree over its 64 lanes, stored at the
-        // physical quarter's index
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
-        if (lane == 0) S.dot_out[(2 * u.b + u.psb) * nsa + 2 * u.a + u.psa] = dot;
+      if (w < nsteps) pl[PL(w - 1) + halo] = nd ? fv : (V)0;
+    };
+    // batch 0 is due at the first batch's barrier
+    fetch(0);
+    __syncthreads();
+    publish(0);
+    if (1 < nb) fetch(1);
+    for (int n = 0; n < nb; ++n) {
+      __syncthreads();  // batch n handed over
+      if (n + 1 < nb) {
+        publish(n + 1);
+        if (n + 2 < nb) fetch(n + 2);
       }
     }
+    __syncthreads();
+    return;
+  }
+  if (wave == 3) {
+    // store wave: batch n - 1's values from the exchange planes (which keep
+    // a batch for the next one) to the output during batch n, 16 bytes per lane
+    // (in physical order); the other pass's mail records of the batch's
+    // steps reset to the sentinel; and in the backward pass the z . r
+    // partial of compute lane 'lane', in step order, as that lane would sum
+    // it: r of batch n is copied from the ring during batch n, z of batch n
+    // read from the planes during batch n + 1
+    typedef unsigned int U4 __attribute__((ext_vector_type(4)));
+    constexpr int kVec = 16 / (int)sizeof(V);
+    constexpr int kPer = 64 / kVec;           // lanes per step
+    constexpr int kOps = kNB * kPer / 64;     // stores per batch
+    struct alignas(16) Quad {
+      V v[kVec];
+    };
+    auto cell = [&](int l) -> uint32_t {
+      return (uint32_t)((kS * sb + (l >> 3) + 1) * (kT + 1) + kS * sa + (l & 7) + 1);
+    };
+    auto put = [&](int n) {
+#pragma unroll
+      for (int j = 0; j < kOps; ++j) {
+        const int w = n * kNB + j * (64 / kPer) + lane / kPer, p = lane % kPer * kVec;
+        if (w < nsteps) {
+          Quad q;
+#pragma unroll
+          for (int k = 0; k < kVec; ++k) q.v[k] = pl[PL(w) + cell(BWD ? 63 - (p + k) : p + k)];
+          *reinterpret_cast<Quad*>(at(S.out, slot(w, p))) = q;
+        }
+      }
+    };
+    constexpr int kClear = kNB * kMail * (int)sizeof(V) / 16;  // 16-byte words per batch
+    static_assert(kClear <= 64, "a batch's records are reset by one store per lane");
+    auto clear = [&](int n) {
+      constexpr int per = kClear / kNB;  // words per step
+      const int w = n * kNB + lane / per;
+      if (lane < kClear && w < nsteps)
+        *reinterpret_cast<U4*>(reinterpret_cast<char*>(
+            at(S.mail_reset, mail_of(A, B) + (uint32_t)w * kMail)) + lane % per * 16) =
+            U4{~0u, ~0u, ~0u, ~0u};
+    };
+    const uint32_t cown = cell(lane);
+    const int cpos = BWD ? 63 - lane : lane;
+    double dot = 0.0;
+    V rsave[kNB];
+    auto take_r = [&](int n) {
+#pragma unroll
+      for (int st = 0; st < kNB; ++st) rsave[st] = rq[n & (kRB - 1)][st][cpos];
+    };
+    auto add_z = [&](int n) {
+#pragma unroll
+      for (int st = 0; st < kNB; ++st) {
+        const int w = n * kNB + st;
+        if (w < nsteps) dot += (double)pl[PL(w) + cown] * (double)rsave[st];
+      }
+    };
+    __syncthreads();
+    for (int n = 0; n < nb; ++n) {
+      __syncthreads();  // batch n - 1 computed, batch n handed over
+      clear(n);
+      if (n > 0) put(n - 1);
+      if constexpr (BWD) {
+        if (n > 0) add_z(n - 1);
+        take_r(n);
+      }
+    }
+    __syncthreads();
+    put(nb - 1);
+    if constexpr (BWD) {
+      add_z(nb - 1);
+      // the unit's partial: a fixed tree over its 64 lanes, stored at the
+      // physical quarter's index
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
+      if (lane == 0) S.dot_out[(2 * b + psb) * nsa + 2 * a + psa] = dot;
+    }
+    return;
   }
   // compute wave: lane (ui, uj) = (lane % 8, lane / 8) is pencil
   // (li, lj) = (8 sa + ui, 8 sb + uj) of the tile
   const int pos = BWD ? 63 - lane : lane;
-  for (;;) {
-    const int unit = claim();
-    if (unit < 0) return;
-    const Unit u = decode(unit);
-    const int li = kS * u.sa + (lane & 7), lj = kS * u.sb + (lane >> 3);
-    const uint32_t base = base_of(u, li, lj);
-    const uint32_t own = (uint32_t)((lj + 1) * (kT + 1) + li + 1);
-    for (int n = 0; n < nb; ++n) {
-      // this wave's plane writes are complete (the face wave sums z . r
-      // from them), and batch n's records and face values are in place
-      wait_lgkmcnt0();
-      __syncthreads();
-      const int r = n & (kRB - 1);
-      // the batch's records and operand addresses first (the ring is
-      // complete for the whole batch), so a step waits on one LDS round
-      // trip only: its operands, written by the step before
-      CellIn<V> ci[kNB];
-      uint32_t src[kNB][3];
+  const int ui = lane & 7, uj = lane >> 3;
+  const uint32_t own = (uint32_t)((kS * sb + uj + 1) * (kT + 1) + kS * sa + ui + 1);
+  // the lanes on the unit's far faces store their record entry; the others'
+  // offset lies past the buffer's end, where a store is dropped (one
+  // instruction for all lanes, with no change of the execution mask)
+  const bool mailer = ui == kS - 1 || uj == kS - 1;
+  const __amdgpu_buffer_rsrc_t mail_buf = __builtin_amdgcn_make_buffer_rsrc(
+      S.mail + mail_of(A, B), 0, nb * kNB * kMail * (int)sizeof(V), 0x00020000);
+  const uint32_t mail_off =
+      mailer ? (uint32_t)(ui == kS - 1 ? uj : kS + ui) * (uint32_t)sizeof(V) : 0x40000000u;
+  // A batch's records are read from the ring during the batch before it
+  // (the loader hands a batch over one barrier early), and the loop is
+  // unrolled over the two batches the planes hold, so that a step's critical
+  // path is its three operand reads, the arithmetic and the plane write.
+  struct Rec {
+    CellIn<V> ci[kNB];
+    uint32_t src[kNB][3];  // the operands' byte offsets in the previous step's plane
+  };
+  auto read = [&](Rec& R, int n, int st) {
+    const int r = n & (kRB - 1);
+    R.ci[st].c = rc[r][st][pos];
+    R.ci[st].rhs = rr[r][st][pos];
+    R.ci[st].code = rk[r][st][pos];
+  };
+  auto locate = [&](Rec& R) {
 #pragma unroll
-      for (int st = 0; st < kNB; ++st) {
-        ci[st].c = rc[r][st][pos];
-        ci[st].rhs = rr[r][st][pos];
-        const uint32_t op = rk[r][st][pos];
-        const uint32_t at0 = PL(n * kNB + st - 1) + own;
+    for (int st = 0; st < kNB; ++st)
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
-          src[st][q] = at0 + (uint32_t)__builtin_amdgcn_sbfe((int)op, 10 * q, 10);
-      }
+      for (int q = 0; q < 3; ++q)
+        R.src[st][q] = (uint32_t)sizeof(V) *
+                       (own + (uint32_t)__builtin_amdgcn_sbfe((int)R.ci[st].code, 10 * q, 10));
+    // (kept in registers: sunk into the steps they would lengthen them)
 #pragma unroll
-      for (int st = 0; st < kNB; ++st) {
-        const int w = n * kNB + st;
-        if (w >= nsteps) break;
-        const V z = sweep_cell_ordered<V>(ci[st], pl[src[st][0]], pl[src[st][1]], pl[src[st][2]]);
-        store_coherent(at(S.out, base + (uint32_t)(sgn * w)), z);
-        pl[PL(w) + own] = z;
-      }
-    }
+    for (int st = 0; st < kNB; ++st)
+      asm volatile("" : "+v"(R.src[st][0]), "+v"(R.src[st][1]), "+v"(R.src[st][2]));
+  };
+  auto lds_at = [](const V* p, uint32_t bytes) -> const V* {
+    return reinterpret_cast<const V*>(reinterpret_cast<const char*>(p) + bytes);
+  };
+  auto batch = [&](auto half, int n, const Rec& cur, Rec& next) {
+    constexpr int w0 = decltype(half)::value * kNB;  // the batch's first plane
+    // this wave's plane writes are complete (the store wave reads them),
+    // and batch n's face values and batch n + 1's records are in place
     wait_lgkmcnt0();
     __syncthreads();
+#pragma unroll
+    for (int st = 0; st < kNB; ++st) {
+      // (the steps past nsteps of the last batch run too: nothing reads
+      // their plane cells or their records)
+      const V* const prev = pl + PL(w0 + st + kSubPlanes - 1);
+      const V v0 = *lds_at(prev, cur.src[st][0]), v1 = *lds_at(prev, cur.src[st][1]),
+              v2 = *lds_at(prev, cur.src[st][2]);
+      __builtin_amdgcn_sched_barrier(0);
+      read(next, n + 1, st);
+      const V z = sweep_cell_ordered<V>(cur.ci[st], v0, v1, v2);
+      pl[PL(w0 + st) + own] = z;
+      store_mail(z, mail_buf, mail_off, (n * kNB + st) * kMail * (int)sizeof(V));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    locate(next);
+  };
+  Rec r0, r1;
+  wait_lgkmcnt0();
+  __syncthreads();  // batch 0's records
+#pragma unroll
+  for (int st = 0; st < kNB; ++st) read(r0, 0, st);
+  locate(r0);
+  for (int n = 0; n < nb; n += 2) {
+    batch(std::integral_constant<int, 0>{}, n, r0, r1);
+    if (n + 1 < nb) batch(std::integral_constant<int, 1>{}, n + 1, r1, r0);
   }
+  wait_lgkmcnt0();
+  __syncthreads();
 }
 
 inline unsigned blocks(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
@@ -1930,6 +1943,7 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const Grid& g, const uint8_t* a
   // again by each factor, not by the applies: once set it stays set)
   WC_HIP(hipMemsetAsync(P.progress.p, 0, sizeof(int) * 8, st));
   P.ticks_zero = true;
+  P.mail_word = 0;
   BoxArgs A;
   A.g = g;
   for (int d = 0; d < 3; ++d) A.o[d] = P.o[d];
@@ -1994,6 +2008,7 @@ void sweep_factor(hipStream_t st, SweepPlan& P, double tau, double mdr) {
   S.out = P.zf.p;
   S.ticket = tick + 3;
   P.ticks_zero = true;   // counters 0 and 1 are not touched by the factor
+  P.mail_word = 0;
   hipLaunchKernelGGL((k_sweep<K_FAC, double>), dim3(P.ntiles), dim3(SweepBlock<K_FAC>::value), 0, st, S);
   WC_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_backward_records, dim3(blocks(P.ncell, 256)), dim3(256), 0, st,
@@ -2033,6 +2048,34 @@ __global__ void k_fill_sentinel(uint4* p, int64_t n) {
     p[i] = ones;
 }
 
+static void fill_sentinel(hipStream_t st, void* p, int64_t words) {
+  hipLaunchKernelGGL(k_fill_sentinel,
+                     dim3((unsigned)std::min<int64_t>((words + 255) / 256, 4096)), dim3(256), 0,
+                     st, reinterpret_cast<uint4*>(p), words);
+  WC_LAUNCH_CHECK();
+}
+
+// values of one pass's mail: a record per unit and step (whole batches)
+static int64_t mail_values(const SweepPlan& P) {
+  return 4ll * P.ntiles * ((P.nsteps + kNB - 1) / kNB * kNB) * kMail;
+}
+
+// The mail of both passes (forward, then backward) in the plan's buffer,
+// which holds the larger type's; filled with the sentinel when the plan, the
+// factor or the value type has changed since the last apply, else left as
+// the last backward and forward pass have reset it.
+template <class V>
+static V* ready_mail(hipStream_t st, SweepPlan& P) {
+  const int64_t n = 2 * mail_values(P);
+  P.mail.ensure(n);
+  V* m = reinterpret_cast<V*>(P.mail.p);
+  if (P.mail_word != (int)sizeof(V)) {
+    fill_sentinel(st, m, (int64_t)sizeof(V) * n / 16);
+    P.mail_word = (int)sizeof(V);
+  }
+  return m;
+}
+
 template <class V>
 static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, const V* cb,
                        V* zf, V* zb, KTimer* timer, int64_t ndof, bool cleared) {
@@ -2045,11 +2088,11 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   int* tick = P.progress.p;
   if (!P.ticks_zero) WC_HIP(hipMemsetAsync(tick, 0, sizeof(int) * 2, st));
   static_assert(kThreads % 16 == 0, "slots come in whole 16-byte words");
-  const int64_t words = (int64_t)sizeof(V) * P.ncell / 16;
-  if (!cleared)  // else the PCG update before this apply has filled zf
-    hipLaunchKernelGGL(k_fill_sentinel,
-                       dim3((unsigned)std::min<int64_t>((words + 255) / 256, 4096)), dim3(256), 0,
-                       st, reinterpret_cast<uint4*>(zf), words);
+  const bool sub = P.sub;
+  // the sub-tile sweeps keep their own records as sentinels between passes
+  V* const mail = sub ? ready_mail<V>(st, P) : nullptr;
+  if (!sub && !cleared)  // else the PCG update before this apply has filled zf
+    fill_sentinel(st, zf, (int64_t)sizeof(V) * P.ncell / 16);
   SweepArgs<V> S = sweep_args<V>(P);
   S.cells = reinterpret_cast<const CellT<V>*>(cf);
   S.in = r;
@@ -2058,10 +2101,12 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   S.code = P.opf.p;  // the sweeps read operand words, not the code
   S.ticket = tick;
   S.next_ticket = tick + 1;
-  const bool sub = P.sub;
   if (sub) {
     S.ntiles = 4 * P.ntiles;  // tickets: the sub-tile units
     S.order = P.order_sub.p;
+    S.reset = nullptr;
+    S.mail = mail;
+    S.mail_reset = mail + mail_values(P);
   }
   P.ndot = S.ntiles;
   hipEvent_t e0 = timer ? timer->mark(st) : nullptr;
@@ -2080,6 +2125,7 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   S.code = P.opb.p;
   S.ticket = tick + 1;
   S.next_ticket = tick;
+  std::swap(S.mail, S.mail_reset);
   hipEvent_t e2 = timer ? timer->mark(st) : nullptr;
   if (sub)
     hipLaunchKernelGGL((k_sweep_sub<K_BWD, V>), dim3(S.ntiles), dim3(kSubThreads), 0, st, S);
@@ -2220,6 +2266,8 @@ void SweepPlan::release() {
   xf15_32.release();
   xf0_32.release();
   progress.release();
+  mail.release();
+  mail_word = 0;
   tdot.release();
   flags.release();
   valid = false;
