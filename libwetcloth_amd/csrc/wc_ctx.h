@@ -112,7 +112,9 @@ struct KTimer {
 // tile layout, where the cells a sweep step touches are consecutive.
 struct SweepPlan {
   bool valid = false;
-  int o[3] = {0, 0, 0}, B[3] = {0, 0, 0};
+  // box origin, extents of the DOFs it holds, and its size (B[0], B[1]: ext
+  // rounded up to whole tiles)
+  int o[3] = {0, 0, 0}, ext[3] = {0, 0, 0}, B[3] = {0, 0, 0};
   int ntile_a = 0, ntile_b = 0, ntiles = 0;
   int nsteps = 0;       // skewed steps per tile (B[2] + 30)
   int64_t ncell = 0;    // slots of the skewed tile layout
@@ -139,6 +141,7 @@ struct SweepPlan {
   DevBuf<double> mail;
   int mail_word = 0;
   int ndot = 0;                     // how many (tiles, or sub-tiles)
+  int nua = 0, nub = 0;             // sub-tiles that hold cells of ext
   // Sub-tile sweeps (one wave per 8x8 quarter of a tile, k_sweep_sub) or
   // the tile sweeps (k_sweep); both give the same values bit for bit
   bool sub = true;
@@ -170,6 +173,7 @@ struct GridSystem {
   const uint32_t* dofscan = nullptr;
   const uint32_t* rowlen = nullptr;
   const uint32_t* col = nullptr;
+  const uint8_t* live = nullptr;  // per DOF: its row holds a nonzero value
 };
 
 // Device work space of the MIC(0)-PCG solver (PCGSolver.h:310-314).
@@ -350,6 +354,7 @@ struct wc_ctx {
   wc::DevBuf<uint32_t> rowlen, col;
   wc::DevBuf<double> val, b, p;
   wc::DevBuf<int32_t> dof_level;
+  wc::DevBuf<uint8_t> dof_live;  // per DOF: its row holds a nonzero value
   int32_t level_min = 0, level_max = 0;
   wc::PcgWork pcg;
 
@@ -462,10 +467,8 @@ void grid_dof_cells(wc_ctx* ctx, int32_t* ijk, const int origin[3]);
 void grid_apply_pressure(wc_ctx* ctx, double dt);
 
 // ---- wc_sweep.hip ----
-void sweep_prepare(hipStream_t st, SweepPlan& P, const Grid& g, const uint8_t* act,
-                   const uint32_t* isdof, const uint32_t* dofscan,
-                   const uint32_t* rowlen, const uint32_t* col, const double* val,
-                   int64_t ndof);
+void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const double* val,
+                   const double* b, int64_t ndof);
 // MIC(0) factor of the prepared box (pipelined), into the sweep records
 void sweep_factor(hipStream_t st, SweepPlan& P, double tau, double mdr);
 // MIC(0) apply on box vectors: r (box) -> P.zb; the backward sweep also

@@ -1001,8 +1001,7 @@ bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,
   }
   const double tolr = tol * res;
   if (w.use_sweeps && w.grid.g)
-    sweep_prepare(st, w.sweep, *w.grid.g, w.grid.act, w.grid.isdof, w.grid.dofscan,
-                  w.grid.rowlen, w.grid.col, A.val, n);
+    sweep_prepare(st, w.sweep, w.grid, A.val, b, n);
   if (w.sweep.valid) {
     sweep_factor(st, w.sweep, tau, mdr);
     if (sweep_aborted(st, w.sweep))

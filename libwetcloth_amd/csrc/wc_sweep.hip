@@ -164,6 +164,7 @@ __host__ __device__ inline int64_t skew_slot(const Skew& K, int a, int b, int li
 struct BoxArgs {
   Grid g;
   int o[3];        // box origin (dense node coordinates)
+  int ext[3];      // extents of the DOFs in the box
   Skew K;
   int64_t nslot;
   const uint8_t* act;
@@ -186,15 +187,27 @@ struct BoxArgs {
   FacIn* fin;    // factor pass inputs
 };
 
-// Bounding box of the DOF nodes: each block strides over the nodes, reduces
-// its threads' bounds through shuffles and LDS, and issues one set of six
-// atomics (the grid is bounded, so a few thousand atomics in all).
+// Bounding box of the DOF nodes whose row or rhs is not empty: each block
+// strides over the nodes, reduces its threads' bounds through shuffles and
+// LDS, and issues one set of six atomics (the grid is bounded, so a few
+// thousand atomics in all).
+// The reference's DOF set also holds cells inside the solid along the border
+// of the activated buckets, 7 cells out from the liquid, whose rows hold
+// only zeros and whose rhs is zero (5 % of the DOFs at 256^3, half of them at
+// 16^3).  Such a row is a null column of the factor (PCGSolver.h:141), its
+// preconditioned value, its product and its solution are zero, and it
+// couples to nothing: the box is drawn around the other DOFs, and the ones
+// outside it keep the zeros of the solution's clear.
 constexpr int kBoxBlocks = 2048;
-__global__ __launch_bounds__(256) void k_dof_box(Grid g, const uint32_t* isdof, int* bb) {
+__global__ __launch_bounds__(256) void k_dof_box(Grid g, const uint32_t* isdof,
+                                                 const uint32_t* dofscan, const uint8_t* live,
+                                                 const double* b, int* bb) {
   __shared__ int sh[6][4];
   int lo[3] = {1 << 30, 1 << 30, 1 << 30}, hi[3] = {-1, -1, -1};
   for (int64_t n = blockIdx.x * 256ll + threadIdx.x; n < g.nnode; n += (int64_t)gridDim.x * 256) {
     if (!isdof[n]) continue;
+    const uint32_t me = dofscan[n];
+    if (!live[me] && b[me] == 0) continue;
     int c[3];
     node_coords(g, n, c[0], c[1], c[2]);
     for (int d = 0; d < 3; ++d) {
@@ -285,6 +298,8 @@ __global__ __launch_bounds__(256) void k_row_sums(BoxArgs A, RowSum* S) {
     int c[3];
     node_coords(g, n, c[0], c[1], c[2]);
     const int x = c[0] - A.o[0], y = c[1] - A.o[1], z = c[2] - A.o[2];
+    // (a DOF outside the box has an empty row)
+    if (x < 0 || y < 0 || z < 0 || x >= A.ext[0] || y >= A.ext[1] || z >= A.ext[2]) continue;
     const int li = x % kT, lj = y % kT;
     const int64_t t = skew_slot(A.K, x / kT, y / kT, li, lj, z + li + lj);
     const uint32_t me = A.dofscan[n];
@@ -893,6 +908,7 @@ enum { K_FWD = 0, K_BWD = 1, K_FAC = 2 };
 template <class V>
 struct SweepArgs {
   Skew K;
+  int nua, nub;            // sub-tiles that hold DOFs
   int ntiles;
   const uint32_t* order;   // ticket -> a | b << 16
   const CellT<V>* cells;   // forward: lower terms; backward: upper terms
@@ -1549,11 +1565,11 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   const int Bz = S.K.Bz;
   const int nsteps = S.K.nsteps;
   const int nb = (nsteps + kNB - 1) / kNB;
-  const int nsa = 2 * S.K.ntile_a;
   auto PL = [](int w) -> uint32_t { return (uint32_t)(w & (kSubPlanes - 1)) * kPlane; };
   const int sgn = BWD ? -kThreads : kThreads;
-  // The unit (A, B), counted from the sweep's start corner.  The grid has
-  // one workgroup per ticket.
+  // The unit (A, B) = (A0 + ua, B0 + ub), counted from the sweep's start
+  // corner, (A0, B0) being the first that holds DOFs.  The grid has one
+  // workgroup per ticket.
   if (threadIdx.x == 0) {
     const int t = atomicAdd(S.ticket, 1);
     sh.unit = (int)S.order[t];
@@ -1562,7 +1578,9 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   __syncthreads();
   const int unit = __builtin_amdgcn_readfirstlane(sh.unit);
   // its tile and quarter in the sweep's frame and the physical ones
-  const int A = unit & 0xFFFF, B = unit >> 16;
+  const int ua = unit & 0xFFFF, ub = unit >> 16;
+  const int A = ua + (BWD ? 2 * S.K.ntile_a - S.nua : 0);
+  const int B = ub + (BWD ? 2 * S.K.ntile_b - S.nub : 0);
   const int sa = A & 1, sb = B & 1;
   const int a = BWD ? S.K.ntile_a - 1 - (A >> 1) : A >> 1;
   const int b = BWD ? S.K.ntile_b - 1 - (B >> 1) : B >> 1;
@@ -1576,9 +1594,9 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     return tile0 + (uint32_t)wp * kThreads +
            (uint32_t)((kS * psb + (p >> 3)) * kT + kS * psa + (p & 7));
   };
-  // a unit's mail records: (step * kMail) from here
-  auto mail_of = [&](int UA, int UB) -> uint32_t {
-    return (uint32_t)((UB * nsa + UA) * nb * kNB) * kMail;
+  // the mail records of unit (ua, ub): (step * kMail) from here
+  auto mail_of = [&](int uA, int uB) -> uint32_t {
+    return (uint32_t)((uB * S.nua + uA) * nb * kNB) * kMail;
   };
   if (wave == 2) {
     // loader; every batch issues the same operations, so the counter waits
@@ -1646,9 +1664,9 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     const bool xf = lane < kNB * kS;
     const int st = (lane / kS) % kNB, m = lane % kS;
     const int li = xf ? kS * sa : kS * sa + m, lj = xf ? kS * sb + m : kS * sb;
-    const bool up = xf ? A > 0 : B > 0;
+    const bool up = xf ? ua > 0 : ub > 0;
     const int ahead = (xf ? sa : sb) ? -1 : kT - 1;
-    const V* const src = S.mail + (up ? mail_of(xf ? A - 1 : A, xf ? B : B - 1) +
+    const V* const src = S.mail + (up ? mail_of(xf ? ua - 1 : ua, xf ? ub : ub - 1) +
                                             (uint32_t)(xf || m == kS - 1 ? m % kS : kS + m)
                                       : 0u);
     const int off = li + lj;
@@ -1734,7 +1752,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
       const int w = n * kNB + lane / per;
       if (lane < kClear && w < nsteps)
         *reinterpret_cast<U4*>(reinterpret_cast<char*>(
-            at(S.mail_reset, mail_of(A, B) + (uint32_t)w * kMail)) + lane % per * 16) =
+            at(S.mail_reset, mail_of(ua, ub) + (uint32_t)w * kMail)) + lane % per * 16) =
             U4{~0u, ~0u, ~0u, ~0u};
     };
     const uint32_t cown = cell(lane);
@@ -1770,7 +1788,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
       // physical quarter's index
 #pragma unroll
       for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
-      if (lane == 0) S.dot_out[(2 * b + psb) * nsa + 2 * a + psa] = dot;
+      if (lane == 0) S.dot_out[(2 * b + psb) * S.nua + 2 * a + psa] = dot;
     }
     return;
   }
@@ -1784,7 +1802,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   // instruction for all lanes, with no change of the execution mask)
   const bool mailer = ui == kS - 1 || uj == kS - 1;
   const __amdgpu_buffer_rsrc_t mail_buf = __builtin_amdgcn_make_buffer_rsrc(
-      S.mail + mail_of(A, B), 0, nb * kNB * kMail * (int)sizeof(V), 0x00020000);
+      S.mail + mail_of(ua, ub), 0, nb * kNB * kMail * (int)sizeof(V), 0x00020000);
   const uint32_t mail_off =
       mailer ? (uint32_t)(ui == kS - 1 ? uj : kS + ui) * (uint32_t)sizeof(V) : 0x40000000u;
   // A batch's records are read from the ring during the batch before it
@@ -1867,27 +1885,28 @@ Skew skew_of(const SweepPlan& P) {
 
 }  // namespace
 
-void sweep_prepare(hipStream_t st, SweepPlan& P, const Grid& g, const uint8_t* act,
-                   const uint32_t* isdof, const uint32_t* dofscan,
-                   const uint32_t* rowlen, const uint32_t* col, const double* val,
-                   int64_t ndof) {
+void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const double* val,
+                   const double* b, int64_t ndof) {
+  const Grid& g = *G.g;
   P.valid = false;
   if (ndof == 0) return;
   P.flags.ensure(8);
   int init[6] = {1 << 30, 1 << 30, 1 << 30, -1, -1, -1};
   WC_HIP(hipMemcpyAsync(P.flags.p, init, sizeof(init), hipMemcpyHostToDevice, st));
   hipLaunchKernelGGL(k_dof_box, dim3((unsigned)std::min<int64_t>(kBoxBlocks, blocks(g.nnode, 256))),
-                     dim3(256), 0, st, g, isdof, P.flags.p);
+                     dim3(256), 0, st, g, G.isdof, G.dofscan, G.live, b, P.flags.p);
   WC_LAUNCH_CHECK();
   int bb[6];
   WC_HIP(hipMemcpyAsync(bb, P.flags.p, sizeof(bb), hipMemcpyDeviceToHost, st));
   WC_HIP(hipStreamSynchronize(st));
+  if (bb[3] < 0) return;  // every row and the rhs are empty
   for (int d = 0; d < 3; ++d) {
     P.o[d] = bb[d];
-    int ext = bb[3 + d] - bb[d] + 1;
-    if (d < 2) ext = (ext + kT - 1) / kT * kT;
-    P.B[d] = ext;
+    P.ext[d] = bb[3 + d] - bb[d] + 1;
+    P.B[d] = d < 2 ? (P.ext[d] + kT - 1) / kT * kT : P.ext[d];
   }
+  P.nua = (P.ext[0] + kS - 1) / kS;
+  P.nub = (P.ext[1] + kS - 1) / kS;
   P.ntile_a = P.B[0] / kT;
   P.ntile_b = P.B[1] / kT;
   P.ntiles = P.ntile_a * P.ntile_b;
@@ -1925,18 +1944,21 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const Grid& g, const uint8_t* a
   P.order.ensure(P.ntiles);
   WC_HIP(hipMemcpyAsync(P.order.p, order.data(), sizeof(uint32_t) * P.ntiles,
                         hipMemcpyHostToDevice, st));
-  // sub-tile tickets in (A+B, A) order over the 2 ntile_a x 2 ntile_b units
+  // sub-tile tickets in (A+B, A) order over the units that hold DOFs
   std::vector<uint32_t> order_sub;
-  const int nua = 2 * P.ntile_a, nub = 2 * P.ntile_b;
-  order_sub.reserve(4 * P.ntiles);
+  const int nua = P.nua, nub = P.nub;
+  order_sub.reserve(nua * nub);
   for (int s = 0; s <= nua + nub - 2; ++s)
     for (int A = 0; A < nua; ++A) {
       const int B = s - A;
       if (B >= 0 && B < nub) order_sub.push_back((uint32_t)A | ((uint32_t)B << 16));
     }
-  P.order_sub.ensure(4 * P.ntiles);
-  WC_HIP(hipMemcpyAsync(P.order_sub.p, order_sub.data(), sizeof(uint32_t) * 4 * P.ntiles,
+  P.order_sub.ensure(order_sub.size());
+  WC_HIP(hipMemcpyAsync(P.order_sub.p, order_sub.data(), sizeof(uint32_t) * order_sub.size(),
                         hipMemcpyHostToDevice, st));
+  // (the units without DOFs are never run: their slots of the outputs stay 0)
+  if (P.nua < 2 * P.ntile_a || P.nub < 2 * P.ntile_b)
+    WC_HIP(hipMemsetAsync(P.zb.p, 0, sizeof(double) * P.ncell, st));
   P.progress.ensure(8);
   P.tdot.ensure(4 * P.ntiles);
   // tickets and the abort flag start at zero (the abort flag is cleared
@@ -1946,14 +1968,17 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const Grid& g, const uint8_t* a
   P.mail_word = 0;
   BoxArgs A;
   A.g = g;
-  for (int d = 0; d < 3; ++d) A.o[d] = P.o[d];
+  for (int d = 0; d < 3; ++d) {
+    A.o[d] = P.o[d];
+    A.ext[d] = P.ext[d];
+  }
   A.K = skew_of(P);
   A.nslot = P.ncell;
-  A.act = act;
-  A.isdof = isdof;
-  A.dofscan = dofscan;
-  A.rowlen = rowlen;
-  A.col = col;
+  A.act = G.act;
+  A.isdof = G.isdof;
+  A.dofscan = G.dofscan;
+  A.rowlen = G.rowlen;
+  A.col = G.col;
   A.val = val;
   A.pdof = P.pdof.p;
   A.code = P.code.p;
@@ -1989,6 +2014,8 @@ template <class V>
 static SweepArgs<V> sweep_args(SweepPlan& P) {
   SweepArgs<V> S = {};
   S.K = skew_of(P);
+  S.nua = P.nua;
+  S.nub = P.nub;
   S.ntiles = P.ntiles;
   S.order = P.order.p;
   S.code = P.scode.p;
@@ -2027,6 +2054,9 @@ void sweep_narrow(hipStream_t st, SweepPlan& P) {
   P.rb32.ensure(P.ncell);
   P.sb32.ensure(P.ncell);
   P.bb.ensure(P.ncell);
+  if (P.nua < 2 * P.ntile_a || P.nub < 2 * P.ntile_b) {  // as for zb in sweep_prepare
+    WC_HIP(hipMemsetAsync(P.zb32.p, 0, sizeof(float) * P.ncell, st));
+  }
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cf.p,
                      P.cf32.p, nrec);
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cb.p,
@@ -2057,7 +2087,7 @@ static void fill_sentinel(hipStream_t st, void* p, int64_t words) {
 
 // values of one pass's mail: a record per unit and step (whole batches)
 static int64_t mail_values(const SweepPlan& P) {
-  return 4ll * P.ntiles * ((P.nsteps + kNB - 1) / kNB * kNB) * kMail;
+  return (int64_t)P.nua * P.nub * ((P.nsteps + kNB - 1) / kNB * kNB) * kMail;
 }
 
 // The mail of both passes (forward, then backward) in the plan's buffer,
@@ -2102,7 +2132,7 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   S.ticket = tick;
   S.next_ticket = tick + 1;
   if (sub) {
-    S.ntiles = 4 * P.ntiles;  // tickets: the sub-tile units
+    S.ntiles = P.nua * P.nub;  // tickets: the sub-tile units
     S.order = P.order_sub.p;
     S.reset = nullptr;
     S.mail = mail;

@@ -209,3 +209,29 @@ def test_kernel_timing_counts_launches(oracle, wc):
     for k in ("p2g", "g2p"):
         ms, nl, units = st[k]
         assert nl == 1 and units == np_ and ms > 0
+
+
+@pytest.mark.parametrize("n,block_hi", [
+    (16, (0.2, 0.2, 0.3)),    # a few cells: one unit, most DOFs empty rows outside the box
+    (20, (0.45, 0.4, 0.5)),   # extents just past a unit (9 = 8 + 1 cells)
+    (33, (0.55, 0.8, 0.3)),   # more units in y than in x, the last ones trimmed
+    (48, (0.36, 0.25, 0.9)),  # 17 cells: a second tile with one unit of DOFs
+])
+def test_box_without_empty_rows(oracle, wc, n, block_hi):
+    """The box is drawn around the rows that hold a value; the DOFs outside it
+    (empty rows) get zeros.  Apply and multiply stay the oracle's bit for bit
+    over all DOFs, and a whole solve leaves the empty rows' pressure at zero."""
+    s = prepared(wc, oracle, n, block_hi=block_hi)
+    ok, it, res, p, val, b = solve(s, True)
+    assert ok
+    rs, col, val, b, p = s.system()
+    rows = np.repeat(np.arange(len(b)), np.diff(rs.astype(np.int64)))
+    empty = np.bincount(rows, weights=(val != 0), minlength=len(b)) == 0
+    assert empty.any() and (b[empty] == 0).all() and (p[empty] == 0).all()
+    r = np.random.default_rng(n).standard_normal(len(b))
+    invdiag, lv = oracle.mic0(rs, col, val)
+    want = oracle.apply_precond(rs, col, invdiag, lv, r)
+    for sub in (1, 0, 1):
+        s.set_option("sweep_subtiles", sub)
+        assert np.array_equal(s.apply_preconditioner(r), want), sub
+    assert np.array_equal(s.multiply(r), oracle.spmv(rs, col, val, r))

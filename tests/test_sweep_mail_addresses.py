@@ -13,42 +13,56 @@ import pytest
 KT, KS, KNB, KMAIL, KTHREADS, KPLANES = 16, 8, 4, 16, 256, 8
 
 
-def mail_of(A, B, nsa, nsteps):
-    return (B * nsa + A) * (-(-nsteps // KNB) * KNB) * KMAIL  # whole batches
+def mail_of(ua, ub, nua, nsteps):
+    return (ub * nua + ua) * (-(-nsteps // KNB) * KNB) * KMAIL  # whole batches
 
 
-@pytest.mark.parametrize("na,nb_,Bz", [(1, 1, 1), (1, 1, 3), (2, 1, 2), (1, 3, 7), (2, 2, 9),
-                                       (3, 2, 16), (2, 3, 33)])
-def test_mail_records(na, nb_, Bz):
-    nsa, nsb, nsteps = 2 * na, 2 * nb_, Bz + 2 * (KT - 1)
-    size = mail_of(0, nsb, nsa, nsteps)
+EXTENTS = [(1, 1, 1), (8, 9, 3), (17, 7, 2), (16, 41, 7), (32, 25, 9), (40, 31, 16), (24, 33, 33)]
+
+
+def units(ex, ey, bwd):
+    """The units that hold cells of an ex x ey box: (ua, ub) with the unit (A, B)
+    of the sweep's frame, counted from its start corner over whole tiles."""
+    nua, nub = -(-ex // KS), -(-ey // KS)
+    na, nb_ = -(-ex // KT), -(-ey // KT)
+    a0, b0 = (2 * na - nua, 2 * nb_ - nub) if bwd else (0, 0)
+    return na, nb_, nua, nub, [(ua, ub, a0 + ua, b0 + ub)
+                               for ua, ub in itertools.product(range(nua), range(nub))]
+
+
+@pytest.mark.parametrize("bwd", [False, True])
+@pytest.mark.parametrize("ex,ey,Bz", EXTENTS)
+def test_mail_records(ex, ey, Bz, bwd):
+    nsteps = Bz + 2 * (KT - 1)
+    na, nb_, nua, nub, todo = units(ex, ey, bwd)
+    size = mail_of(0, nub, nua, nsteps)
     # what each entry holds: the cell (x, y, kk) in the sweep's frame, and its step
     entry = {}
-    for A, B in itertools.product(range(nsa), range(nsb)):
+    for ua, ub, A, B in todo:
         for lane in range(64):
             ui, uj = lane & 7, lane >> 3
             if ui != KS - 1 and uj != KS - 1:
                 continue
             li, lj = KS * (A & 1) + ui, KS * (B & 1) + uj
             for w in range(-(-nsteps // KNB) * KNB):
-                e = mail_of(A, B, nsa, nsteps) + (uj if ui == KS - 1 else KS + ui) + w * KMAIL
+                e = mail_of(ua, ub, nua, nsteps) + (uj if ui == KS - 1 else KS + ui) + w * KMAIL
                 assert 0 <= e < size and e not in entry
                 entry[e] = (KT * (A >> 1) + li, KT * (B >> 1) + lj, w - li - lj)
     reads = 0
     nbat = (nsteps + KNB - 1) // KNB
-    for A, B in itertools.product(range(nsa), range(nsb)):
+    for ua, ub, A, B in todo:
         sa, sb = A & 1, B & 1
         for lane in range(64):
             xf, st, m = lane < KNB * KS, (lane // KS) % KNB, lane % KS
             li, lj = (KS * sa, KS * sb + m) if xf else (KS * sa + m, KS * sb)
-            up = A > 0 if xf else B > 0
+            up = ua > 0 if xf else ub > 0
             ahead = -1 if (sa if xf else sb) else KT - 1
             off = li + lj
             for n in range(nbat):
                 w = n * KNB + st
                 if not (up and w < nsteps and off <= w and w - off < Bz):
                     continue
-                src = mail_of(A - 1, B, nsa, nsteps) if xf else mail_of(A, B - 1, nsa, nsteps)
+                src = mail_of(ua - 1, ub, nua, nsteps) if xf else mail_of(ua, ub - 1, nua, nsteps)
                 src += m if (xf or m == KS - 1) else KS + m
                 e = src + (w + ahead) * KMAIL
                 assert 0 <= w + ahead < nsteps
@@ -56,30 +70,33 @@ def test_mail_records(na, nb_, Bz):
                 assert entry[e] == ((x - 1, y, kk) if xf else (x, y - 1, kk))
                 reads += 1
     # every face between two units, once per cell of its pencils
-    assert reads == ((nsa - 1) * nsb + (nsb - 1) * nsa) * KS * Bz
+    assert reads == ((nua - 1) * nub + (nub - 1) * nua) * KS * Bz
 
 
 @pytest.mark.parametrize("word", [4, 8])
 @pytest.mark.parametrize("bwd", [False, True])
-@pytest.mark.parametrize("na,nb_,Bz", [(1, 1, 1), (2, 1, 2), (1, 2, 7), (2, 2, 9)])
-def test_resets_and_output(na, nb_, Bz, bwd, word):
-    nsa, nsb, nsteps = 2 * na, 2 * nb_, Bz + 2 * (KT - 1)
+@pytest.mark.parametrize("ex,ey,Bz", EXTENTS[:5])
+def test_resets_and_output(ex, ey, Bz, bwd, word):
+    nsteps = Bz + 2 * (KT - 1)
+    na, nb_, nua, nub, todo = units(ex, ey, bwd)
     nbat = (nsteps + KNB - 1) // KNB
-    reset = np.zeros(mail_of(0, nsb, nsa, nsteps) * word, dtype=int)
+    reset = np.zeros(mail_of(0, nub, nua, nsteps) * word, dtype=int)
     out = np.zeros(na * nb_ * nsteps * KTHREADS, dtype=int)
+    dots = []
     vec = 16 // word
     per = 64 // vec
-    for A, B in itertools.product(range(nsa), range(nsb)):
+    for ua, ub, A, B in todo:
         sa, sb = A & 1, B & 1
         a, b = (na - 1 - (A >> 1), nb_ - 1 - (B >> 1)) if bwd else (A >> 1, B >> 1)
         psa, psb = (1 - sa, 1 - sb) if bwd else (sa, sb)
         tile0 = (b * na + a) * nsteps * KTHREADS
+        dots.append((2 * b + psb) * nua + 2 * a + psa)
         for n in range(nbat):
             words = KNB * KMAIL * word // 16
             for lane in range(words):
                 w = n * KNB + lane // (words // KNB)
                 if w < nsteps:
-                    at = (mail_of(A, B, nsa, nsteps) + w * KMAIL) * word
+                    at = (mail_of(ua, ub, nua, nsteps) + w * KMAIL) * word
                     at += lane % (words // KNB) * 16
                     reset[at:at + 16] += 1
             for j, lane in itertools.product(range(KNB * per // 64), range(64)):
@@ -99,5 +116,12 @@ def test_resets_and_output(na, nb_, Bz, bwd, word):
                 # stored during batch n + 1; the plane is next written by step w + 8,
                 # and its halos (read by step w + 9) one batch before that step's
                 assert (w + KPLANES) // KNB > n + 1 and (w + KPLANES + 1) // KNB - 1 >= n + 1
-    per_unit = reset.reshape(nsa * nsb, -1)[:, :nsteps * KMAIL * word]
-    assert (per_unit == 1).all() and reset.max() == 1 and (out == 1).all()
+    per_unit = reset.reshape(nua * nub, -1)[:, :nsteps * KMAIL * word]
+    assert (per_unit == 1).all() and reset.max() == 1
+    # every slot of the box's cells once, and no slot twice; one partial per unit
+    slot = np.arange(out.size)
+    lane, tile = slot % KTHREADS, slot // KTHREADS // nsteps
+    x, y = tile % na * KT + lane % KT, tile // na * KT + lane // KT
+    inside = (x < nua * KS) & (y < nub * KS)
+    assert (out == inside).all()
+    assert sorted(dots) == list(range(nua * nub))
