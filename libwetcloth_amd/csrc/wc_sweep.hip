@@ -1468,10 +1468,10 @@ __global__ __launch_bounds__(SweepBlock<KIND>::value) void k_sweep(SweepArgs<V> 
 // sees it), and the only barriers are those that hand over a batch of kNB
 // steps of records and face values from the loader and face waves.
 //
-// A sub-tile (sa, sb) of tile (a, b) runs every step w of the tile, 0 ..
-// nsteps - 1, for its 64 pencils (li, lj) = (8 sa + ui, 8 sb + uj): the
-// steps outside its pencils' cells are padding, which it writes as +0 like
-// every other slot, so each slot of the box is still written once per pass.
+// A sub-tile (sa, sb) of tile (a, b) runs the tile's steps from 8 (sa + sb)
+// on (its step 0) for its 64 pencils (li, lj) = (8 sa + ui, 8 sb + uj), Bz +
+// 14 of them rounded up to whole batches; slots of other steps are padding,
+// which keep the plan's zeros.
 // Units are claimed by ticket in (A + B, A) order over the sub-tile grid
 // (A, B) = (2 a + sa, 2 b + sb), one unit per workgroup, and a unit waits
 // only for the units at (A - 1, B) and (A, B - 1).
@@ -1498,6 +1498,9 @@ constexpr int kSubPlanes = 8;     // exchange planes (step % 8), two batches
 constexpr int kSubThreads = 256;  // compute, face, loader and store waves
 constexpr int kMail = 2 * kS;     // values of a mail record (the last unused)
 
+// batches of a unit: its pencils' cells lie on Bz + 2 (kS - 1) steps
+__host__ __device__ inline int sub_batches(int Bz) { return (Bz + 2 * (kS - 1) + kNB - 1) / kNB; }
+
 template <class V>
 struct SubRing {
   static constexpr int kCellOps = kNB * 64 * (int)sizeof(CellT<V>) / 1024;
@@ -1505,7 +1508,10 @@ struct SubRing {
   static constexpr int kOpOps = kNB * 64 * 4 / 1024;
   static constexpr int kFwdLoads = kCellOps + kRhsOps + kOpOps;
   static constexpr int kBwdLoads = kFwdLoads + kRhsOps;  // and r for z . r
-  // ring depth (batches, a power of two): 64 KB of factor records
+  // ring depth in batches, a power of two: 64 KB of factor records.  (One
+  // unit per compute unit then; half the ring and two units measured slower
+  // at 256^3, whose 340 units exceed the 256 compute units: FP32 126 / 128
+  // against 114 / 118 us, FP64 190 / 190 against 143 / 153.)
   static constexpr int kBatches = 64 * 1024 / (kNB * 64 * (int)sizeof(CellT<V>));
   // batches loaded ahead: as many as the 6-bit load counter and the ring allow
   static constexpr int ahead() {
@@ -1564,7 +1570,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   const int lane = threadIdx.x & 63;
   const int Bz = S.K.Bz;
   const int nsteps = S.K.nsteps;
-  const int nb = (nsteps + kNB - 1) / kNB;
+  const int nb = sub_batches(Bz);
   auto PL = [](int w) -> uint32_t { return (uint32_t)(w & (kSubPlanes - 1)) * kPlane; };
   const int sgn = BWD ? -kThreads : kThreads;
   // The unit (A, B) = (A0 + ua, B0 + ub), counted from the sweep's start
@@ -1585,11 +1591,13 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   const int a = BWD ? S.K.ntile_a - 1 - (A >> 1) : A >> 1;
   const int b = BWD ? S.K.ntile_b - 1 - (B >> 1) : B >> 1;
   const int psa = BWD ? 1 - sa : sa, psb = BWD ? 1 - sb : sb;
-  // the unit's 64 slots of step w are 8 rows of 8 consecutive slots
-  // (physical order p = row * 8 + column); steps past the end give the last
+  // the unit's 64 slots of its step w are 8 rows of 8 consecutive slots
+  // (physical order p = row * 8 + column); steps past the tile's end give its
+  // last
+  const int w0 = kS * (sa + sb), wend = nsteps - w0;
   const uint32_t tile0 = (uint32_t)skew_slot(S.K, a, b, 0, 0, 0);
   auto slot = [&](int w, int p) -> uint32_t {
-    const int wc = w < nsteps ? w : nsteps - 1;
+    const int wc = w < wend ? w0 + w : nsteps - 1;
     const int wp = BWD ? nsteps - 1 - wc : wc;
     return tile0 + (uint32_t)wp * kThreads +
            (uint32_t)((kS * psb + (p >> 3)) * kT + kS * psa + (p & 7));
@@ -1656,31 +1664,32 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   if (wave == 1) {
     // face wave: lane (face, step, row) takes one value of the batch, from
     // the x-upstream unit's record entry m (row m's pencil) or the
-    // y-upstream unit's entry of column m.  Both upstream pencils lie one
-    // step back inside a tile and, the steps of a tile being counted from
-    // its own corner, kT - 1 steps on across tiles.  The read of batch n + 2
-    // is issued when batch n + 1 is published, during batch n.
+    // y-upstream unit's entry of column m.  The upstream pencil lies kS - 1
+    // of its unit's steps on.  The read of batch n + 2 is issued when batch
+    // n + 1 is published, during batch n.
     static_assert(2 * kNB * kS == 64, "a batch's face values fill the wave");
     const bool xf = lane < kNB * kS;
     const int st = (lane / kS) % kNB, m = lane % kS;
     const int li = xf ? kS * sa : kS * sa + m, lj = xf ? kS * sb + m : kS * sb;
     const bool up = xf ? ua > 0 : ub > 0;
-    const int ahead = (xf ? sa : sb) ? -1 : kT - 1;
     const V* const src = S.mail + (up ? mail_of(xf ? ua - 1 : ua, xf ? ub : ub - 1) +
-                                            (uint32_t)(xf || m == kS - 1 ? m % kS : kS + m)
+                                            (uint32_t)((kS - 1) * kMail) +
+                                            (uint32_t)(xf || m == kS - 1 ? m : kS + m)
                                       : 0u);
-    const int off = li + lj;
     // the halo cell beside the pencil in the exchange plane
     const uint32_t halo = (uint32_t)(xf ? (lj + 1) * (kT + 1) + li : lj * (kT + 1) + li + 1);
     // the pencil has a cell at step w and an upstream value beside it
-    auto need = [&](int w) -> bool { return up && w < nsteps && w >= off && w - off < Bz; };
+    auto need = [&](int w) -> bool { return up && w >= m && w - m < Bz; };
     V fv = (V)0;
     auto fetch = [&](int n) {
       const int w = n * kNB + st;
-      fv = need(w) ? load_coherent(at(src, (uint32_t)((w + ahead) * kMail))) : (V)0;
+      fv = need(w) ? load_coherent(at(src, (uint32_t)(w * kMail))) : (V)0;
     };
     // batch n's values into the halos of the planes its steps read;
-    // a value still the sentinel is read again (bounded wait)
+    // a value still the sentinel is read again (bounded wait).  One read at a
+    // time, none ahead of its turn: reads of records being written delay
+    // the stores to them (a batch read two batches ahead and again when it
+    // was too early: 112 / 118 -> 191 / 191 us at 256^3 FP32)
     auto publish = [&](int n) {
       const int w = n * kNB + st;
       const bool nd = need(w);
@@ -1689,16 +1698,16 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
       if (__any(nd && is_sentinel(fv))) {
         long long spins = 0;
         for (;;) {
-          if (++spins > kSpinLimit || load_flag(S.abort_flag)) {
+          if ((++spins & 1023) == 0 && (spins > kSpinLimit || load_flag(S.abort_flag))) {
             store_flag(S.abort_flag, 1);
             fv = (V)0;
             break;
           }
-          if (nd && is_sentinel(fv)) fv = load_coherent(at(src, (uint32_t)((w + ahead) * kMail)));
+          if (nd && is_sentinel(fv)) fv = load_coherent(at(src, (uint32_t)(w * kMail)));
           if (!__any(nd && is_sentinel(fv))) break;
         }
       }
-      if (w < nsteps) pl[PL(w - 1) + halo] = nd ? fv : (V)0;
+      pl[PL(w - 1) + halo] = nd ? fv : (V)0;
     };
     // batch 0 is due at the first batch's barrier
     fetch(0);
@@ -1737,7 +1746,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
 #pragma unroll
       for (int j = 0; j < kOps; ++j) {
         const int w = n * kNB + j * (64 / kPer) + lane / kPer, p = lane % kPer * kVec;
-        if (w < nsteps) {
+        if (w < wend) {
           Quad q;
 #pragma unroll
           for (int k = 0; k < kVec; ++k) q.v[k] = pl[PL(w) + cell(BWD ? 63 - (p + k) : p + k)];
@@ -1750,7 +1759,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     auto clear = [&](int n) {
       constexpr int per = kClear / kNB;  // words per step
       const int w = n * kNB + lane / per;
-      if (lane < kClear && w < nsteps)
+      if (lane < kClear)
         *reinterpret_cast<U4*>(reinterpret_cast<char*>(
             at(S.mail_reset, mail_of(ua, ub) + (uint32_t)w * kMail)) + lane % per * 16) =
             U4{~0u, ~0u, ~0u, ~0u};
@@ -1767,7 +1776,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
 #pragma unroll
       for (int st = 0; st < kNB; ++st) {
         const int w = n * kNB + st;
-        if (w < nsteps) dot += (double)pl[PL(w) + cown] * (double)rsave[st];
+        if (w < wend) dot += (double)pl[PL(w) + cown] * (double)rsave[st];
       }
     };
     __syncthreads();
@@ -1842,8 +1851,6 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     __syncthreads();
 #pragma unroll
     for (int st = 0; st < kNB; ++st) {
-      // (the steps past nsteps of the last batch run too: nothing reads
-      // their plane cells or their records)
       const V* const prev = pl + PL(w0 + st + kSubPlanes - 1);
       const V v0 = *lds_at(prev, cur.src[st][0]), v1 = *lds_at(prev, cur.src[st][1]),
               v2 = *lds_at(prev, cur.src[st][2]);
@@ -1956,9 +1963,9 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const doub
   P.order_sub.ensure(order_sub.size());
   WC_HIP(hipMemcpyAsync(P.order_sub.p, order_sub.data(), sizeof(uint32_t) * order_sub.size(),
                         hipMemcpyHostToDevice, st));
-  // (the units without DOFs are never run: their slots of the outputs stay 0)
-  if (P.nua < 2 * P.ntile_a || P.nub < 2 * P.ntile_b)
-    WC_HIP(hipMemsetAsync(P.zb.p, 0, sizeof(double) * P.ncell, st));
+  // (the sub-tile sweeps write no slot outside their units' steps: those
+  // keep this zero, and the factor's in zf)
+  WC_HIP(hipMemsetAsync(P.zb.p, 0, sizeof(double) * P.ncell, st));
   P.progress.ensure(8);
   P.tdot.ensure(4 * P.ntiles);
   // tickets and the abort flag start at zero (the abort flag is cleared
@@ -2054,9 +2061,8 @@ void sweep_narrow(hipStream_t st, SweepPlan& P) {
   P.rb32.ensure(P.ncell);
   P.sb32.ensure(P.ncell);
   P.bb.ensure(P.ncell);
-  if (P.nua < 2 * P.ntile_a || P.nub < 2 * P.ntile_b) {  // as for zb in sweep_prepare
-    WC_HIP(hipMemsetAsync(P.zb32.p, 0, sizeof(float) * P.ncell, st));
-  }
+  WC_HIP(hipMemsetAsync(P.zf32.p, 0, sizeof(float) * P.ncell, st));  // as in sweep_prepare
+  WC_HIP(hipMemsetAsync(P.zb32.p, 0, sizeof(float) * P.ncell, st));
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cf.p,
                      P.cf32.p, nrec);
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cb.p,
@@ -2087,7 +2093,7 @@ static void fill_sentinel(hipStream_t st, void* p, int64_t words) {
 
 // values of one pass's mail: a record per unit and step (whole batches)
 static int64_t mail_values(const SweepPlan& P) {
-  return (int64_t)P.nua * P.nub * ((P.nsteps + kNB - 1) / kNB * kNB) * kMail;
+  return (int64_t)P.nua * P.nub * sub_batches(P.B[2]) * kNB * kMail;
 }
 
 // The mail of both passes (forward, then backward) in the plan's buffer,

@@ -13,8 +13,13 @@ import pytest
 KT, KS, KNB, KMAIL, KTHREADS, KPLANES = 16, 8, 4, 16, 256, 8
 
 
-def mail_of(ua, ub, nua, nsteps):
-    return (ub * nua + ua) * (-(-nsteps // KNB) * KNB) * KMAIL  # whole batches
+def batches(Bz):
+    """Of a unit: its pencils' cells lie on Bz + 14 of the tile's steps."""
+    return (Bz + 2 * (KS - 1) + KNB - 1) // KNB
+
+
+def mail_of(ua, ub, nua, Bz):
+    return (ub * nua + ua) * batches(Bz) * KNB * KMAIL
 
 
 EXTENTS = [(1, 1, 1), (8, 9, 3), (17, 7, 2), (16, 41, 7), (32, 25, 9), (40, 31, 16), (24, 33, 33)]
@@ -33,9 +38,8 @@ def units(ex, ey, bwd):
 @pytest.mark.parametrize("bwd", [False, True])
 @pytest.mark.parametrize("ex,ey,Bz", EXTENTS)
 def test_mail_records(ex, ey, Bz, bwd):
-    nsteps = Bz + 2 * (KT - 1)
     na, nb_, nua, nub, todo = units(ex, ey, bwd)
-    size = mail_of(0, nub, nua, nsteps)
+    size = mail_of(0, nub, nua, Bz)
     # what each entry holds: the cell (x, y, kk) in the sweep's frame, and its step
     entry = {}
     for ua, ub, A, B in todo:
@@ -44,29 +48,24 @@ def test_mail_records(ex, ey, Bz, bwd):
             if ui != KS - 1 and uj != KS - 1:
                 continue
             li, lj = KS * (A & 1) + ui, KS * (B & 1) + uj
-            for w in range(-(-nsteps // KNB) * KNB):
-                e = mail_of(ua, ub, nua, nsteps) + (uj if ui == KS - 1 else KS + ui) + w * KMAIL
+            for w in range(batches(Bz) * KNB):
+                e = mail_of(ua, ub, nua, Bz) + (uj if ui == KS - 1 else KS + ui) + w * KMAIL
                 assert 0 <= e < size and e not in entry
-                entry[e] = (KT * (A >> 1) + li, KT * (B >> 1) + lj, w - li - lj)
+                entry[e] = (KT * (A >> 1) + li, KT * (B >> 1) + lj, w - ui - uj)
     reads = 0
-    nbat = (nsteps + KNB - 1) // KNB
     for ua, ub, A, B in todo:
         sa, sb = A & 1, B & 1
         for lane in range(64):
             xf, st, m = lane < KNB * KS, (lane // KS) % KNB, lane % KS
             li, lj = (KS * sa, KS * sb + m) if xf else (KS * sa + m, KS * sb)
             up = ua > 0 if xf else ub > 0
-            ahead = -1 if (sa if xf else sb) else KT - 1
-            off = li + lj
-            for n in range(nbat):
+            for n in range(batches(Bz)):
                 w = n * KNB + st
-                if not (up and w < nsteps and off <= w and w - off < Bz):
+                if not (up and w >= m and w - m < Bz):
                     continue
-                src = mail_of(ua - 1, ub, nua, nsteps) if xf else mail_of(ua, ub - 1, nua, nsteps)
-                src += m if (xf or m == KS - 1) else KS + m
-                e = src + (w + ahead) * KMAIL
-                assert 0 <= w + ahead < nsteps
-                x, y, kk = KT * (A >> 1) + li, KT * (B >> 1) + lj, w - off
+                e = mail_of(ua - 1, ub, nua, Bz) if xf else mail_of(ua, ub - 1, nua, Bz)
+                e += (KS - 1 + w) * KMAIL + (m if (xf or m == KS - 1) else KS + m)
+                x, y, kk = KT * (A >> 1) + li, KT * (B >> 1) + lj, w - m
                 assert entry[e] == ((x - 1, y, kk) if xf else (x, y - 1, kk))
                 reads += 1
     # every face between two units, once per cell of its pencils
@@ -79,8 +78,8 @@ def test_mail_records(ex, ey, Bz, bwd):
 def test_resets_and_output(ex, ey, Bz, bwd, word):
     nsteps = Bz + 2 * (KT - 1)
     na, nb_, nua, nub, todo = units(ex, ey, bwd)
-    nbat = (nsteps + KNB - 1) // KNB
-    reset = np.zeros(mail_of(0, nub, nua, nsteps) * word, dtype=int)
+    nbat = batches(Bz)
+    reset = np.zeros(mail_of(0, nub, nua, Bz) * word, dtype=int)
     out = np.zeros(na * nb_ * nsteps * KTHREADS, dtype=int)
     dots = []
     vec = 16 // word
@@ -89,21 +88,21 @@ def test_resets_and_output(ex, ey, Bz, bwd, word):
         sa, sb = A & 1, B & 1
         a, b = (na - 1 - (A >> 1), nb_ - 1 - (B >> 1)) if bwd else (A >> 1, B >> 1)
         psa, psb = (1 - sa, 1 - sb) if bwd else (sa, sb)
+        w0 = KS * (sa + sb)
         tile0 = (b * na + a) * nsteps * KTHREADS
         dots.append((2 * b + psb) * nua + 2 * a + psa)
         for n in range(nbat):
             words = KNB * KMAIL * word // 16
             for lane in range(words):
                 w = n * KNB + lane // (words // KNB)
-                if w < nsteps:
-                    at = (mail_of(ua, ub, nua, nsteps) + w * KMAIL) * word
-                    at += lane % (words // KNB) * 16
-                    reset[at:at + 16] += 1
+                at = (mail_of(ua, ub, nua, Bz) + w * KMAIL) * word
+                at += lane % (words // KNB) * 16
+                reset[at:at + 16] += 1
             for j, lane in itertools.product(range(KNB * per // 64), range(64)):
                 w, p = n * KNB + j * (64 // per) + lane // per, lane % per * vec
-                if w >= nsteps:
+                if w >= nsteps - w0:
                     continue
-                wp = nsteps - 1 - w if bwd else w
+                wp = nsteps - 1 - (w0 + w) if bwd else w0 + w
                 slot = tile0 + wp * KTHREADS + (KS * psb + (p >> 3)) * KT + KS * psa + (p & 7)
                 assert slot * word % 16 == 0
                 for k in range(vec):
@@ -116,12 +115,14 @@ def test_resets_and_output(ex, ey, Bz, bwd, word):
                 # stored during batch n + 1; the plane is next written by step w + 8,
                 # and its halos (read by step w + 9) one batch before that step's
                 assert (w + KPLANES) // KNB > n + 1 and (w + KPLANES + 1) // KNB - 1 >= n + 1
-    per_unit = reset.reshape(nua * nub, -1)[:, :nsteps * KMAIL * word]
-    assert (per_unit == 1).all() and reset.max() == 1
-    # every slot of the box's cells once, and no slot twice; one partial per unit
+    assert (reset == 1).all()
+    # every cell of the units' pencils is stored once, no slot twice, and what
+    # is stored besides is padding; one partial per unit
     slot = np.arange(out.size)
-    lane, tile = slot % KTHREADS, slot // KTHREADS // nsteps
+    lane, step, tile = slot % KTHREADS, slot // KTHREADS % nsteps, slot // KTHREADS // nsteps
     x, y = tile % na * KT + lane % KT, tile // na * KT + lane // KT
+    kk = step - lane % KT - lane // KT
     inside = (x < nua * KS) & (y < nub * KS)
-    assert (out == inside).all()
+    assert (out[inside & (kk >= 0) & (kk < Bz)] == 1).all()
+    assert (out[~inside] == 0).all() and out.max() == 1
     assert sorted(dots) == list(range(nua * nub))
