@@ -947,6 +947,7 @@ wc_status wc_apply_preconditioner(wc_ctx* c, const double* r, double* z) {
       wc::box_scatter(c->stream, P, P.zb.p, dz.p);
     } else {
       wc::pcg_apply(c->stream, c->pcg, system_csr(c), dr.p, dz.p);
+      wc::pcg_check(c->stream, c->pcg);
     }
     WC_HIP(hipMemcpyAsync(z, dz.p, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
     WC_HIP(hipStreamSynchronize(c->stream));
@@ -1610,6 +1611,7 @@ wc_status wc_mic0_apply_csr(int64_t n, const uint32_t* rowstart,
     dz.ensure(n);
     WC_HIP(hipMemcpyAsync(dr.p, r, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
     wc::pcg_apply(S.st, S.work, S.csr.A, dr.p, dz.p);
+    wc::pcg_check(S.st, S.work);
     WC_HIP(hipMemcpyAsync(z, dz.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
     WC_HIP(hipStreamSynchronize(S.st));
     dr.release();

@@ -190,12 +190,17 @@ struct PcgWork {
   SweepPlan sweep;
   DevBuf<double> invdiag, adiag, lv, r, z, s, x, partial, scal;
   DevBuf<uint32_t> tpos;
-  DevBuf<int> flags;  // [0] relaxation changed, [1] factor overflow, [2] max level
+  // [0], [1] tickets of the waiting passes, [2] factor overflow, max level,
+  // [3] bits: a wait ran out of its bound (F_ABORT), an entry has no transpose
+  DevBuf<int> flags;
   DevBuf<int32_t> level;
   DevBuf<uint32_t> lvl_count, lvl_cursor, lvl_list;
   std::vector<uint32_t> lvl_start;  // host copy: start of each level
   std::vector<uint32_t> lvl_size;
   int nlevels = 0;
+  int64_t nwaves = 0;     // the schedule's waves (their starts in lvl_cursor); 0: launch per level
+  int pass_waves = 0;     // resident waves of a waiting pass
+  bool lower_ready = false;  // adiag holds the lower solve's result, ready for the next apply
   const int32_t* level_in = nullptr;  // caller's per-row level, or null
   int32_t level_span = 0;
   bool levels_ready = false;
@@ -517,6 +522,8 @@ void pcg_factor(hipStream_t st, PcgWork& w, const DevCsr& A, double tau,
                 double mdr);
 void pcg_apply(hipStream_t st, PcgWork& w, const DevCsr& A, const double* r,
                double* z);
+// throws if one of the applies so far ran out of a wait's bound
+void pcg_check(hipStream_t st, PcgWork& w);
 void pcg_spmv(hipStream_t st, const DevCsr& A, const double* x, double* y);
 // PCGSolver::solve on device vectors b -> x; returns true when converged.
 bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,

@@ -3,9 +3,11 @@
 //
 // The factorization and both triangular solves are level-scheduled: rows are
 // grouped by their depth in the lower-triangular dependency graph (for the
-// pressure grid that is the i+j+k hyperplane) and each level is one launch in
-// which every row only reads rows of earlier levels.  Each row is computed in
-// gather ("left-looking") form, applying exactly the updates the reference's
+// pressure grid that is the i+j+k hyperplane), and a row only reads rows of
+// earlier levels.  One launch runs all levels of a pass: its waves take 64
+// rows of one level at a time by ticket, in level order, and wait for the
+// values they read (a matrix whose pattern is not symmetric is run with one
+// launch per level).  Each row is computed in gather ("left-looking") form, applying exactly the updates the reference's
 // column-sweeping loops apply to it and in the same order (ascending column),
 // so the factor and the preconditioned vector are bitwise the sequential
 // ones.  Inner products are two-stage block reductions in FP64 with a fixed
@@ -46,17 +48,82 @@ __device__ inline uint32_t upper_begin(const DevCsr& A, int64_t i, uint32_t b,
   return b;
 }
 
-__global__ void k_tpos_adiag(DevCsr A, uint32_t* tpos, double* adiag) {
+// The waiting passes: a value not yet written holds the all-ones NaN
+// sentinel, and every value another wave waits for is written once with an
+// agent-scope store, so a reader knows that it is final when it no longer
+// reads the sentinel.  A wave's rows belong to one level, so it never waits
+// for itself, and tickets are taken in an order in which every row a wave
+// waits for belongs to an earlier ticket: the wave with the first unfinished
+// ticket always runs.  Every wait is bounded (kPassSpins) and ends the pass
+// with F_ABORT set.
+constexpr int F_ABORT = 1, F_UNSYM = 2;  // bits of PcgWork::flags[3]
+constexpr int kPassSpins = 1 << 22;      // ~seconds; a correct run waits us
+constexpr unsigned long long kUnset = ~0ull;
+
+__device__ inline double load_agent(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool unset(double v) { return __double_as_longlong(v) == (long long)kUnset; }
+__device__ inline void store_agent(double* p, double v) {
+  if (unset(v)) v = __longlong_as_double(0x7FF8000000000000ll);  // another NaN
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ inline bool give_up(int& spins, int* flags) {
+  if (++spins <= kPassSpins &&
+      !(__hip_atomic_load(flags + 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & F_ABORT))
+    return false;
+  atomicOr(flags + 3, F_ABORT);
+  return true;
+}
+// the value at p once it is set (0 after an abort), v being its first read
+__device__ inline double settle(double v, const double* p, int* flags) {
+  int spins = 0;
+  while (unset(v)) {
+    if ((spins & 63) == 63 && give_up(spins, flags)) return 0.0;
+    ++spins;
+    __builtin_amdgcn_s_sleep(1);
+    v = load_agent(p);
+  }
+  return v;
+}
+
+// The next wave of the schedule: its ticket t, and through start / count its
+// rows list[start, start + count).  The counters are taken one ahead, so the
+// atomic's round trip is hidden by the rows in hand.
+// A loop over tickets ends its body with whole(): the lanes without a row
+// must not go round before the others (given a divergent continue, the
+// compiler nests a loop of the continuing lanes alone, whose first lane then
+// is not the one that holds the ticket).
+__device__ inline void whole() { __builtin_amdgcn_wave_barrier(); }
+struct Tickets {
+  int* counter;
+  int next;
+  __device__ void prime(int* c) {
+    counter = c;
+    next = (threadIdx.x & 63) == 0 ? atomicAdd(counter, 1) : 0;
+  }
+  __device__ int take() {
+    const int t = __builtin_amdgcn_readfirstlane(next);
+    next = (threadIdx.x & 63) == 0 ? atomicAdd(counter, 1) : 0;
+    return t;
+  }
+};
+
+// Positions of the transposed entries and the diagonal; F_UNSYM if an entry
+// off the diagonal has no transpose.
+__global__ void k_tpos_adiag(DevCsr A, uint32_t* tpos, double* adiag, int* flags) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (i >= A.n) return;
   uint32_t b, e;
   row_range(A, i, b, e);
   double d = 0.0;
+  bool whole = true;
   for (uint32_t q = b; q < e; ++q) {
     const uint32_t c = A.col[q];
     uint32_t t = kNone;
-    if (c == (uint32_t)i) d = A.val[q];
-    if (c < (uint32_t)i) {
+    if (c == (uint32_t)i) {
+      d = A.val[q];
+    } else {
       uint32_t kb, ke;
       row_range(A, c, kb, ke);
       for (uint32_t r = kb; r < ke; ++r)
@@ -64,32 +131,55 @@ __global__ void k_tpos_adiag(DevCsr A, uint32_t* tpos, double* adiag) {
           t = r;
           break;
         }
+      whole = whole && t != kNone;
+      if (c > (uint32_t)i) t = kNone;
     }
     tpos[q] = t;
   }
   adiag[i] = d;
+  if (!whole) atomicOr(flags + 3, F_UNSYM);
 }
 
-__global__ void k_level_relax(DevCsr A, int32_t* level, int* changed) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= A.n) return;
-  uint32_t b, e;
-  row_range(A, i, b, e);
-  int32_t lv = 0;
-  for (uint32_t q = b; q < e; ++q) {
-    const uint32_t c = A.col[q];
-    if (c < (uint32_t)i) lv = max(lv, level[c] + 1);
+// Every row's level, one more than the largest of the rows it reads (the
+// lower neighbours, which have smaller indices), and the largest of all.
+// Waves take 64 consecutive rows by ticket in row order; rows of one wave may
+// read each other, so a wave goes round until all its rows have theirs.
+// level is filled with -1.
+__global__ __launch_bounds__(256) void k_levels(DevCsr A, int32_t* level, int* flags) {
+  const int lane = threadIdx.x & 63;
+  const int64_t nw = (A.n + 63) / 64;
+  Tickets T;
+  T.prime(flags);
+  bool quit = false;
+  for (int t = T.take(); t < nw && !quit; t = T.take()) {
+    const int64_t i = (int64_t)t * 64 + lane;
+    uint32_t q = 0, e = 0;
+    if (i < A.n) row_range(A, i, q, e);
+    int32_t lv = 0;
+    bool done = i >= A.n;
+    int spins = 0;
+    while (__any(!done) && !quit) {
+      if (!done) {
+        while (q < e && A.col[q] < (uint32_t)i) {
+          const int32_t L = __hip_atomic_load(level + A.col[q], __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT);
+          if (L < 0) break;
+          lv = max(lv, L + 1);
+          ++q;
+        }
+        if (!(q < e && A.col[q] < (uint32_t)i)) {
+          __hip_atomic_store(level + i, lv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          done = true;
+        }
+      }
+      if ((spins & 63) == 63) quit = __any(give_up(spins, flags));
+      ++spins;
+      whole();
+    }
+    for (int o = 32; o > 0; o >>= 1) lv = max(lv, __shfl_xor(lv, o, 64));
+    if (lane == 0) atomicMax(flags + 2, lv);
+    whole();
   }
-  if (lv != level[i]) {
-    level[i] = lv;
-    *changed = 1;
-  }
-}
-
-__global__ void k_level_max(const int32_t* level, int64_t n, int* out) {
-  const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  atomicMax(out, level[i]);
 }
 
 __global__ void k_level_count(const int32_t* level, int64_t n, int32_t base,
@@ -107,23 +197,54 @@ __global__ void k_level_scatter(const int32_t* level, int64_t n, int32_t base,
   list[pos] = (uint32_t)i;
 }
 
-// factor_modified_incomplete_cholesky0 (PCGSolver.h:97-205), one level.
+// The same with the levels (at most kLdsLevels) counted per block in LDS, so
+// a block adds to each level's counter once (110,000 rows over 151 levels:
+// one atomic per row took 136 us for either pass).  With list the block takes
+// its places in each level and writes its rows, else it only counts.
+constexpr int kLdsLevels = 4096, kLevelRows = 16;  // rows per thread
+__global__ __launch_bounds__(256) void k_level_sort(const int32_t* level, int64_t n, int span,
+                                                    uint32_t* count, uint32_t* list) {
+  __shared__ uint32_t have[kLdsLevels];
+  for (int l = threadIdx.x; l < span; l += 256) have[l] = 0;
+  __syncthreads();
+  const int64_t i0 = blockIdx.x * (int64_t)(256 * kLevelRows) + threadIdx.x;
+  uint32_t rank[kLevelRows];
+#pragma unroll
+  for (int k = 0; k < kLevelRows; ++k) {
+    const int64_t i = i0 + 256 * k;
+    rank[k] = i < n ? atomicAdd(&have[level[i]], 1u) : 0u;
+  }
+  __syncthreads();
+  for (int l = threadIdx.x; l < span; l += 256)
+    if (have[l]) {
+      const uint32_t base = atomicAdd(&count[l], have[l]);
+      have[l] = base;
+    }
+  if (!list) return;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kLevelRows; ++k) {
+    const int64_t i = i0 + 256 * k;
+    if (i < n) list[have[level[i]] + rank[k]] = (uint32_t)i;
+  }
+}
+
+// factor_modified_incomplete_cholesky0 (PCGSolver.h:97-205), one row.
 // Column j collects, in ascending k, every update the right-looking loop of
 // column k applies to it: the diagonal -= L_jk*L_jk, the fill-in matches
-// L_rj -= L_jk*L_rk, and the diagonal -= tau*L_jk*missing.
-__global__ void k_mic0_level(DevCsr A, const uint32_t* tpos,
-                             const double* adiag, const uint32_t* list,
-                             uint32_t count, double tau, double mdr,
-                             double* invdiag, double* lv, int* overflow) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= count) return;
-  const int64_t j = list[t];
+// L_rj -= L_jk*L_rk, and the diagonal -= tau*L_jk*missing.  get(e) is the
+// finished factor entry e (of an earlier row), put(e, v) stores one.
+template <class Get, class Put>
+__device__ inline void mic0_row(const DevCsr& A, int64_t j, const uint32_t* tpos,
+                                const double* adiag, double tau, double mdr, double* invdiag,
+                                int* overflow, Get get, Put put) {
   uint32_t jb, je;
   row_range(A, j, jb, je);
   const uint32_t ju = upper_begin(A, j, jb, je);
   const int nu = (int)(je - ju);
   if (nu > kMaxUpper) {
     *overflow = 1;
+    for (uint32_t q = ju; q < je; ++q) put(q, 0.0);  // (nothing may wait for them)
     return;
   }
   double lvj[kMaxUpper];
@@ -139,7 +260,7 @@ __global__ void k_mic0_level(DevCsr A, const uint32_t* tpos,
     uint32_t kb, ke;
     row_range(A, k, kb, ke);
     const uint32_t c0 = upper_begin(A, k, kb, ke);
-    const double multiplier = lv[pk];
+    const double multiplier = get(pk);
     double missing = 0;
     uint32_t a = c0;
     uint32_t bb = jb;
@@ -150,36 +271,36 @@ __global__ void k_mic0_level(DevCsr A, const uint32_t* tpos,
         else if (A.col[bb] == A.col[a])
           break;
         else {
-          missing += lv[a];
+          missing += get(a);
           break;
         }
       }
       ++a;
     }
-    if (a < ke && A.col[a] == (uint32_t)j) d -= multiplier * lv[a];
+    if (a < ke && A.col[a] == (uint32_t)j) d -= multiplier * get(a);
     ++a;
     int ub = 0;
     while (a < ke && ub < nu) {
       if (A.col[ju + ub] < A.col[a])
         ++ub;
       else if (A.col[ju + ub] == A.col[a]) {
-        lvj[ub] -= multiplier * lv[a];
+        lvj[ub] -= multiplier * get(a);
         ++a;
         ++ub;
       } else {
-        missing += lv[a];
+        missing += get(a);
         ++a;
       }
     }
     while (a < ke) {
-      missing += lv[a];
+      missing += get(a);
       ++a;
     }
     d -= tau * multiplier * missing;
   }
   if (aj == 0) {
     invdiag[j] = d;
-    for (int u = 0; u < nu; ++u) lv[ju + u] = lvj[u];
+    for (int u = 0; u < nu; ++u) put(ju + u, lvj[u]);
     return;
   }
   double inv;
@@ -188,7 +309,43 @@ __global__ void k_mic0_level(DevCsr A, const uint32_t* tpos,
   else
     inv = 1 / sqrt(d);
   invdiag[j] = inv;
-  for (int u = 0; u < nu; ++u) lv[ju + u] = lvj[u] * inv;
+  for (int u = 0; u < nu; ++u) put(ju + u, lvj[u] * inv);
+}
+
+__global__ void k_mic0_level(DevCsr A, const uint32_t* tpos,
+                             const double* adiag, const uint32_t* list,
+                             uint32_t count, double tau, double mdr,
+                             double* invdiag, double* lv, int* overflow) {
+  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= count) return;
+  mic0_row(A, list[t], tpos, adiag, tau, mdr, invdiag, overflow,
+           [&](uint32_t e) { return lv[e]; }, [&](uint32_t e, double v) { lv[e] = v; });
+}
+
+// The rows of a level schedule: wave w holds rows list[start[w]] to the next
+// wave's start (or n), all of one level.
+struct Schedule {
+  const uint32_t *start, *list;
+  int nwaves;
+  uint32_t n;
+  int* flags;
+};
+
+// All levels in one launch; lv holds the sentinel above the diagonal.
+__global__ __launch_bounds__(64) void k_mic0_pass(DevCsr A, Schedule P, const uint32_t* tpos,
+                                                  const double* adiag, double tau, double mdr,
+                                                  double* invdiag, double* lv) {
+  const int lane = threadIdx.x & 63;
+  Tickets T;
+  T.prime(P.flags);
+  for (int t = T.take(); t < P.nwaves; t = T.take()) {
+    const uint32_t at = P.start[t] + lane;
+    if (at < (t + 1 < P.nwaves ? P.start[t + 1] : P.n))
+      mic0_row(A, P.list[at], tpos, adiag, tau, mdr, invdiag, P.flags + 2,
+               [&](uint32_t e) { return settle(load_agent(lv + e), lv + e, P.flags); },
+               [&](uint32_t e, double v) { store_agent(lv + e, v); });
+    whole();
+  }
 }
 
 // solve_lower (PCGSolver.h:211-223) for one level: z_j = (r_j - sum over
@@ -226,6 +383,71 @@ __global__ void k_upper_level(DevCsr A, const double* invdiag,
   for (uint32_t q = upper_begin(A, j, jb, je); q < je; ++q)
     acc -= lv[q] * z[A.col[q]];
   z[j] = acc * invdiag[j];
+}
+
+// Either solve in one launch: LOWER y = (r - L y) * invdiag over the levels
+// ascending, else z = (y - L^T z) * invdiag descending, the terms in
+// ascending column order as above.  out holds the sentinel, and the pass
+// resets the other one's output (each row's own entry, which no other row
+// reads any more or yet) and ticket counter.  What bounds it is the chain of
+// levels: a row's coefficients are read before it waits, so a level costs
+// a store-to-load round trip between two compute units and the polls it
+// takes to see it, about 1.2 us (a launch per level: 2.5-5 us).  Whole solves,
+// ms: 1334 rows 7.4 -> 2.6, 112,828 rows (151 levels) 102 -> 26, 755,018 rows
+// 359 -> 107.  Reading the missing values one after another took 37 ms where
+// reading them together takes 26.
+constexpr int kAhead = 4;  // entries a row holds in registers at a time
+template <bool LOWER>
+__global__ __launch_bounds__(64) void k_solve_pass(DevCsr A, Schedule P, const uint32_t* tpos,
+                                                   const double* invdiag, const double* lv,
+                                                   const double* in, double* out,
+                                                   double* reset) {
+  const int lane = threadIdx.x & 63;
+  auto row = [&](uint32_t j) {
+    uint32_t q, e;
+    row_range(A, j, q, e);
+    if (!LOWER) q = upper_begin(A, j, q, e);
+    double acc = in[j];
+    const double inv = invdiag[j];
+    for (bool more = true; more && q < e; q += kAhead) {
+      double l[kAhead], v[kAhead];
+      uint32_t c[kAhead];
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) {
+        c[s] = q + s < e ? A.col[q + s] : kNone;
+        if (LOWER && c[s] >= j) c[s] = kNone;
+        l[s] = c[s] != kNone ? lv[LOWER ? tpos[q + s] : q + s] : 0.0;
+      }
+      // the values not yet set are read again together, one round trip for all
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) v[s] = c[s] != kNone ? load_agent(out + c[s]) : 0.0;
+      for (int spins = 0;; ++spins) {
+        bool wait = false;
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s) wait = wait || unset(v[s]);
+        if (!wait) break;
+        const bool stop = (spins & 63) == 63 && give_up(spins, P.flags);
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s)
+          if (unset(v[s])) v[s] = stop ? 0.0 : load_agent(out + c[s]);
+      }
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s)
+        if (c[s] != kNone) acc -= l[s] * v[s];
+      more = c[kAhead - 1] != kNone;
+    }
+    store_agent(out + j, acc * inv);
+    reset[j] = __longlong_as_double((long long)kUnset);
+  };
+  Tickets T;
+  T.prime(P.flags + (LOWER ? 0 : 1));
+  for (int t = T.take(); t < P.nwaves; t = T.take()) {
+    if (t == 0 && lane == 0) P.flags[LOWER ? 1 : 0] = 0;
+    const int w = LOWER ? t : P.nwaves - 1 - t;
+    const uint32_t at = P.start[w] + lane;
+    if (at < (w + 1 < P.nwaves ? P.start[w + 1] : P.n)) row(P.list[at]);
+    whole();
+  }
 }
 
 // multiply(FixedSparseMatrix) (SparseMatrix.h:298-322)
@@ -271,6 +493,30 @@ __global__ __launch_bounds__(kRedThreads) void k_dot_partial(
     acc += (double)a[i] * (double)b[i];
   const double s = block_sum(acc, sh);
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+// y = A x and the block partials of x . y
+__global__ __launch_bounds__(kRedThreads) void k_spmv_dot(DevCsr A, const double* x, double* y,
+                                                          double* partial) {
+  __shared__ double sh[kRedThreads];
+  double dot = 0;
+  for (int64_t i = blockIdx.x * (int64_t)kRedThreads + threadIdx.x; i < A.n;
+       i += (int64_t)gridDim.x * kRedThreads) {
+    uint32_t b, e;
+    row_range(A, i, b, e);
+    double acc = 0;
+    for (uint32_t q = b; q < e; ++q) acc += A.val[q] * x[A.col[q]];
+    y[i] = acc;
+    dot += x[i] * acc;
+  }
+  const double s = block_sum(dot, sh);
+  if (threadIdx.x == 0) partial[blockIdx.x] = s;
+}
+
+__global__ void k_fill_unset(double* p, int64_t n) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = __longlong_as_double((long long)kUnset);
 }
 
 // modes of the final reduction
@@ -562,6 +808,12 @@ void PcgWork::release() {
   host_part_dev = nullptr;
 }
 
+// Levels whose waves a waiting pass keeps resident: enough to hide the reads
+// a row makes before it waits, few enough that the waiting waves' polls do not
+// slow the stores (112,828 rows: 28.7 ms with 4, 26.1 with 8 and 16, 27.9 with
+// 32; 755,018 rows: 117 / 107 / 119 / 167).
+constexpr int64_t kPassLevels = 8;
+
 static size_t slot_count(const DevCsr& A) { return (size_t)A.nnz_slots; }
 
 void pcg_prepare(hipStream_t st, PcgWork& w, const DevCsr& A,
@@ -612,56 +864,61 @@ void pcg_prepare_vectors(hipStream_t st, PcgWork& w, int64_t n) {
   w.nlevels = 0;
 }
 
+static void fill_unset(hipStream_t st, double* p, int64_t n) {
+  hipLaunchKernelGGL(k_fill_unset, dim3(std::min(blocks_for(n, 256), 4096u)), dim3(256), 0, st, p, n);
+  WC_LAUNCH_CHECK();
+}
+
+// a waiting pass that ran out of its bound
+constexpr const char* kPassAbort = "level-scheduled pass: a row's wait exceeded its bound";
+static void throw_if_aborted(int flags3) {
+  if (flags3 & F_ABORT) throw HipError{hipErrorLaunchTimeOut, kPassAbort, __FILE__, __LINE__};
+}
+
 // The level schedule of the level-scheduled kernels (built on first use, so
 // systems solved with the pipelined sweeps never pay for it).
 static void pcg_levels(hipStream_t st, PcgWork& w, const DevCsr& A) {
   if (w.levels_ready) return;
   w.levels_ready = true;
+  w.nwaves = 0;
+  w.lower_ready = false;
   const int64_t n = A.n;
   if (n == 0) {
     w.nlevels = 0;
     return;
   }
+  WC_HIP(hipMemsetAsync(w.flags.p, 0, sizeof(int) * 4, st));
   hipLaunchKernelGGL(k_tpos_adiag, dim3(blocks_for(n, 256)), dim3(256), 0, st, A,
-                     w.tpos.p, w.adiag.p);
+                     w.tpos.p, w.adiag.p, w.flags.p);
   WC_LAUNCH_CHECK();
 
   const int32_t* lev = w.level_in;
   int32_t span = w.level_span;
+  int hf[4] = {0, 0, 0, 0};
   if (!lev) {
     w.level.ensure(n);
-    WC_HIP(hipMemsetAsync(w.level.p, 0, sizeof(int32_t) * n, st));
-    int* changed = w.flags.p;
-    int hchanged = 1;
-    int64_t iters = 0;
-    while (hchanged) {
-      WC_HIP(hipMemsetAsync(changed, 0, sizeof(int), st));
-      hipLaunchKernelGGL(k_level_relax, dim3(blocks_for(n, 256)), dim3(256), 0,
-                         st, A, w.level.p, changed);
-      WC_LAUNCH_CHECK();
-      WC_HIP(hipMemcpyAsync(&hchanged, changed, sizeof(int),
-                            hipMemcpyDeviceToHost, st));
-      WC_HIP(hipStreamSynchronize(st));
-      if (++iters > n + 1) break;
-    }
-    // relaxation in place can converge in fewer passes than the depth
-    WC_HIP(hipMemsetAsync(w.flags.p + 2, 0, sizeof(int), st));
-    hipLaunchKernelGGL(k_level_max, dim3(blocks_for(n, 256)), dim3(256), 0, st,
-                       w.level.p, n, w.flags.p + 2);
+    WC_HIP(hipMemsetAsync(w.level.p, 0xFF, sizeof(int32_t) * n, st));
+    const int64_t nw = (n + 63) / 64;
+    hipLaunchKernelGGL(k_levels, dim3((unsigned)std::min<int64_t>((nw + 3) / 4, 512)), dim3(256),
+                       0, st, A, w.level.p, w.flags.p);
     WC_LAUNCH_CHECK();
-    int hmax = 0;
-    WC_HIP(hipMemcpyAsync(&hmax, w.flags.p + 2, sizeof(int),
-                          hipMemcpyDeviceToHost, st));
-    WC_HIP(hipStreamSynchronize(st));
-    span = hmax + 1;
     lev = w.level.p;
   }
+  WC_HIP(hipMemcpyAsync(hf, w.flags.p, sizeof(hf), hipMemcpyDeviceToHost, st));
+  WC_HIP(hipStreamSynchronize(st));
+  throw_if_aborted(hf[3]);
+  if (!w.level_in) span = hf[2] + 1;
   w.lvl_count.ensure(span);
-  w.lvl_cursor.ensure(span);
   w.lvl_list.ensure(n);
   WC_HIP(hipMemsetAsync(w.lvl_count.p, 0, sizeof(uint32_t) * span, st));
-  hipLaunchKernelGGL(k_level_count, dim3(blocks_for(n, 256)), dim3(256), 0, st,
-                     lev, n, 0, w.lvl_count.p);
+  const bool lds = span <= kLdsLevels;
+  const unsigned sort_blocks = blocks_for(n, 256 * kLevelRows);
+  if (lds)
+    hipLaunchKernelGGL(k_level_sort, dim3(sort_blocks), dim3(256), 0, st, lev, n, (int)span,
+                       w.lvl_count.p, nullptr);
+  else
+    hipLaunchKernelGGL(k_level_count, dim3(blocks_for(n, 256)), dim3(256), 0, st,
+                       lev, n, 0, w.lvl_count.p);
   WC_LAUNCH_CHECK();
   std::vector<uint32_t> cnt(span);
   WC_HIP(hipMemcpyAsync(cnt.data(), w.lvl_count.p, sizeof(uint32_t) * span,
@@ -669,48 +926,92 @@ static void pcg_levels(hipStream_t st, PcgWork& w, const DevCsr& A) {
   WC_HIP(hipStreamSynchronize(st));
   w.lvl_start.clear();
   w.lvl_size.clear();
-  std::vector<uint32_t> start(span);
+  std::vector<uint32_t> start(span), waves;
   uint32_t acc = 0;
   for (int32_t l = 0; l < span; ++l) {
     start[l] = acc;
     if (cnt[l]) {
       w.lvl_start.push_back(acc);
       w.lvl_size.push_back(cnt[l]);
+      for (uint32_t k = 0; k < cnt[l]; k += 64) waves.push_back(acc + k);
     }
     acc += cnt[l];
   }
   w.nlevels = (int)w.lvl_size.size();
+  w.lvl_cursor.ensure(std::max<size_t>((size_t)span, waves.size()));
   WC_HIP(hipMemcpyAsync(w.lvl_cursor.p, start.data(), sizeof(uint32_t) * span,
                         hipMemcpyHostToDevice, st));
-  hipLaunchKernelGGL(k_level_scatter, dim3(blocks_for(n, 256)), dim3(256), 0,
-                     st, lev, n, 0, w.lvl_cursor.p, w.lvl_list.p);
+  if (lds)
+    hipLaunchKernelGGL(k_level_sort, dim3(sort_blocks), dim3(256), 0, st, lev, n, (int)span,
+                       w.lvl_cursor.p, w.lvl_list.p);
+  else
+    hipLaunchKernelGGL(k_level_scatter, dim3(blocks_for(n, 256)), dim3(256), 0,
+                       st, lev, n, 0, w.lvl_cursor.p, w.lvl_list.p);
   WC_LAUNCH_CHECK();
-  // the host vector 'start' must outlive the async copy
+  if (!(hf[3] & F_UNSYM)) {
+    // the cursors have done their work: the wave starts take their place
+    WC_HIP(hipMemcpyAsync(w.lvl_cursor.p, waves.data(), sizeof(uint32_t) * waves.size(),
+                          hipMemcpyHostToDevice, st));
+    w.nwaves = (int64_t)waves.size();
+    // a few levels' waves are resident, which hides the latency of the rows'
+    // coefficients; more would only poll
+    const int64_t per_level = (w.nwaves + w.nlevels - 1) / w.nlevels;
+    w.pass_waves = (int)std::min<int64_t>(w.nwaves, std::min<int64_t>(2048, std::max<int64_t>(64, kPassLevels * per_level)));
+    WC_HIP(hipMemsetAsync(w.flags.p, 0, sizeof(int) * 4, st));  // the passes' tickets
+  }
+  // the host vectors must outlive the async copies
   WC_HIP(hipStreamSynchronize(st));
+}
+
+static Schedule schedule_of(const PcgWork& w, const DevCsr& A) {
+  return Schedule{w.lvl_cursor.p, w.lvl_list.p, (int)w.nwaves, (uint32_t)A.n, w.flags.p};
 }
 
 void pcg_factor(hipStream_t st, PcgWork& w, const DevCsr& A, double tau,
                 double mdr) {
   if (A.n == 0) return;
+  if (w.lower_ready) w.levels_ready = false;  // an apply has overwritten the diagonal
   pcg_levels(st, w, A);
-  int* overflow = w.flags.p + 1;
-  WC_HIP(hipMemsetAsync(overflow, 0, sizeof(int), st));
-  for (int l = 0; l < w.nlevels; ++l) {
+  WC_HIP(hipMemsetAsync(w.flags.p, 0, sizeof(int) * 4, st));
+  if (w.nwaves > 0) {
+    fill_unset(st, w.lv.p, A.nnz_slots);
+    hipLaunchKernelGGL(k_mic0_pass, dim3(w.pass_waves), dim3(64), 0, st, A, schedule_of(w, A),
+                       w.tpos.p, w.adiag.p, tau, mdr, w.invdiag.p, w.lv.p);
+    WC_LAUNCH_CHECK();
+  }
+  for (int l = 0; w.nwaves == 0 && l < w.nlevels; ++l) {
     const uint32_t cnt = w.lvl_size[l];
     hipLaunchKernelGGL(k_mic0_level, dim3(blocks_for(cnt, 64)), dim3(64), 0, st,
                        A, w.tpos.p, w.adiag.p, w.lvl_list.p + w.lvl_start[l], cnt,
-                       tau, mdr, w.invdiag.p, w.lv.p, overflow);
+                       tau, mdr, w.invdiag.p, w.lv.p, w.flags.p + 2);
     WC_LAUNCH_CHECK();
   }
-  int hov = 0;
-  WC_HIP(hipMemcpyAsync(&hov, overflow, sizeof(int), hipMemcpyDeviceToHost, st));
+  int hf[4] = {0, 0, 0, 0};
+  WC_HIP(hipMemcpyAsync(hf, w.flags.p, sizeof(hf), hipMemcpyDeviceToHost, st));
   WC_HIP(hipStreamSynchronize(st));
-  if (hov) throw HipError{hipErrorInvalidValue, "MIC(0): a row has more than 16 entries above the diagonal", __FILE__, __LINE__};
+  throw_if_aborted(hf[3]);
+  if (hf[2]) throw HipError{hipErrorInvalidValue, "MIC(0): a row has more than 16 entries above the diagonal", __FILE__, __LINE__};
+  WC_HIP(hipMemsetAsync(w.flags.p, 0, sizeof(int) * 4, st));  // the solves' tickets
 }
 
+// z = the preconditioned r.  The waiting passes keep the lower solve's result
+// in w.adiag, which only the factor needs, as the sentinel between applies,
+// and set z to it on the way.
 void pcg_apply(hipStream_t st, PcgWork& w, const DevCsr& A, const double* r,
                double* z) {
   pcg_levels(st, w, A);
+  if (w.nwaves > 0) {
+    const Schedule P = schedule_of(w, A);
+    double* y = w.adiag.p;
+    if (!w.lower_ready) fill_unset(st, y, A.n);
+    w.lower_ready = true;
+    hipLaunchKernelGGL((k_solve_pass<true>), dim3(w.pass_waves), dim3(64), 0, st, A, P, w.tpos.p,
+                       w.invdiag.p, w.lv.p, r, y, z);
+    hipLaunchKernelGGL((k_solve_pass<false>), dim3(w.pass_waves), dim3(64), 0, st, A, P, w.tpos.p,
+                       w.invdiag.p, w.lv.p, y, z, y);
+    WC_LAUNCH_CHECK();
+    return;
+  }
   for (int l = 0; l < w.nlevels; ++l) {
     const uint32_t cnt = w.lvl_size[l];
     hipLaunchKernelGGL(k_lower_level, dim3(blocks_for(cnt, 64)), dim3(64), 0, st,
@@ -725,6 +1026,14 @@ void pcg_apply(hipStream_t st, PcgWork& w, const DevCsr& A, const double* r,
                        cnt, z);
     WC_LAUNCH_CHECK();
   }
+}
+
+void pcg_check(hipStream_t st, PcgWork& w) {
+  if (w.nwaves == 0) return;
+  int f = 0;
+  WC_HIP(hipMemcpyAsync(&f, w.flags.p + 3, sizeof(f), hipMemcpyDeviceToHost, st));
+  WC_HIP(hipStreamSynchronize(st));
+  throw_if_aborted(f);
 }
 
 void pcg_spmv(hipStream_t st, const DevCsr& A, const double* x, double* y) {
@@ -765,7 +1074,9 @@ static void clear_residual(PcgWork& w) {
   for (int i = 0; i < w.red_blocks; ++i) w.host_part[i] = -1.0;
 }
 
-static double box_residual_max(hipStream_t st, PcgWork& w) {
+static double box_residual_max(hipStream_t st, PcgWork& w,
+                               const char* abort_text = "pipelined MIC(0) sweep: a tile wait "
+                                                        "exceeded its bound") {
   volatile const double* hp = w.host_part;
   const int nb = w.red_blocks;
   int i = 0;
@@ -788,9 +1099,7 @@ static double box_residual_max(hipStream_t st, PcgWork& w) {
   }
   __atomic_thread_fence(__ATOMIC_ACQUIRE);
   if (hp[0] == -2.0)
-    throw HipError{hipErrorLaunchTimeOut,
-                   "pipelined MIC(0) sweep: a tile wait exceeded its bound", __FILE__,
-                   __LINE__};
+    throw HipError{hipErrorLaunchTimeOut, abort_text, __FILE__, __LINE__};
   double m = 0;
   for (int k = 0; k < nb; ++k) m = fmax(m, hp[k]);
   clear_residual(w);  // for the next update, which the host enqueues after this
@@ -1027,12 +1336,48 @@ bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,
     return false;
   }
   WC_HIP(hipMemcpyAsync(s, z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+  if (w.host_part) {
+    // As in pcg_loop_box: the update takes alpha from the partials and leaves
+    // the |r|_inf partials in mapped memory, and the next apply is enqueued
+    // before the host has read them.
+    clear_residual(w);
+    int rho_slot = S_RHO, it;
+    bool ok = false;
+    for (it = 0; it < maxit; ++it) {
+      hipEvent_t e0 = w.timer.on ? w.timer.mark(st) : nullptr;
+      hipLaunchKernelGGL(k_spmv_dot, dim3(nb), dim3(kRedThreads), 0, st, A, s, z, w.partial.p);
+      if (e0) w.timer.add(KTimer::SPMV, n, e0, w.timer.mark(st));
+      hipLaunchKernelGGL(k_update_xr_fused<double>, dim3(nb), dim3(kRedThreads), 0, st, x, r, s,
+                         z, n, w.partial.p, nb, w.scal.p, rho_slot, w.host_part_dev,
+                         w.flags.p + 3, nullptr);
+      WC_LAUNCH_CHECK();
+      if (it + 1 < maxit) {
+        pcg_apply(st, w, A, r, z);
+        hipLaunchKernelGGL(k_dot_partial<double>, dim3(nb), dim3(kRedThreads), 0, st, z, r, n,
+                           w.partial.p);
+        const int rho_next = rho_slot == S_RHO ? S_RHO2 : S_RHO;
+        hipLaunchKernelGGL(k_update_s_fused<double>, dim3(nb), dim3(kRedThreads), 0, st, s, z, n,
+                           w.partial.p, nb, w.scal.p, rho_slot, rho_next, nullptr, nullptr);
+        WC_LAUNCH_CHECK();
+        rho_slot = rho_next;
+      }
+      res = box_residual_max(st, w, kPassAbort);
+      *residual_out = res;
+      if (res <= tolr) {
+        ++it;
+        ok = true;
+        break;
+      }
+    }
+    *iters_out = it;
+    settle_timer(st, w);
+    return ok;
+  }
   const unsigned gb = blocks_for(n, 256);
   int it;
-  for (it = 0; it < maxit; ++it) {
-    hipEvent_t e0 = w.timer.on ? w.timer.mark(st) : nullptr;
+  bool ok = false;
+  for (it = 0; it < maxit && !ok; ++it) {
     hipLaunchKernelGGL(k_spmv, dim3(gb), dim3(256), 0, st, A, s, z);
-    if (e0) w.timer.add(KTimer::SPMV, n, e0, w.timer.mark(st));
     hipLaunchKernelGGL(k_dot_partial<double>, dim3(nb), dim3(kRedThreads), 0, st, s, z,
                        n, w.partial.p);
     hipLaunchKernelGGL(k_dot_final, dim3(1), dim3(kRedThreads), 0, st,
@@ -1045,8 +1390,8 @@ bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,
     res = read_scal(st, w, S_RES);
     *residual_out = res;
     if (res <= tolr) {
-      *iters_out = it + 1;
-      return true;
+      ok = true;
+      continue;
     }
     pcg_apply(st, w, A, r, z);
     hipLaunchKernelGGL(k_dot_partial<double>, dim3(nb), dim3(kRedThreads), 0, st, z, r,
@@ -1058,7 +1403,8 @@ bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,
     WC_LAUNCH_CHECK();
   }
   *iters_out = it;
-  return false;
+  pcg_check(st, w);
+  return ok;
 }
 
 // AMGPCGSolveSparse (AlgebraicMultigrid.h:247-359): x = 0, r = b; the

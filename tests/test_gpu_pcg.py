@@ -100,3 +100,88 @@ def test_csr_validation_rejects_unsorted(wc):
     col = np.array([1, 0, 1], np.uint32)  # row 0 unsorted
     with pytest.raises(wc.WetclothError):
         wc.spmv_csr(rs, col, np.ones(3), np.ones(2))
+
+
+def tridiagonal(n, seed):
+    """A chain: every row is a level of its own."""
+    rng = np.random.default_rng(seed)
+    import scipy.sparse as sp
+    w = rng.uniform(0.1, 1.0, n - 1)
+    d = np.full(n, 0.05)
+    d[:-1] += w
+    d[1:] += w
+    return csr_parts(sp.diags([-w, d, -w], [-1, 0, 1]))
+
+
+def wide_rows(n, k, seed):
+    """Random symmetric M-matrix, about 2 k entries off the diagonal per row
+    (more than a row holds in registers at a time), at most 16 above it."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    rows = np.repeat(np.arange(n), k)
+    cols = rows + rng.integers(1, 40, n * k)
+    m = cols < n
+    W = sp.coo_matrix((-rng.uniform(0.1, 1.0, m.sum()), (rows[m], cols[m])), shape=(n, n)).tocsr()
+    W = W + W.T
+    return csr_parts(W + sp.diags(-np.asarray(W.sum(axis=1)).ravel() + 0.1))
+
+
+@pytest.mark.parametrize("kind,n", [
+    ("chain", 2), ("chain", 64), ("chain", 65), ("chain", 300),
+    ("chain", 4097),             # more levels than a block counts in LDS
+    ("diagonal", 1), ("diagonal", 63), ("diagonal", 1000),   # one level, its last wave partial
+    ("wide", 400),
+])
+def test_level_passes_bitwise(oracle, wc, kind, n):
+    """The factor and the apply run all levels in one launch, waiting for the
+    values they read: bit for bit the sequential form's, whatever the depth
+    and width of the levels."""
+    if kind == "chain":
+        rs, col, val = tridiagonal(n, n)
+    elif kind == "diagonal":
+        rs, col = np.arange(n + 1, dtype=np.uint32), np.arange(n, dtype=np.uint32)
+        val = np.random.default_rng(n).uniform(0.5, 2.0, n)
+    else:
+        rs, col, val = wide_rows(n, 6, n)
+    inv_gpu, lv_gpu = wc.mic0_factor_csr(rs, col, val)
+    inv, lv = oracle.mic0(rs, col, val)
+    upper = col > np.repeat(np.arange(n), np.diff(rs.astype(np.int64)))
+    assert np.array_equal(inv_gpu, inv) and np.array_equal(lv_gpu[upper], lv[upper])
+    r = np.random.default_rng(n + 1).standard_normal(n)
+    assert np.array_equal(wc.mic0_apply_csr(rs, col, inv, lv, r),
+                          oracle.apply_precond(rs, col, inv, lv, r))
+    # (solutions of two solves to a 1e-10 residual; kappa is below 1e4 here)
+    for no_alloc in (False, True):
+        ok, x, it, res = wc.pcg_solve_csr(rs, col, val, r, tol=1e-10, maxit=5000,
+                                          no_alloc=no_alloc)
+        ok_c, x_c, it_c, _ = oracle.pcg(rs, col, val, r, tol=1e-10, maxit=5000)
+        assert ok and ok_c and abs(it - it_c) <= 1
+        assert np.abs(x - x_c).max() <= 1e-6 * np.abs(x_c).max()
+
+
+def test_factor_row_too_wide(wc):
+    """A row with 17 entries above its diagonal is refused (and nothing waits
+    for the entries it has not written)."""
+    n = 40
+    A = np.eye(n) * 40.0
+    A[0, 1:18] = A[1:18, 0] = -1.0
+    A[np.arange(1, n), np.arange(n - 1)] = A[np.arange(n - 1), np.arange(1, n)] = -1.0
+    with pytest.raises(wc.WetclothError, match="16 entries"):
+        wc.mic0_factor_csr(*csr_parts(A))
+
+
+def test_apply_pattern_not_symmetric(wc):
+    """An entry without its transpose: such a matrix is run level by level, a
+    row subtracting the entries of its own row that have a transpose (lower)
+    and all above the diagonal (upper)."""
+    rs = np.array([0, 3, 6, 8], np.uint32)
+    col = np.array([0, 1, 2, 0, 1, 2, 1, 2], np.uint32)  # (2, 0) is missing
+    lv = np.array([0, -0.5, -0.25, 0, 0, -0.75, 0, 0])
+    inv, r = np.array([0.9, 0.8, 0.7]), np.array([1.0, 2.0, 3.0])
+    y0 = r[0] * inv[0]
+    y1 = (r[1] - lv[1] * y0) * inv[1]
+    y2 = (r[2] - lv[5] * y1) * inv[2]
+    z2 = y2 * inv[2]
+    z1 = (y1 - lv[5] * z2) * inv[1]
+    z0 = ((y0 - lv[1] * z1) - lv[2] * z2) * inv[0]
+    assert np.array_equal(wc.mic0_apply_csr(rs, col, inv, lv, r), [z0, z1, z2])
