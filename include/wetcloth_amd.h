@@ -316,7 +316,8 @@ wc_status wc_phase_times(const wc_ctx* ctx, double ms[7]);
  *   consecutive skewed steps with its neighbours in LDS; 0 selects one row
  *   per thread.  Both give bitwise the same product; the PCG's s . A s is
  *   summed per run or per block, so whole solves agree to rounding.
- *   "spmv_run" (default 12, 1..4096): the steps of one run.
+ *   "spmv_run" (1..4096; 1 to 8 by the system's size until it is set): the
+ *   steps of one run.
  *   "debug_abort_sweeps" (default 0; a test hook): the pipelined sweeps'
  *   abort flag is set before each PCG loop, as a sweep whose bounded wait
  *   ran out sets it; the solve then fails with WC_ERR_HIP and a message

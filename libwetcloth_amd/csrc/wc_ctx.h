@@ -151,7 +151,7 @@ struct SweepPlan {
   // bit.  spart: the windowed product's x . y partials, one per block.
   bool debug_abort = false;  // test hook: the sweeps' abort flag set before each PCG loop
   bool spmv_win = true;
-  int spmv_run = 12;
+  int spmv_run = 0;  // 0: by size (spmv_run_of)
   DevBuf<double> spart;
   // its x faces as compact columns (ncell / 16 each): li = 15 and li = 0 of
   // the operand (written by the s update, else extracted), and li = 15 of

@@ -2189,17 +2189,30 @@ static unsigned spmv_blocks(const SweepPlan& P) {
   return (unsigned)std::min<int64_t>(1024, blocks(P.ncell, kSpmvThreads));
 }
 
+// The steps of one run of the windowed SpMV, where the option does not set
+// them: a block walks its run at about 1 us a step, so a small system takes
+// short runs, and a large one longer ones, which read the two steps around a
+// run less often.  us per launch (runs of 1 / 2 / 4 / 8 / 12): 16^3 FP64 6.5 /
+// 7.6 / 8.7 / 12.1 / 14.5, 64^3 FP64 9.5 / 8.9 / 10.3 / 13.4 / 16.6, 128^3
+// FP32 15.9 / 14.3 / 13.4 / 15.4 / 19.4, 256^3 FP32 69 / 54 / 47 / 45 / 48.
+static int spmv_run_of(const SweepPlan& P) {
+  if (P.spmv_run > 0) return P.spmv_run;
+  const int64_t steps = (int64_t)P.ntiles * P.nsteps;
+  return steps < 1024 ? 1 : steps < 2048 ? 2 : steps < 8192 ? 4 : 8;
+}
+
 // faces_ready: the columns of x are already in f15 / f0 (the s update
 // writes them); else they are extracted first
 template <class V, bool DOT>
 static DotParts spmv_win(hipStream_t st, SweepPlan& P, const V* coef, const V* c15, V* f15,
                          V* f0, const V* x, V* y, bool faces_ready) {
-  const int nrun = (P.nsteps + P.spmv_run - 1) / P.spmv_run;
+  const int run = spmv_run_of(P);
+  const int nrun = (P.nsteps + run - 1) / run;
   const int nb = P.ntiles * nrun;
   if (DOT) P.spart.ensure(nb);
   if (!faces_ready) face_cols<V>(st, P.ncell, x, f15, f0);
   hipLaunchKernelGGL((k_box_spmv_win<V, DOT>), dim3(nb), dim3(kThreads), 0, st,
-                     (uint32_t)P.ncell, skew_of(P), P.spmv_run, nrun, P.sflag.p, coef, x, f15,
+                     (uint32_t)P.ncell, skew_of(P), run, nrun, P.sflag.p, coef, x, f15,
                      f0, c15, y, DOT ? P.spart.p : nullptr);
   WC_LAUNCH_CHECK();
   return DotParts{P.spart.p, nb};
