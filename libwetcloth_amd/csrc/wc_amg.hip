@@ -248,8 +248,8 @@ __global__ void k_amg_redflag(int64_t n, const uint8_t* red, uint32_t* flag) {
 // row i to position p (red rows first); its entries to the planes.  scan
 // holds the exclusive scan of the red flags, and scan[n] their count.
 __global__ void k_amg_compact(DevCsr A, const uint8_t* red, const uint32_t* scan,
-                              uint32_t* crow, uint32_t* ccol, double* cval, uint8_t* clen,
-                              int* err) {
+                              uint32_t* crow, uint32_t* cpos, uint32_t* ccol, double* cval,
+                              double* cdiag, uint8_t* clen, int* err) {
   const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const int64_t n = A.n;
   if (i >= n) return;
@@ -262,25 +262,41 @@ __global__ void k_amg_compact(DevCsr A, const uint8_t* red, const uint32_t* scan
     return;
   }
   crow[p] = (uint32_t)i;
+  cpos[i] = (uint32_t)p;
   clen[p] = (uint8_t)(re - rb);
+  double diag = 0;  // as rbgs_row picks it
   for (uint32_t s = rb; s < re; ++s) {
-    ccol[(int64_t)(s - rb) * n + p] = A.col[s];
+    const uint32_t c = A.col[s];
+    ccol[(int64_t)(s - rb) * n + p] = c;
     cval[(int64_t)(s - rb) * n + p] = A.val[s];
+    if (c == (uint32_t)i || c >= (uint64_t)n) diag = A.val[s];
   }
+  cdiag[p] = diag;
 }
 
-// rbgs_row on a colour-ordered row: the same operations in the same order
+// rbgs_row on a colour-ordered row: the same operations in the same order;
+// at(c) is x[c].  Every entry of the row is loaded before the first is used.
+template <class X>
 __device__ inline double rbgs_crow(const uint32_t* ccol, const double* cval, int len, int64_t n,
-                                   int64_t p, uint32_t i, double bi, const double* x) {
-  double sum = 0, diag = 0;
-  for (int s = 0; s < len; ++s) {
-    const uint32_t c = ccol[(int64_t)s * n + p];
-    const double v = cval[(int64_t)s * n + p];
-    if (c != i && c < (uint64_t)n)
-      sum += v * x[c];
-    else
-      diag = v;
+                                   int64_t p, uint32_t i, double bi, X at) {
+  uint32_t c[kSlots];
+  double v[kSlots], xv[kSlots];
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) {
+    c[s] = s < len ? ccol[(int64_t)s * n + p] : i;
+    v[s] = s < len ? cval[(int64_t)s * n + p] : 0.0;
   }
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s) xv[s] = c[s] != i && c[s] < (uint64_t)n ? at(c[s]) : 0.0;
+  double sum = 0, diag = 0;
+#pragma unroll
+  for (int s = 0; s < kSlots; ++s)
+    if (s < len) {
+      if (c[s] != i && c[s] < (uint64_t)n)
+        sum += v[s] * xv[s];
+      else
+        diag = v[s];
+    }
   return diag != 0 ? (bi - sum) / diag : 0.0;
 }
 
@@ -291,20 +307,74 @@ __global__ void k_amg_rbgs_c(int64_t n, int64_t p0, int64_t p1, const uint32_t* 
   const int64_t p = p0 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (p >= p1) return;
   const uint32_t i = crow[p];
-  x[i] = rbgs_crow(ccol, cval, clen[p], n, p, i, b[i], x);
+  x[i] = rbgs_crow(ccol, cval, clen[p], n, p, i, b[i], [&](uint32_t c) { return x[c]; });
 }
 
-// r = b - A x on the colour-ordered rows (as k_amg_resid)
-__global__ void k_amg_resid_c(int64_t n, const uint32_t* crow, const uint32_t* ccol,
-                              const double* cval, const uint8_t* clen, const double* b,
-                              const double* x, double* r) {
+// The first red pass from x = 0, with the clear of x: a row's products are
+// then all +-0 and their sum +0, so no entry but the divisor is read.
+__global__ void k_amg_first_red(int64_t n, int64_t nred, const uint32_t* crow,
+                                const double* cdiag, const double* b, double* x) {
   const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   if (p >= n) return;
   const uint32_t i = crow[p];
-  const int len = clen[p];
-  double v = b[i];
-  for (int s = 0; s < len; ++s) v -= cval[(int64_t)s * n + p] * x[ccol[(int64_t)s * n + p]];
-  r[i] = v;
+  double v = 0.0;
+  if (p < nred) {
+    const double diag = cdiag[p];
+    v = diag != 0 ? (b[i] - 0.0) / diag : 0.0;
+  }
+  x[i] = v;
+}
+
+// The first red pass after the prolongation x += P x_c (AlgebraicMultigrid.h:
+// 106-116: xx = P x_c from 0, then x += 1 * xx), formed where the pass reads
+// it.  The smoother overwrites every row without reading its old value, red
+// rows now and black rows (which read red ones only) in the pass after this
+// one, so the prolonged x is never stored.
+__global__ void k_amg_prolong_red(int64_t n, int64_t nred, const uint32_t* crow,
+                                  const uint32_t* ccol, const double* cval, const uint8_t* clen,
+                                  const double* b, const uint32_t* parent, const double* xc,
+                                  double* x) {
+  const int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (p >= nred) return;
+  const uint32_t i = crow[p];
+  x[i] = rbgs_crow(ccol, cval, clen[p], n, p, i, b[i],
+                   [&](uint32_t c) { return x[c] + 1.0 * (0.0 + 1.0 * xc[parent[c]]); });
+}
+
+// b_c = R (b - A x) in one pass (as k_amg_resid, then k_amg_restrict): eight
+// lanes per coarse DOF, lane q forming the residual of child q, which the
+// first lane adds up in order.
+__global__ __launch_bounds__(256) void k_amg_resid_restrict(
+    int64_t n, int64_t nc, const uint32_t* kids, const uint32_t* cpos, const uint32_t* ccol,
+    const double* cval, const uint8_t* clen, const double* b, const double* x, double* bc) {
+  const int64_t t = blockIdx.x * 256ll + threadIdx.x;
+  const uint32_t k = t < 8 * nc ? kids[t] : kNone;
+  double r = 0;
+  if (k != kNone) {
+    const int64_t p = cpos[k];
+    const int len = clen[p];
+    uint32_t c[kSlots];
+    double v[kSlots], xv[kSlots];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      c[s] = s < len ? ccol[(int64_t)s * n + p] : 0u;
+      v[s] = s < len ? cval[(int64_t)s * n + p] : 0.0;
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) xv[s] = s < len ? x[c[s]] : 0.0;
+    r = b[k];
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+      if (s < len) r -= v[s] * xv[s];
+  }
+  double acc = 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const double rq = __shfl(r, q, 8);
+    const uint32_t kq = __shfl(k, q, 8);
+    if (kq != kNone) acc += 0.125 * rq;
+  }
+  if (t < 8 * nc && (t & 7) == 0) bc[t >> 3] = acc;
 }
 
 // y = A x on the colour-ordered rows (multiply, SparseMatrix.h:298-322)
@@ -319,12 +389,101 @@ __global__ void k_amg_spmv_c(int64_t n, const uint32_t* crow, const uint32_t* cc
   y[crow[p]] = acc;
 }
 
-// the coarsest level's sweeps with each thread's rows in registers: thread t
-// owns positions t + q * 1024; x in LDS
+// a / d correctly rounded, given y = 1 / d correctly rounded: two fma
+// refinements of a y, the last of an exact remainder (Markstein, IBM J. Res.
+// Dev. 34, 1990).  Holds while nothing over- or underflows: safe(a) and
+// safe(d) leave every exponent far from its ends.
+__device__ inline bool safe(double v) { return fabs(v) > 0x1p-400 && fabs(v) < 0x1p400; }
+__device__ inline double div_by(double a, double d, double y) {
+  const double q0 = a * y;
+  const double q1 = fma(fma(-d, q0, a), y, q0);
+  return fma(fma(-d, q1, a), y, q1);
+}
+
+// The coarsest level's sweeps in one workgroup, from x = 0 in LDS, for at most
+// 2 rows of each colour per thread, held in registers.  One compute unit's
+// issue bounds it, so a row's step is straight code: the entries in their
+// order, the diagonal's (and a short row's missing) place taken by 0 times an
+// LDS cell that holds 0, which adds +0 to a sum that is never -0, and the
+// division by the row's diagonal from its reciprocal (div_by; true division
+// where a wave holds a value outside its range).  200 sweeps of the coarsest
+// level of a 128^3 dam break: 268 us with a branch per entry and the
+// compiler's division, 156 now (a 64x61x83 tank: 231 and 113).
+constexpr int kFastRows = 2;
+struct FastRow {
+  double v[kSlots], b, d, y;
+  uint32_t c[(kSlots + 1) / 2];  // LDS cells, two per word
+  uint32_t out;                  // the row's own cell, or the spare one
+  bool zero;                     // no diagonal: the row's value is 0
+};
+__global__ __launch_bounds__(kCoarsestThreads) void k_amg_coarsest_f(
+    int n, int nred, const uint32_t* crow, const uint32_t* ccol, const double* cval,
+    const double* cdiag, const uint8_t* clen, const double* b, double* x, int iters) {
+  // cell n: 0; cell n + 1: written by threads without a row
+  __shared__ double xs[kCoarsestMax + 2];
+  const int nt = (int)blockDim.x;
+  FastRow R[2][kFastRows];  // red, black
+  bool fast = true;
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+#pragma unroll
+    for (int q = 0; q < kFastRows; ++q) {
+      FastRow& r = R[k][q];
+      const int p = (k ? nred : 0) + (int)threadIdx.x + q * nt;
+      const bool have = p < (k ? n : nred);
+      const uint32_t i = have ? crow[p] : 0u;
+      const int len = have ? clen[p] : 0;
+      const double diag = have ? cdiag[p] : 0.0;
+      r.out = have ? i : (uint32_t)n + 1;
+      r.zero = !(diag != 0);
+      r.d = r.zero ? 1.0 : diag;
+      r.y = 1.0 / r.d;
+      r.b = r.zero ? 1.0 : b[i];
+      fast = fast && safe(r.d);
+      uint32_t c[kSlots + 1];
+      c[kSlots] = 0;
+#pragma unroll
+      for (int s = 0; s < kSlots; ++s) {
+        const uint32_t cc = s < len ? ccol[(int64_t)s * n + p] : i;
+        const bool off = !r.zero && cc != i && cc < (uint32_t)n;
+        c[s] = off ? cc : (uint32_t)n;
+        r.v[s] = off ? cval[(int64_t)s * n + p] : 0.0;
+      }
+#pragma unroll
+      for (int s = 0; s < (kSlots + 1) / 2; ++s) r.c[s] = c[2 * s] | c[2 * s + 1] << 16;
+    }
+  for (int i = threadIdx.x; i < n + 2; i += nt) xs[i] = 0.0;
+  __syncthreads();
+  const bool all_fast = __all(fast);
+  for (int it = 0; it < iters; ++it)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+#pragma unroll
+      for (int q = 0; q < kFastRows; ++q) {
+        const FastRow& r = R[k][q];
+        if (q > 0 && (k ? n - nred : nred) <= q * nt) break;
+        double sum = 0;
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s)
+          sum += r.v[s] * xs[s & 1 ? r.c[s / 2] >> 16 : r.c[s / 2] & 0xFFFFu];
+        const double a = r.b - sum;
+        double v;
+        if (all_fast && __all(safe(a)))
+          v = div_by(a, r.d, r.y);
+        else
+          v = a / r.d;
+        xs[r.out] = r.zero ? 0.0 : v;
+      }
+      __syncthreads();
+    }
+  for (int i = threadIdx.x; i < n; i += nt) x[i] = xs[i];
+}
+
+// the same where a colour has more rows: thread t owns positions t + q * 1024
 __global__ __launch_bounds__(kCoarsestThreads) void k_amg_coarsest_c(
     int n, int nred, const uint32_t* crow, const uint32_t* ccol, const double* cval,
     const uint8_t* clen, const double* b, double* x, int iters) {
-  __shared__ double xs[kCoarsestMax];
+  __shared__ double xs[kCoarsestMax];  // from 0
   uint32_t row[kCoarsestRows];
   int len[kCoarsestRows];
   double bi[kCoarsestRows];
@@ -347,7 +506,7 @@ __global__ __launch_bounds__(kCoarsestThreads) void k_amg_coarsest_c(
       val[q][s] = s < len[q] ? cval[(int64_t)s * n + p] : 0.0;
     }
   }
-  for (int i = threadIdx.x; i < n; i += kCoarsestThreads) xs[i] = x[i];
+  for (int i = threadIdx.x; i < n; i += kCoarsestThreads) xs[i] = 0.0;
   __syncthreads();
   for (int it = 0; it < iters; ++it)
     for (int color = 1; color >= 0; --color) {
@@ -405,10 +564,12 @@ __global__ void k_amg_prolong(int64_t n, const uint32_t* parent, const double* x
   x[f] += 1.0 * (0.0 + 1.0 * xc[parent[f]]);
 }
 
+// iters red-black sweeps of a level; done: red passes already made
 void smooth(hipStream_t st, const AmgHier& H, const AmgLevel& L, const double* b, double* x,
-            int iters) {
+            int iters, int done = 0) {
   for (int it = 0; it < iters; ++it)
     for (int color = 1; color >= 0; --color) {
+      if (color && it < done) continue;
       if (H.compact) {
         const int64_t p0 = color ? 0 : L.nred, p1 = color ? L.nred : L.n;
         if (p1 > p0)
@@ -438,6 +599,8 @@ void AmgHier::release() {
     L.b.release();
     L.r.release();
     L.crow.release();
+    L.cpos.release();
+    L.cdiag.release();
     L.ccol.release();
     L.cval.release();
     L.clen.release();
@@ -534,11 +697,14 @@ void amg_build(hipStream_t st, AmgHier& H, const DevCsr& A, const int32_t* ijk, 
     WC_HIP(hipMemcpyAsync(H.nred.p + l, H.flag.p + L.n, sizeof(uint32_t),
                           hipMemcpyDeviceToDevice, st));
     L.crow.ensure((size_t)L.n);
+    L.cpos.ensure((size_t)L.n);
+    L.cdiag.ensure((size_t)L.n);
     L.clen.ensure((size_t)L.n);
     L.ccol.ensure((size_t)kSlots * L.n);
     L.cval.ensure((size_t)kSlots * L.n);
     hipLaunchKernelGGL(k_amg_compact, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.A, L.red.p,
-                       H.flag.p, L.crow.p, L.ccol.p, L.cval.p, L.clen.p, H.err.p);
+                       H.flag.p, L.crow.p, L.cpos.p, L.ccol.p, L.cval.p, L.cdiag.p, L.clen.p,
+                       H.err.p);
     WC_LAUNCH_CHECK();
   }
   int herr = 0;
@@ -568,7 +734,11 @@ bool amg_spmv(hipStream_t st, AmgHier& H, const double* x, double* y) {
   return true;
 }
 
-// AlgebraicMultigrid.h:179-245
+// AlgebraicMultigrid.h:179-245.  On colour-ordered rows the passes that only
+// prepare or carry vectors are part of the smoother's and the restriction's
+// kernels: the clear of x of the first red pass, the prolongation of the first
+// red pass after it, the residual of the restriction.  AMG-PCG solve, ms: 64^3
+// 4.2 -> 3.7, 128^3 4.9 -> 3.9, 256^3 16.0 -> 13.4 (with k_amg_coarsest_f).
 void amg_vcycle(hipStream_t st, AmgHier& H, const double* b, double* z) {
   const int nl = H.nl;
   const double* bl[kAmgMaxLevels];
@@ -576,24 +746,37 @@ void amg_vcycle(hipStream_t st, AmgHier& H, const double* b, double* z) {
   for (int l = 0; l < nl; ++l) {
     bl[l] = l == 0 ? b : H.L[l].b.p;
     xl[l] = l == 0 ? z : H.L[l].x.p;
-    WC_HIP(hipMemsetAsync(xl[l], 0, sizeof(double) * (size_t)H.L[l].n, st));
+    if (!H.compact || (l + 1 == nl && H.L[l].n > kCoarsestMax))
+      WC_HIP(hipMemsetAsync(xl[l], 0, sizeof(double) * (size_t)H.L[l].n, st));
   }
   for (int l = 0; l + 1 < nl; ++l) {
     AmgLevel& L = H.L[l];
-    smooth(st, H, L, bl[l], xl[l], 4);
-    if (H.compact)
-      hipLaunchKernelGGL(k_amg_resid_c, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.n, L.crow.p,
-                         L.ccol.p, L.cval.p, L.clen.p, bl[l], xl[l], L.r.p);
-    else
+    const int64_t nc = H.L[l + 1].n;
+    if (H.compact) {
+      hipLaunchKernelGGL(k_amg_first_red, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.n, L.nred,
+                         L.crow.p, L.cdiag.p, bl[l], xl[l]);
+      smooth(st, H, L, bl[l], xl[l], 4, 1);
+      hipLaunchKernelGGL(k_amg_resid_restrict, dim3(nblk(8 * nc, 256)), dim3(256), 0, st, L.n,
+                         nc, H.L[l + 1].kids.p, L.cpos.p, L.ccol.p, L.cval.p, L.clen.p, bl[l],
+                         xl[l], H.L[l + 1].b.p);
+    } else {
+      smooth(st, H, L, bl[l], xl[l], 4);
       hipLaunchKernelGGL(k_amg_resid, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.A, bl[l], xl[l],
                          L.r.p);
-    hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(H.L[l + 1].n, 256)), dim3(256), 0, st,
-                       H.L[l + 1].n, H.L[l + 1].kids.p, L.r.p, H.L[l + 1].b.p);
+      hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(nc, 256)), dim3(256), 0, st, nc,
+                         H.L[l + 1].kids.p, L.r.p, H.L[l + 1].b.p);
+    }
     WC_LAUNCH_CHECK();
   }
   AmgLevel& T = H.L[nl - 1];
   if (T.n <= kCoarsestMax) {
-    if (T.n > 0 && H.compact)
+    const int64_t most = std::max<int64_t>(T.nred, T.n - T.nred);  // rows of a colour
+    if (T.n > 0 && H.compact && most <= kFastRows * kCoarsestThreads)
+      hipLaunchKernelGGL(k_amg_coarsest_f, dim3(1),
+                         dim3((unsigned)std::min<int64_t>(kCoarsestThreads, (most + 63) / 64 * 64)),
+                         0, st, (int)T.n, (int)T.nred, T.crow.p, T.ccol.p, T.cval.p, T.cdiag.p,
+                         T.clen.p, bl[nl - 1], xl[nl - 1], 200);
+    else if (T.n > 0 && H.compact)
       hipLaunchKernelGGL(k_amg_coarsest_c, dim3(1), dim3(kCoarsestThreads), 0, st, (int)T.n,
                          (int)T.nred, T.crow.p, T.ccol.p, T.cval.p, T.clen.p, bl[nl - 1],
                          xl[nl - 1], 200);
@@ -606,10 +789,17 @@ void amg_vcycle(hipStream_t st, AmgHier& H, const double* b, double* z) {
   }
   for (int l = nl - 2; l >= 0; --l) {
     AmgLevel& L = H.L[l];
-    hipLaunchKernelGGL(k_amg_prolong, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.n, L.parent.p,
-                       xl[l + 1], xl[l]);
+    if (H.compact) {
+      if (L.nred > 0)
+        hipLaunchKernelGGL(k_amg_prolong_red, dim3(nblk(L.nred, 256)), dim3(256), 0, st, L.n,
+                           L.nred, L.crow.p, L.ccol.p, L.cval.p, L.clen.p, bl[l], L.parent.p,
+                           xl[l + 1], xl[l]);
+    } else {
+      hipLaunchKernelGGL(k_amg_prolong, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.n, L.parent.p,
+                         xl[l + 1], xl[l]);
+    }
     WC_LAUNCH_CHECK();
-    smooth(st, H, L, bl[l], xl[l], 4);
+    smooth(st, H, L, bl[l], xl[l], 4, H.compact ? 1 : 0);
   }
 }
 

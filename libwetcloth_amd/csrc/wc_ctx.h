@@ -231,7 +231,8 @@ struct AmgLevel {
   // ascending) with each row's entries in their order as 7 planes of n, so a
   // colour's smoothing reads only its own rows, coalesced
   int64_t nred = 0;
-  DevBuf<uint32_t> crow;        // compacted position -> row
+  DevBuf<uint32_t> crow, cpos;  // compacted position -> row, and back
+  DevBuf<double> cdiag;         // the value a position's row is divided by (0: none)
   DevBuf<uint32_t> ccol;        // [s * n + p]
   DevBuf<double> cval;
   DevBuf<uint8_t> clen;
