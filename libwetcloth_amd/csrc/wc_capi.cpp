@@ -1240,30 +1240,165 @@ struct CsrUpload {
   }
 };
 
+// What a context-free call works with: a stream and its buffers.  Creating
+// and freeing them took half of a call on 245,666 rows (72 allocations and
+// frees 5 ms, the stream 0.8 ms of 11 ms), so a call hands its session back to
+// a pool, at most kIdleSessions of at most kIdleBytes each per device; a
+// larger one is freed with its call, and the idle ones when an allocation of
+// any context or call fails (drop_idle_sessions, then tried once more).  A
+// session is used by one call at a time, with every array written by the call
+// itself; one whose call failed is not kept.
 struct FreeSession {
   hipStream_t st = nullptr;
+  int device = 0;
   CsrUpload csr;
   wc::PcgWork work;
+  wc::AmgHier amg;
+  wc::DevBuf<int32_t> ijk;
+  wc::DevBuf<double> in, out;
   FreeSession() { WC_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking)); }
   ~FreeSession() {
     if (st) (void)hipStreamSynchronize(st);
     csr.release();
     work.release();
+    amg.release();
+    ijk.release();
+    in.release();
+    out.release();
     if (st) (void)hipStreamDestroy(st);
   }
+  // upper bound of the device bytes held: the arrays are sized by rows or by
+  // stored entries, and no call allocates others
+  size_t held() const {
+    size_t b = 4 * (csr.rowptr.cap + csr.col.cap + work.tpos.cap + work.level.cap +
+                    work.lvl_count.cap + work.lvl_cursor.cap + work.lvl_list.cap + ijk.cap +
+                    amg.cmin.cap + amg.flag.cap) +
+               8 * (csr.val.cap + work.invdiag.cap + work.adiag.cap + work.lv.cap + work.r.cap +
+                    work.z.cap + work.s.cap + work.x.cap + in.cap + out.cap);
+    for (const wc::AmgLevel& L : amg.L)
+      b += 4 * (L.col.cap + L.len.cap + L.ijk.cap + L.parent.cap + L.kids.cap + L.crow.cap +
+                L.cpos.cap + L.ccol.cap) +
+           8 * (L.val.cap + L.x.cap + L.b.cap + L.r.cap + L.cval.cap + L.cdiag.cap) +
+           L.red.cap + L.clen.cap;
+    return b;
+  }
+};
+
+constexpr size_t kIdleSessions = 2, kIdleBytes = size_t(256) << 20;
+struct SessionPool {
+  std::mutex mu;
+  std::vector<FreeSession*> idle;
+};
+SessionPool& session_pool() {
+  // never destroyed: the runtime may be gone when static objects are
+  static SessionPool* p = new SessionPool;
+  return *p;
+}
+
+}  // namespace
+
+namespace wc {
+void drop_idle_sessions() {
+  SessionPool& P = session_pool();
+  std::vector<FreeSession*> idle;
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    idle.swap(P.idle);
+  }
+  for (FreeSession* f : idle) delete f;
+}
+}  // namespace wc
+
+namespace {
+
+// The session of one call, on the calling thread's device.
+class Session {
+ public:
+  Session() {
+    int dev = 0;
+    WC_HIP(hipGetDevice(&dev));
+    {
+      SessionPool& P = session_pool();
+      std::lock_guard<std::mutex> lock(P.mu);
+      for (size_t k = 0; k < P.idle.size(); ++k)
+        if (P.idle[k]->device == dev) {
+          s_ = P.idle[k];
+          P.idle.erase(P.idle.begin() + (ptrdiff_t)k);
+          break;
+        }
+    }
+    if (!s_) {
+      s_ = new FreeSession;
+      s_->device = dev;
+    }
+  }
+  ~Session() {
+    if (keep_ && s_->held() <= kIdleBytes) {
+      SessionPool& P = session_pool();
+      std::lock_guard<std::mutex> lock(P.mu);
+      size_t here = 0;
+      for (const FreeSession* f : P.idle) here += f->device == s_->device;
+      if (here < kIdleSessions) {
+        try {
+          P.idle.push_back(s_);
+          return;
+        } catch (const std::bad_alloc&) {
+        }
+      }
+    }
+    delete s_;
+  }
+  Session(const Session&) = delete;
+  Session& operator=(const Session&) = delete;
+  FreeSession& operator*() { return *s_; }
+  // the call has succeeded and its stream is idle
+  void done() { keep_ = true; }
+
+ private:
+  FreeSession* s_ = nullptr;
+  bool keep_ = false;
 };
 
 wc_status check_csr(int64_t n, const uint32_t* rs, const uint32_t* col) {
   if (n < 0 || (n > 0 && (!rs || !col))) return WC_ERR_ARG;
   if (n >= 0xFFFFFFFFll) return WC_ERR_ARG;
   if (rs && rs[0] != 0) return WC_ERR_ARG;
-  for (int64_t i = 0; i < n; ++i) {
+  // rows in ascending order first: the columns are only read below rs[n]
+  for (int64_t i = 0; i < n; ++i)
     if (rs[i + 1] < rs[i]) return WC_ERR_ARG;
-    for (uint32_t e = rs[i]; e < rs[i + 1]; ++e) {
-      if (col[e] >= (uint64_t)n) return WC_ERR_ARG;
-      if (e > rs[i] && col[e] <= col[e - 1]) return WC_ERR_ARG;
+  // each row's columns ascending and the last one below n
+  auto rows_ok = [&](int64_t i0, int64_t i1) {
+    bool bad = false;
+    for (int64_t i = i0; i < i1; ++i) {
+      const uint32_t b = rs[i], e = rs[i + 1];
+      if (b == e) continue;
+      for (uint32_t q = b + 1; q < e; ++q) bad |= col[q] <= col[q - 1];
+      bad |= col[e - 1] >= (uint64_t)n;
+    }
+    return !bad;
+  };
+  // 1.7 M entries take 1.9 ms on one core; threads pay from about 0.1 ms on
+  constexpr int kMost = 8;
+  const int64_t per = 1 << 17;  // entries a thread is worth
+  const int64_t nnz = n > 0 ? rs[n] : 0;
+  const int nthr = (int)std::min<int64_t>(
+      {nnz / per, kMost, (int64_t)std::max(1u, std::thread::hardware_concurrency())});
+  if (nthr < 2) return rows_ok(0, n) ? WC_OK : WC_ERR_ARG;
+  bool ok[kMost] = {};
+  std::thread th[kMost];
+  auto part = [&](int t) { ok[t] = rows_ok(n * t / nthr, n * (t + 1) / nthr); };
+  for (int t = 1; t < nthr; ++t) {
+    try {
+      th[t] = std::thread(part, t);
+    } catch (const std::exception&) {  // no thread to be had: the rows are checked below
     }
   }
+  for (int t = 0; t < nthr; ++t)
+    if (!th[t].joinable()) part(t);
+  for (int t = 1; t < nthr; ++t)
+    if (th[t].joinable()) th[t].join();
+  for (int t = 0; t < nthr; ++t)
+    if (!ok[t]) return WC_ERR_ARG;
   return WC_OK;
 }
 
@@ -1283,10 +1418,11 @@ wc_status wc_pcg_solve_csr(int64_t n, const uint32_t* rowstart,
   int it = 0;
   bool ok = true;
   try {
-    FreeSession S;
     if (n > 0) {
+      Session H;
+      FreeSession& S = *H;
       S.csr.up(S.st, n, rowstart, col, val);
-      wc::DevBuf<double> b, x;
+      wc::DevBuf<double>&b = S.in, &x = S.out;
       b.ensure(n);
       x.ensure(n);
       WC_HIP(hipMemcpyAsync(b.p, rhs, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
@@ -1295,11 +1431,12 @@ wc_status wc_pcg_solve_csr(int64_t n, const uint32_t* rowstart,
                          &res, &it);
       WC_HIP(hipMemcpyAsync(result, x.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
       WC_HIP(hipStreamSynchronize(S.st));
-      b.release();
-      x.release();
+      H.done();
     }
   } catch (const HipError& e) {
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
   if (residual_out) *residual_out = res;
   if (iters_out) *iters_out = it;
@@ -1474,9 +1611,25 @@ wc_status check_ijk(int64_t n, const int32_t* ijk, int32_t ni, int32_t nj, int32
       return WC_ERR_ARG;
   // every DOF its own cell: a coarse DOF keeps one child per position in
   // its 2x2x2 block
+  auto cell = [&](int64_t f) {
+    return ((int64_t)ijk[3 * f + 2] * nj + ijk[3 * f + 1]) * ni + ijk[3 * f];
+  };
+  // a bit per cell of the grid where that is no more memory than the cells'
+  // keys (245,666 DOFs: 0.3 ms, sorting the keys 5 ms)
+  const int64_t cells = (int64_t)ni * nj * nk;
+  if (cells <= 64 * n) {
+    std::vector<uint64_t> taken((size_t)(cells / 64 + 1));
+    for (int64_t f = 0; f < n; ++f) {
+      const int64_t k = cell(f);
+      uint64_t& w = taken[(size_t)(k >> 6)];
+      const uint64_t bit = 1ull << (k & 63);
+      if (w & bit) return WC_ERR_ARG;
+      w |= bit;
+    }
+    return WC_OK;
+  }
   std::vector<int64_t> key((size_t)n);
-  for (int64_t f = 0; f < n; ++f)
-    key[f] = ((int64_t)ijk[3 * f + 2] * nj + ijk[3 * f + 1]) * ni + ijk[3 * f];
+  for (int64_t f = 0; f < n; ++f) key[f] = cell(f);
   std::sort(key.begin(), key.end());
   for (int64_t f = 1; f < n; ++f)
     if (key[f] == key[f - 1]) return WC_ERR_ARG;
@@ -1487,29 +1640,28 @@ wc_status check_ijk(int64_t n, const int32_t* ijk, int32_t ni, int32_t nj, int32
 template <class F>
 wc_status with_amg(int64_t n, const uint32_t* rowstart, const uint32_t* col, const double* val,
                    const int32_t* ijk, int32_t ni, int32_t nj, int32_t nk, F run) {
-  if (check_csr(n, rowstart, col) != WC_OK || (n > 0 && !val))
-    return fail(nullptr, WC_ERR_ARG, "invalid CSR matrix (rows must be sorted, columns < n)");
-  if (check_ijk(n, ijk, ni, nj, nk) != WC_OK)
-    return fail(nullptr, WC_ERR_ARG,
-                "invalid DOF cells (need 0 <= i < ni, 0 <= j < nj, 0 <= k < nk, and no two DOFs in one cell)");
   try {
-    FreeSession S;
-    wc::AmgHier H;
-    wc::DevBuf<int32_t> dijk;
-    if (n > 0) {
-      S.csr.up(S.st, n, rowstart, col, val);
-      dijk.ensure(3 * (size_t)n);
-      WC_HIP(hipMemcpyAsync(dijk.p, ijk, sizeof(int32_t) * 3 * (size_t)n, hipMemcpyHostToDevice,
-                            S.st));
-      wc::amg_build(S.st, H, S.csr.A, dijk.p, ni, nj, nk);
-    }
-    const wc_status st = run(S, H);
+    if (check_csr(n, rowstart, col) != WC_OK || (n > 0 && !val))
+      return fail(nullptr, WC_ERR_ARG, "invalid CSR matrix (rows must be sorted, columns < n)");
+    if (check_ijk(n, ijk, ni, nj, nk) != WC_OK)
+      return fail(nullptr, WC_ERR_ARG,
+                  "invalid DOF cells (need 0 <= i < ni, 0 <= j < nj, 0 <= k < nk, and no two DOFs in one cell)");
+    if (n == 0) return WC_OK;
+    Session H;
+    FreeSession& S = *H;
+    S.csr.up(S.st, n, rowstart, col, val);
+    S.ijk.ensure(3 * (size_t)n);
+    WC_HIP(hipMemcpyAsync(S.ijk.p, ijk, sizeof(int32_t) * 3 * (size_t)n, hipMemcpyHostToDevice,
+                          S.st));
+    wc::amg_build(S.st, S.amg, S.csr.A, S.ijk.p, ni, nj, nk);
+    run(S);
     WC_HIP(hipStreamSynchronize(S.st));
-    H.release();
-    dijk.release();
-    return st;
+    H.done();
+    return WC_OK;
   } catch (const HipError& e) {
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
 }
 }  // namespace
@@ -1527,19 +1679,14 @@ wc_status wc_amgpcg_solve_csr(int64_t n, const uint32_t* rowstart, const uint32_
   int it = 0;
   bool ok = true;
   const wc_status st = with_amg(n, rowstart, col, val, dof_ijk, ni, nj, nk,
-                                [&](FreeSession& S, wc::AmgHier& H) -> wc_status {
-    if (n == 0) return WC_OK;
-    wc::DevBuf<double> b, x;
+                                [&](FreeSession& S) {
+    wc::DevBuf<double>&b = S.in, &x = S.out;
     b.ensure(n);
     x.ensure(n);
     WC_HIP(hipMemcpyAsync(b.p, rhs, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
     wc::pcg_prepare_vectors(S.st, S.work, n);
-    ok = wc::amgpcg_solve(S.st, S.work, H, S.csr.A, b.p, x.p, tol, maxit, &res, &it);
+    ok = wc::amgpcg_solve(S.st, S.work, S.amg, S.csr.A, b.p, x.p, tol, maxit, &res, &it);
     WC_HIP(hipMemcpyAsync(result, x.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
-    WC_HIP(hipStreamSynchronize(S.st));
-    b.release();
-    x.release();
-    return WC_OK;
   });
   if (st != WC_OK) return st;
   if (residual_out) *residual_out = res;
@@ -1552,18 +1699,12 @@ wc_status wc_amg_apply_csr(int64_t n, const uint32_t* rowstart, const uint32_t* 
                            int32_t nk, const double* r, double* z) {
   if (n > 0 && (!r || !z)) return fail(nullptr, WC_ERR_ARG, "bad argument");
   return with_amg(n, rowstart, col, val, dof_ijk, ni, nj, nk,
-                  [&](FreeSession& S, wc::AmgHier& H) -> wc_status {
-    if (n == 0) return WC_OK;
-    wc::DevBuf<double> dr, dz;
-    dr.ensure(n);
-    dz.ensure(n);
-    WC_HIP(hipMemcpyAsync(dr.p, r, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
-    wc::amg_vcycle(S.st, H, dr.p, dz.p);
-    WC_HIP(hipMemcpyAsync(z, dz.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
-    WC_HIP(hipStreamSynchronize(S.st));
-    dr.release();
-    dz.release();
-    return WC_OK;
+                  [&](FreeSession& S) {
+    S.in.ensure(n);
+    S.out.ensure(n);
+    WC_HIP(hipMemcpyAsync(S.in.p, r, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
+    wc::amg_vcycle(S.st, S.amg, S.in.p, S.out.p);
+    WC_HIP(hipMemcpyAsync(z, S.out.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
   });
 }
 
@@ -1574,7 +1715,8 @@ wc_status wc_mic0_factor_csr(int64_t n, const uint32_t* rowstart,
     return fail(nullptr, WC_ERR_ARG, "invalid CSR matrix");
   if (n == 0) return WC_OK;
   try {
-    FreeSession S;
+    Session H;
+    FreeSession& S = *H;
     S.csr.up(S.st, n, rowstart, col, val);
     wc::pcg_prepare(S.st, S.work, S.csr.A, nullptr, 0);
     wc::pcg_factor(S.st, S.work, S.csr.A, tau, mdr);
@@ -1584,11 +1726,14 @@ wc_status wc_mic0_factor_csr(int64_t n, const uint32_t* rowstart,
     std::vector<double> h(nnz);
     if (nnz) WC_HIP(hipMemcpyAsync(h.data(), S.work.lv.p, sizeof(double) * nnz, hipMemcpyDeviceToHost, S.st));
     WC_HIP(hipStreamSynchronize(S.st));
+    H.done();
     for (int64_t i = 0; i < n; ++i)
       for (uint32_t e = rowstart[i]; e < rowstart[i + 1]; ++e)
         lv[e] = col[e] > (uint32_t)i ? h[e] : 0.0;
   } catch (const HipError& e) {
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
   return WC_OK;
 }
@@ -1600,24 +1745,25 @@ wc_status wc_mic0_apply_csr(int64_t n, const uint32_t* rowstart,
     return fail(nullptr, WC_ERR_ARG, "invalid CSR matrix");
   if (n == 0) return WC_OK;
   try {
-    FreeSession S;
+    Session H;
+    FreeSession& S = *H;
     S.csr.up(S.st, n, rowstart, col, nullptr);
     wc::pcg_prepare(S.st, S.work, S.csr.A, nullptr, 0);
     const int64_t nnz = rowstart[n];
     WC_HIP(hipMemcpyAsync(S.work.invdiag.p, invdiag, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
     if (nnz) WC_HIP(hipMemcpyAsync(S.work.lv.p, lv, sizeof(double) * nnz, hipMemcpyHostToDevice, S.st));
-    wc::DevBuf<double> dr, dz;
-    dr.ensure(n);
-    dz.ensure(n);
-    WC_HIP(hipMemcpyAsync(dr.p, r, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
-    wc::pcg_apply(S.st, S.work, S.csr.A, dr.p, dz.p);
+    S.in.ensure(n);
+    S.out.ensure(n);
+    WC_HIP(hipMemcpyAsync(S.in.p, r, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
+    wc::pcg_apply(S.st, S.work, S.csr.A, S.in.p, S.out.p);
     wc::pcg_check(S.st, S.work);
-    WC_HIP(hipMemcpyAsync(z, dz.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
+    WC_HIP(hipMemcpyAsync(z, S.out.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
     WC_HIP(hipStreamSynchronize(S.st));
-    dr.release();
-    dz.release();
+    H.done();
   } catch (const HipError& e) {
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
   return WC_OK;
 }
@@ -1628,19 +1774,20 @@ wc_status wc_spmv_csr(int64_t n, const uint32_t* rowstart, const uint32_t* col,
     return fail(nullptr, WC_ERR_ARG, "invalid CSR matrix");
   if (n == 0) return WC_OK;
   try {
-    FreeSession S;
+    Session H;
+    FreeSession& S = *H;
     S.csr.up(S.st, n, rowstart, col, val);
-    wc::DevBuf<double> dx, dy;
-    dx.ensure(n);
-    dy.ensure(n);
-    WC_HIP(hipMemcpyAsync(dx.p, x, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
-    wc::pcg_spmv(S.st, S.csr.A, dx.p, dy.p);
-    WC_HIP(hipMemcpyAsync(y, dy.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
+    S.in.ensure(n);
+    S.out.ensure(n);
+    WC_HIP(hipMemcpyAsync(S.in.p, x, sizeof(double) * n, hipMemcpyHostToDevice, S.st));
+    wc::pcg_spmv(S.st, S.csr.A, S.in.p, S.out.p);
+    WC_HIP(hipMemcpyAsync(y, S.out.p, sizeof(double) * n, hipMemcpyDeviceToHost, S.st));
     WC_HIP(hipStreamSynchronize(S.st));
-    dx.release();
-    dy.release();
+    H.done();
   } catch (const HipError& e) {
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
   return WC_OK;
 }

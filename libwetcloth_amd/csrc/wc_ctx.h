@@ -28,6 +28,9 @@ struct HipError {
   } while (0)
 #define WC_LAUNCH_CHECK() WC_HIP(hipGetLastError())
 
+// frees the idle workspaces of the context-free calls (wc_capi.cpp)
+void drop_idle_sessions();
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -53,7 +56,12 @@ struct DevBuf {
     cap = 0;
     size_t c = n ? n : 1;
     if (regrow) c += c / 4;
-    WC_HIP(hipMalloc((void**)&p, c * sizeof(T)));
+    if (hipMalloc((void**)&p, c * sizeof(T)) != hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+      drop_idle_sessions();
+      WC_HIP(hipMalloc((void**)&p, c * sizeof(T)));
+    }
     cap = c;
   }
   void release() {

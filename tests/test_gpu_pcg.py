@@ -185,3 +185,40 @@ def test_apply_pattern_not_symmetric(wc):
     z1 = (y1 - lv[5] * z2) * inv[1]
     z0 = ((y0 - lv[1] * z1) - lv[2] * z2) * inv[0]
     assert np.array_equal(wc.mic0_apply_csr(rs, col, inv, lv, r), [z0, z1, z2])
+
+
+def test_calls_share_workspaces_safely(oracle, wc, systems):
+    """Calls of different kinds and sizes one after another, and from several
+    threads at once, give each its own answer (their workspaces are reused),
+    and a refused call in between changes nothing."""
+    from concurrent.futures import ThreadPoolExecutor
+    jobs = []
+    for name in ("dam16", "grid9", "grid9_null_rows"):
+        rs, col, val, b = systems[name]
+        inv, lv = oracle.mic0(rs, col, val)
+        jobs.append((lambda a=(rs, col, inv, lv, b): wc.mic0_apply_csr(*a),
+                     oracle.apply_precond(rs, col, inv, lv, b)))
+        jobs.append((lambda a=(rs, col, val, b): wc.spmv_csr(*a), oracle.spmv(rs, col, val, b)))
+    for job, want in jobs + jobs[::-1]:
+        assert np.array_equal(job(), want)
+        with pytest.raises(wc.WetclothError):
+            wc.spmv_csr(np.array([0, 1], np.uint32), np.array([5], np.uint32), np.ones(1),
+                        np.ones(1))
+    with ThreadPoolExecutor(4) as pool:
+        for (_, want), got in zip(jobs * 6, pool.map(lambda j: j[0](), jobs * 6)):
+            assert np.array_equal(got, want)
+
+
+def test_large_csr_validation(wc):
+    """A matrix large enough to be checked by several threads: one bad column
+    in any part is found, a good one passes."""
+    n = 200_000
+    rs = np.arange(0, 3 * n + 1, 3, dtype=np.uint32)
+    col = (np.clip(np.arange(n), 1, n - 2)[:, None] + np.array([-1, 0, 1])).astype(np.uint32)
+    val, x = np.ones(3 * n), np.ones(n)
+    assert np.array_equal(wc.spmv_csr(rs, col.ravel(), val, x), np.full(n, 3.0))
+    for row, bad in ((0, n), (n // 2, 0), (n - 1, n + 7)):
+        c = col.copy()
+        c[row, 2] = bad
+        with pytest.raises(wc.WetclothError):
+            wc.spmv_csr(rs, c.ravel(), val, x)
