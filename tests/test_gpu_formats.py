@@ -84,3 +84,37 @@ def test_load_position_only_rejects_mismatched_files(wc, tmp_path):
     x4b, _, _ = s.particles_reference_layout()
     assert np.array_equal(x4b, x4)
     s.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [1, 255, 256, 769])
+def test_particle_arrays_round_trip(wc, prec, n):
+    """Host arrays in and out in both layouts, exactly (FP32-rounded in the mixed
+    form), at the edges of a launch, in a context sized for n and then for a third
+    of it (the staging memory holds all of C at once or a group at a time), in
+    sorted order after a substep, with missing quantities zero."""
+    s = wc.Scene((N, N, N), 1.0 / N, precision=wc.WC_FP64 if prec == "fp64" else wc.WC_MIXED)
+    rng = np.random.default_rng(n)
+    rnd = (lambda a: a) if prec == "fp64" else (lambda a: a.astype(np.float32).astype(np.float64))
+    for m in (n, (n + 2) // 3):
+        x = rng.uniform(0.1, 0.9, (3, m))
+        v = rng.normal(size=(3, m))
+        Cm = rng.normal(size=(9, m))
+        s.set_particles(x, v, Cm)
+        for a, b in zip(s.particles(), (x, v, Cm)):
+            assert np.array_equal(a, rnd(b))
+        s.step(DT, 1e-8, 500)
+        xs, vs, Cs = s.particles()
+        x4, v4, fB = s.particles_reference_layout()
+        assert np.array_equal(x4.reshape(m, 4)[:, :3].T, xs)
+        assert np.array_equal(v4.reshape(m, 4)[:, :3].T, vs)
+        assert not x4[3::4].any() and not v4[3::4].any()
+        # fB is 3N x 3, column-major: value (3 p + r, c) is C_rc of particle p
+        assert np.array_equal(fB.reshape(3, m, 3).transpose(2, 0, 1).reshape(9, m), Cs)
+        s.set_particles_reference_layout(x4, v4, fB)
+        for a, b in zip(s.particles(), (xs, vs, Cs)):
+            assert np.array_equal(a, b)
+        s.set_particles(x)
+        xs, vs, Cs = s.particles()
+        assert np.array_equal(xs, rnd(x)) and not vs.any() and not Cs.any()
+    s.close()
