@@ -166,6 +166,9 @@ struct SweepPlan {
   // the -x coupling plane (once per plan)
   DevBuf<double> cf15, xf15, xf0;
   DevBuf<float> cf15_32, xf15_32, xf0_32;
+  // for box_spmv_pcg, of the solve's value type: the preconditioned vector's
+  // columns (li = 15, then li = 0), a second direction and its columns
+  DevBuf<double> zc, s2, sc2;
   // The forward sweep's ticket counter is zero: the sweeps zero each
   // other's counter, so only the first apply after the plan needs a clear.
   bool ticks_zero = false;
@@ -183,6 +186,8 @@ struct GridSystem {
   const uint32_t* col = nullptr;
   const uint8_t* live = nullptr;  // per DOF: its row holds a nonzero value
 };
+
+constexpr int kHostParts = 1024;  // |r|_inf partials in mapped host memory
 
 // Device work space of the MIC(0)-PCG solver (PCGSolver.h:310-314).
 struct PcgWork {
@@ -216,7 +221,7 @@ struct PcgWork {
   double* host_scal = nullptr;  // pinned, or host_scal_own when no_alloc
   bool no_alloc = false;        // every buffer lent (DevBuf::lend); no pinned memory either
   double host_scal_own[8] = {};
-  double* host_part = nullptr;  // mapped host memory, red_blocks |r| partials
+  double* host_part = nullptr;  // mapped host memory, kHostParts |r| partials
   double* host_part_dev = nullptr;  // its device address
   void release();
 };
@@ -510,7 +515,42 @@ struct DotParts {
 DotParts box_spmv_dot(hipStream_t st, SweepPlan& P, const double* x, double* y,
                       double* partial, int nblocks, bool faces_ready = false);
 DotParts box_spmv32_dot(hipStream_t st, SweepPlan& P, const float* x, float* y,
-                        double* partial, int nblocks, bool faces_ready = false);
+                        double* partial, int nblocks, bool faces_ready = false);// PCG's residual update inside the forward sub-tile sweep that applies the
+// preconditioner to it: r -= y alpha, alpha = scal[rho] / (the sum of d) left
+// in scal[alpha], and each unit's |r|_inf in rpart (-2 for the first unit's
+// where the abort flag is set; P.nua * P.nub entries, mapped host memory).
+bool pcg_in_passes(const SweepPlan& P);
+template <class V>
+struct ResidualUpdate {
+  const V* y;
+  V* r;
+  DotParts d;
+  double* scal;
+  int rho, alpha;
+  double* rpart;
+};
+// the apply with r updated first; z's x-face columns are written too, for
+// box_spmv_pcg
+void sweep_apply_pcg(hipStream_t st, SweepPlan& P, double* r, KTimer* timer, int64_t ndof,
+                     const ResidualUpdate<double>& U);
+void sweep_apply_pcg(hipStream_t st, SweepPlan& P, float* r, KTimer* timer, int64_t ndof,
+                     const ResidualUpdate<float>& U);
+
+// One PCG direction in box layout with its x-face columns.
+template <class V>
+struct Direction {
+  V *v, *c15, *c0;
+};
+// The PCG iteration's head in one launch (sub-tile sweeps and windowed SpMV
+// only): sn = z + s beta, the solution P.xb += s alpha, y = A sn and the
+// partials of sn . y, z being the last apply's result and beta taken from
+// its z . r partials; scal holds rho_old and alpha, and rho_new is written.
+DotParts box_spmv_pcg(hipStream_t st, SweepPlan& P, const Direction<double>& s,
+                      const Direction<double>& sn, double* y, double* scal, int rho_old,
+                      int rho_new, int alpha);
+DotParts box_spmv_pcg(hipStream_t st, SweepPlan& P, const Direction<float>& s,
+                      const Direction<float>& sn, float* y, double* scal, int rho_old,
+                      int rho_new, int alpha);
 void box_residual(hipStream_t st, const SweepPlan& P, const double* b, const double* x,
                   float* r, double* partial, int nblocks);
 void box_gather(hipStream_t st, const SweepPlan& P, const double* dof, double* box);

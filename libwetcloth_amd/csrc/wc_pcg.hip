@@ -676,6 +676,52 @@ __global__ __launch_bounds__(kRedThreads) void k_update_xr_fused(
   }
 }
 
+// The same without x, which box_spmv_pcg updates an iteration later:
+// r -= z alpha, alpha left in scal for it.
+template <class V>
+__global__ __launch_bounds__(kRedThreads) void k_update_r(
+    V* r, const V* z, int64_t n, const double* dpart, int nb, double* scal, int rho_slot,
+    double* rpart, const int* flag) {
+  __shared__ double sh[kRedThreads];
+  double acc = 0;
+  for (int i = threadIdx.x; i < nb; i += kRedThreads) acc += dpart[i];
+  const double sz = block_sum(acc, sh);
+  const double alpha = scal[rho_slot] / sz;  // PCGSolver.h:291
+  if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_ALPHA] = alpha;
+  const double nalpha = -alpha;
+  __syncthreads();  // every thread has read the sum before sh is reused
+  double m = 0;
+  auto one = [&](V& r_, V z_) {
+    r_ = (V)((double)r_ + (double)z_ * nalpha);
+    m = fmax(m, fabs((double)r_));
+  };
+  using PV = Pack<V>;
+  constexpr int N = PV::N;
+  const int64_t nv = n / N;
+  for (int64_t i = blockIdx.x * (int64_t)kRedThreads + threadIdx.x; i < nv;
+       i += (int64_t)gridDim.x * kRedThreads) {
+    PV rv = reinterpret_cast<const PV*>(r)[i];
+    const PV zv = reinterpret_cast<const PV*>(z)[i];
+#pragma unroll
+    for (int k = 0; k < N; ++k) one(rv.v[k], zv.v[k]);
+    reinterpret_cast<PV*>(r)[i] = rv;
+  }
+  for (int64_t i = nv * N + blockIdx.x * (int64_t)kRedThreads + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * kRedThreads)
+    one(r[i], z[i]);
+  const double mm = block_max(m, sh);
+  if (threadIdx.x == 0) rpart[blockIdx.x] = blockIdx.x == 0 && *flag ? -2.0 : mm;
+}
+
+// x += s alpha for the last iteration of a solve
+template <class V>
+__global__ __launch_bounds__(256) void k_update_x(double* x, const V* s, int64_t n,
+                                                 const double* scal) {
+  const double alpha = scal[S_ALPHA];
+  for (int64_t i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+    x[i] += (double)s[i] * alpha;
+}
+
 // beta = (z . r) / rho_old (PCGSolver.h:301), s = z + s beta; the new rho is
 // written to the other rho slot, which no block reads here.  With f15 / f0,
 // also the x-face columns of s that the windowed SpMV reads: s at the slots
@@ -828,7 +874,8 @@ void pcg_prepare(hipStream_t st, PcgWork& w, const DevCsr& A,
   w.r.ensure(n);
   w.s.ensure(n);
   w.x.ensure(n);
-  w.red_blocks = (int)std::min<int64_t>(1024, std::max<int64_t>(1, (n + kRedThreads - 1) / kRedThreads));
+  w.red_blocks = (int)std::min<int64_t>(
+      kHostParts, std::max<int64_t>(1, (n + kRedThreads - 1) / kRedThreads));
   w.partial.ensure(w.red_blocks);
   w.scal.ensure(S_NSCAL);
   w.level_in = level;
@@ -845,7 +892,7 @@ void pcg_prepare(hipStream_t st, PcgWork& w, const DevCsr& A,
   }
   // written by the update kernels of the box loops, read by the host
   if (!w.host_part) {
-    WC_HIP(hipHostMalloc((void**)&w.host_part, sizeof(double) * 1024,
+    WC_HIP(hipHostMalloc((void**)&w.host_part, sizeof(double) * kHostParts,
                          hipHostMallocMapped | hipHostMallocCoherent));
     WC_HIP(hipHostGetDevicePointer((void**)&w.host_part_dev, w.host_part, 0));
   }
@@ -856,7 +903,8 @@ void pcg_prepare_vectors(hipStream_t st, PcgWork& w, int64_t n) {
   w.r.ensure(n);
   w.z.ensure(n);
   w.s.ensure(n);
-  w.red_blocks = (int)std::min<int64_t>(1024, std::max<int64_t>(1, (n + kRedThreads - 1) / kRedThreads));
+  w.red_blocks = (int)std::min<int64_t>(
+      kHostParts, std::max<int64_t>(1, (n + kRedThreads - 1) / kRedThreads));
   w.partial.ensure(w.red_blocks);
   w.scal.ensure(S_NSCAL);
   if (!w.host_scal) WC_HIP(hipHostMalloc((void**)&w.host_scal, sizeof(double) * S_NSCAL));
@@ -1071,14 +1119,14 @@ static void force_abort(hipStream_t st, SweepPlan& P) {
 }
 
 static void clear_residual(PcgWork& w) {
-  for (int i = 0; i < w.red_blocks; ++i) w.host_part[i] = -1.0;
+  for (int i = 0; i < kHostParts; ++i) w.host_part[i] = -1.0;
 }
 
-static double box_residual_max(hipStream_t st, PcgWork& w,
+// nb: how many partials the update writes
+static double box_residual_max(hipStream_t st, PcgWork& w, int nb,
                                const char* abort_text = "pipelined MIC(0) sweep: a tile wait "
                                                         "exceeded its bound") {
   volatile const double* hp = w.host_part;
-  const int nb = w.red_blocks;
   int i = 0;
   const auto t0 = std::chrono::steady_clock::now();
   for (long spin = 1;; ++spin) {
@@ -1102,7 +1150,8 @@ static double box_residual_max(hipStream_t st, PcgWork& w,
     throw HipError{hipErrorLaunchTimeOut, abort_text, __FILE__, __LINE__};
   double m = 0;
   for (int k = 0; k < nb; ++k) m = fmax(m, hp[k]);
-  clear_residual(w);  // for the next update, which the host enqueues after this
+  // for the next update, which the host enqueues after this
+  for (int k = 0; k < nb; ++k) w.host_part[k] = -1.0;
   return m;
 }
 
@@ -1112,6 +1161,68 @@ static double box_residual_max(hipStream_t st, PcgWork& w,
 static void settle_timer(hipStream_t, PcgWork& w) {
   if (w.timer.on && !w.timer.pending.empty()) w.timer.harvest_ready();
 }
+
+// The PCG iteration of small plans (pcg_in_passes), every vector updated in a
+// pass that reads its operands anyway: s and the solution in the SpMV
+// (box_spmv_pcg), r in the forward sweep that is applied to it
+// (ResidualUpdate).  Two directions in turn; y = A s in the forward sweep's
+// output, which is dead until the sweep has read y.
+template <class V>
+struct FusedIter {
+  hipStream_t st;
+  PcgWork& w;
+  SweepPlan& P;
+  Direction<V> d[2];
+  V *r, *y;
+  int cur = 0, rho_slot = S_RHO;
+  bool first = true;
+  FusedIter(hipStream_t st_, PcgWork& w_, V* s, V* c15, V* c0, V* r_, V* y_)
+      : st(st_), w(w_), P(w_.sweep), r(r_), y(y_) {
+    const int64_t words = (P.ncell * (int64_t)sizeof(V) + 7) / 8;
+    P.s2.ensure(words);
+    P.sc2.ensure(words / 8);  // two columns of ncell / 16
+    V* c = reinterpret_cast<V*>(P.sc2.p);
+    d[0] = {s, c15, c0};
+    d[1] = {reinterpret_cast<V*>(P.s2.p), c, c + P.ncell / 16};
+  }
+  // One iteration up to the next apply (where one follows); |r|_inf
+  double step(KTimer* ti, int64_t ndof, bool more) {
+    hipEvent_t e0 = ti ? ti->mark(st) : nullptr;
+    DotParts dp;
+    if (first) {
+      if constexpr (sizeof(V) == sizeof(double))
+        dp = box_spmv_dot(st, P, d[cur].v, y, w.partial.p, w.red_blocks, false);
+      else
+        dp = box_spmv32_dot(st, P, d[cur].v, y, w.partial.p, w.red_blocks, false);
+      first = false;
+    } else {
+      const int next = rho_slot == S_RHO ? S_RHO2 : S_RHO;
+      dp = box_spmv_pcg(st, P, d[cur], d[cur ^ 1], y, w.scal.p, rho_slot, next, (int)S_ALPHA);
+      rho_slot = next;
+      cur ^= 1;
+    }
+    if (e0) ti->add(KTimer::SPMV, ndof, e0, ti->mark(st));
+    if (more) {
+      const ResidualUpdate<V> U = {y, r, dp, w.scal.p, rho_slot, (int)S_ALPHA, w.host_part_dev};
+      sweep_apply_pcg(st, P, r, ti, ndof, U);
+      return box_residual_max(st, w, P.nua * P.nub);
+    }
+    hipLaunchKernelGGL(k_update_r<V>, dim3(w.red_blocks), dim3(kRedThreads), 0, st, r, y, P.ncell,
+                       dp.p, dp.n, w.scal.p, rho_slot, w.host_part_dev, P.progress.p + 2);
+    WC_LAUNCH_CHECK();
+    return box_residual_max(st, w, w.red_blocks);
+  }
+  // the solution's update the next SpMV would have made
+  void finish() {
+    if (first) return;
+    hipLaunchKernelGGL(k_update_x<V>, dim3(blocks_upto(P.ncell)), dim3(256), 0, st, P.xb.p,
+                       d[cur].v, P.ncell, w.scal.p);
+    WC_LAUNCH_CHECK();
+  }
+  static unsigned blocks_upto(int64_t n) {
+    return (unsigned)std::min<int64_t>(4096, (n + 255) / 256);
+  }
+};
 
 // The PCG loop of PCGSolver::solve (PCGSolver.h:280-304) on box vectors: the
 // pipelined sweeps apply MIC(0) in place and the SpMV is the box stencil.
@@ -1150,6 +1261,24 @@ static bool pcg_loop_box(hipStream_t st, PcgWork& w, int64_t ndof, const double*
   int rho_slot = S_RHO;
   int it;
   bool ok = false;
+  if (pcg_in_passes(P)) {
+    FusedIter<double> F(st, w, s, P.xf15.p, P.xf0.p, r, P.zf.p);
+    for (it = 0; it < maxit; ++it) {
+      KTimer* ti = tm ? tm->sample() : nullptr;
+      const double res = F.step(ti, ndof, it + 1 < maxit);
+      *residual_out = res;
+      if (res <= tolr) {
+        ++it;
+        ok = true;
+        break;
+      }
+    }
+    F.finish();
+    *iters_out = it;
+    box_scatter(st, P, x, x_dof);
+    settle_timer(st, w);
+    return ok;
+  }
   for (it = 0; it < maxit; ++it) {
     KTimer* ti = tm ? tm->sample() : nullptr;
     hipEvent_t e0 = ti ? ti->mark(st) : nullptr;
@@ -1170,7 +1299,7 @@ static bool pcg_loop_box(hipStream_t st, PcgWork& w, int64_t ndof, const double*
       WC_LAUNCH_CHECK();
       rho_slot = rho_next;
     }
-    const double res = box_residual_max(st, w);
+    const double res = box_residual_max(st, w, nb);
     *residual_out = res;
     if (res <= tolr) {
       ++it;
@@ -1251,6 +1380,17 @@ static bool pcg_loop_box_mixed(hipStream_t st, PcgWork& w, int64_t ndof, const d
     // outputs, which the next refinement pass recomputes)
     clear_residual(w);
     int rho_slot = S_RHO;
+    if (pcg_in_passes(P)) {
+      FusedIter<float> F(st, w, s, P.xf15_32.p, P.xf0_32.p, r, P.zf32.p);
+      while (total < maxit) {
+        KTimer* ti = tm ? tm->sample() : nullptr;
+        ++total;
+        const double r32 = F.step(ti, ndof, total < maxit);
+        if (r32 <= inner_tol || r32 != r32) break;
+      }
+      F.finish();
+      continue;
+    }
     bool faces = false;  // s's face columns, written by the s update
     while (total < maxit) {
       KTimer* ti = tm ? tm->sample() : nullptr;
@@ -1273,7 +1413,7 @@ static bool pcg_loop_box_mixed(hipStream_t st, PcgWork& w, int64_t ndof, const d
         WC_LAUNCH_CHECK();
         rho_slot = rho_next;
       }
-      const double r32 = box_residual_max(st, w);
+      const double r32 = box_residual_max(st, w, nb);
       if (r32 <= inner_tol || r32 != r32) break;
     }
   }
@@ -1361,7 +1501,7 @@ bool pcg_solve(hipStream_t st, PcgWork& w, const DevCsr& A, const double* b,
         WC_LAUNCH_CHECK();
         rho_slot = rho_next;
       }
-      res = box_residual_max(st, w, kPassAbort);
+      res = box_residual_max(st, w, w.red_blocks, kPassAbort);
       *residual_out = res;
       if (res <= tolr) {
         ++it;

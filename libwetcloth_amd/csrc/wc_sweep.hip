@@ -737,9 +737,30 @@ struct WinRow {
   uint16_t f;
   V a0, up[3], xn;          // diagonal, upper planes; x of the next step
   V cl[2], xl[2], xu[2];    // face neighbours in the next tile (x, y)
+  V sn, sl[2], su[2];       // PCG: the old s beside xn, xl and xu (z) ...
+  double q;                 // ... and the solution at the next step
 };
 
-template <class V, bool DOT>
+// With PCG, x is not stored before the product but formed by it: the PCG's
+// new direction s = z + s beta (k_update_s_fused's expression, so its bits),
+// with beta from the backward sweep's z . r partials, each block summing them;
+// and the solution's update for the previous iteration, q += s alpha, which
+// needs the old s that is read here anyway.  A block's halo (the steps beside
+// its run, the faces of the next tiles) is formed again from z and the old s,
+// so the new s goes to a second buffer.
+template <class V>
+struct PcgUpdate {
+  const V *z, *z15, *z0;     // the preconditioned vector and its x-face columns
+  const V *s, *s15, *s0;     // the old direction
+  V *sn, *sn15, *sn0;        // the new one
+  double* q;
+  const double* zr;          // partials of z . r
+  int nzr;
+  double* scal;
+  int rho_old, rho_new, alpha;
+};
+
+template <class V, bool DOT, bool PCG>
 __global__ __launch_bounds__(256) void k_box_spmv_win(uint32_t nslot, Skew K, int run, int nrun,
                                                      const uint16_t* __restrict__ sflag,
                                                      const V* __restrict__ coef,
@@ -747,7 +768,8 @@ __global__ __launch_bounds__(256) void k_box_spmv_win(uint32_t nslot, Skew K, in
                                                      const V* __restrict__ f15,
                                                      const V* __restrict__ f0,
                                                      const V* __restrict__ c15,
-                                                     V* __restrict__ y, double* partial) {
+                                                     V* __restrict__ y, double* partial,
+                                                     PcgUpdate<V> U) {
   __shared__ V xs[4][kThreads];     // x of step w at [w & 3]
   __shared__ V us[3][3][kThreads];  // upper planes of step w at [w % 3]
   __shared__ double sh[kThreads / 64];  // the waves' x . y sums
@@ -761,7 +783,12 @@ __global__ __launch_bounds__(256) void k_box_spmv_win(uint32_t nslot, Skew K, in
   const uint32_t dx = (uint32_t)(int32_t)K.dx, dy = (uint32_t)(int32_t)K.dy;
   const uint32_t last = nslot - 1;
   auto clampn = [&](uint32_t n) { return n < last ? n : last; };
-  auto ldx = [&](int w) -> V { return w >= 0 && w < nsteps ? x[tb + (uint32_t)w * kThreads] : (V)0; };
+  const V* const vx = PCG ? U.z : x;
+  const V* const v15 = PCG ? U.z15 : f15;
+  const V* const v0 = PCG ? U.z0 : f0;
+  auto ldx = [&](const V* p, int w) -> V {
+    return w >= 0 && w < nsteps ? p[tb + (uint32_t)w * kThreads] : (V)0;
+  };
   // the loads of step w (w0 <= w < w1); the face slots are clamped into the
   // box and used only where the neighbour exists (then they are in it); the
   // x faces come from the compact columns of x and of the -x coupling plane
@@ -771,36 +798,92 @@ __global__ __launch_bounds__(256) void k_box_spmv_win(uint32_t nslot, Skew K, in
     R.a0 = coef[t];
 #pragma unroll
     for (int d = 0; d < 3; ++d) R.up[d] = coef[(uint32_t)(4 + d) * nslot + t];
-    R.xn = ldx(w + 1);
+    R.xn = ldx(vx, w + 1);
+    if constexpr (PCG) {
+      R.sn = ldx(U.s, w + 1);
+      if (w + 1 < w1) R.q = U.q[t + kThreads];
+    }
     if (li == 0) {
       const uint32_t n = clampn(t + dx) >> 4;
       R.cl[0] = c15[n];
-      R.xl[0] = f15[n];
+      R.xl[0] = v15[n];
+      if constexpr (PCG) R.sl[0] = U.s15[n];
     }
     if (lj == 0) {
       const uint32_t n = clampn(t + dy);
       R.cl[1] = coef[5u * nslot + n];
-      R.xl[1] = x[n];
+      R.xl[1] = vx[n];
+      if constexpr (PCG) R.sl[1] = U.s[n];
     }
-    if (li == kT - 1) R.xu[0] = f0[clampn(t - dx) >> 4];
-    if (lj == kT - 1) R.xu[1] = x[clampn(t - dy)];
+    if (li == kT - 1) {
+      const uint32_t n = clampn(t - dx) >> 4;
+      R.xu[0] = v0[n];
+      if constexpr (PCG) R.su[0] = U.s0[n];
+    }
+    if (lj == kT - 1) {
+      const uint32_t n = clampn(t - dy);
+      R.xu[1] = vx[n];
+      if constexpr (PCG) R.su[1] = U.s[n];
+    }
   };
-  xs[(w0 + 3) & 3][lane] = ldx(w0 - 1);
-  xs[w0 & 3][lane] = ldx(w0);
+  V xp0 = ldx(vx, w0 - 1), xc0 = ldx(vx, w0);  // the run's first two steps
 #pragma unroll
   for (int d = 0; d < 3; ++d)
     us[(w0 + 2) % 3][d][lane] =
         w0 > 0 ? coef[(uint32_t)(4 + d) * nslot + tb + (uint32_t)(w0 - 1) * kThreads] : (V)0;
   WinRow<V> R;
   R.cl[0] = R.cl[1] = R.xl[0] = R.xl[1] = R.xu[0] = R.xu[1] = (V)0;
+  R.sn = R.sl[0] = R.sl[1] = R.su[0] = R.su[1] = (V)0;
+  R.q = 0.0;
   fetch(w0, R);
+  double beta = 0.0, alpha = 0.0;
+  auto dir = [&](V z, V s) -> V {
+    return PCG ? (V)((double)z + (double)s * beta) : z;
+  };
+  // step w's s and solution stored (q: the solution before), for its own run
+  auto keep = [&](int w, V v, V s, double q) {
+    const uint32_t t = tb + (uint32_t)w * kThreads;
+    U.sn[t] = v;
+    if (li == kT - 1) U.sn15[t >> 4] = v;
+    if (li == 0) U.sn0[t >> 4] = v;
+    U.q[t] = q + (double)s * alpha;
+  };
+  if constexpr (PCG) {
+    const V sp = ldx(U.s, w0 - 1), sc = ldx(U.s, w0);
+    const double q0 = U.q[tb + (uint32_t)w0 * kThreads];
+    double zr = 0.0;
+    for (int i = lane; i < U.nzr; i += kThreads) zr += U.zr[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) zr += __shfl_xor(zr, o, 64);
+    if ((lane & 63) == 0) sh[lane >> 6] = zr;
+    __syncthreads();
+    zr = ((sh[0] + sh[1]) + sh[2]) + sh[3];
+    beta = zr / U.scal[U.rho_old];  // PCGSolver.h:301
+    alpha = U.scal[U.alpha];
+    if (blockIdx.x == 0 && lane == 0) U.scal[U.rho_new] = zr;
+    xp0 = dir(xp0, sp);
+    xc0 = dir(xc0, sc);
+    keep(w0, xc0, sc, q0);
+  }
+  xs[(w0 + 3) & 3][lane] = xp0;
+  xs[w0 & 3][lane] = xc0;
   double acc = 0.0;
   for (int w = w0; w < w1; ++w) {
-    const WinRow<V> C = R;
+    WinRow<V> C = R;
 #pragma unroll
     for (int d = 0; d < 3; ++d) us[w % 3][d][lane] = C.up[d];
+    if constexpr (PCG) {
+      C.xn = dir(C.xn, C.sn);
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        C.xl[d] = dir(C.xl[d], C.sl[d]);
+        C.xu[d] = dir(C.xu[d], C.su[d]);
+      }
+    }
     xs[(w + 1) & 3][lane] = C.xn;
     if (w + 1 < w1) fetch(w + 1, R);
+    if constexpr (PCG)
+      if (w + 1 < w1) keep(w + 1, C.xn, C.sn, C.q);
     __syncthreads();  // step w + 1's x and step w's planes are in place
     const uint32_t f = C.f;
     const bool dof = (f & M_DOF) != 0;
@@ -918,6 +1001,16 @@ struct SweepArgs {
   V* reset;                // forward tile sweep: set to the sentinel step by step
   V* mail;                 // sub-tile sweeps: the records units exchange ...
   V* mail_reset;           // ... and the other pass's, set to the sentinel
+  // the PCG forms of the sub-tile sweeps: the backward result's x-face
+  // columns; forward r (in) -= y alpha first, as ResidualUpdate
+  V *col15, *col0;
+  const V* y;
+  V* r;
+  const double* dpart;
+  int ndpart;
+  double* scal;
+  int rho, alpha;
+  double* rpart;
   const V* dot_r;          // backward sweep: r (the forward sweep's input) ...
   double* dot_out;         // ... and its per-tile partials of z . r
   int* ticket;
@@ -1520,7 +1613,7 @@ struct SubRing {
     return a;
   }
   static constexpr int kAhead = ahead();
-  static_assert(kAhead >= 2 && kAhead < kBatches, "the ring holds the batches in flight");
+  static_assert(kAhead >= 4 && kAhead < kBatches, "the ring holds the batches in flight");
 };
 
 // s_waitcnt lgkmcnt(0) alone (gfx9 encoding)
@@ -1540,10 +1633,11 @@ __device__ inline void store_mail(double v, __amdgpu_buffer_rsrc_t b, uint32_t o
                                         kSc1);
 }
 
-template <int KIND, class V>
-__global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
+template <int KIND, class V, bool PCG>
+__global__ __launch_bounds__(kSubThreads + (PCG ? 64 : 0)) void k_sweep_sub(SweepArgs<V> S) {
   static_assert(KIND == K_FWD || KIND == K_BWD, "sweeps only");
   constexpr bool BWD = KIND == K_BWD;
+  constexpr bool UPD = PCG && !BWD;  // r's update first
   using Ring = SubRing<V>;
   constexpr int kRB = Ring::kBatches;
   constexpr int kLA = Ring::kAhead;
@@ -1557,7 +1651,8 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     CellT<V> rc[kRB][kNB][64];
     V rr[kRB][kNB][64];
     uint32_t rk[kRB][kNB][64];
-    V rq[BWD ? kRB : 1][kNB][64];
+    V rq[BWD || UPD ? kRB : 1][kNB][64];  // backward: r; r's update: y
+    double red[4];
     int unit;
   } sh;
   auto& pl = sh.pl;
@@ -1580,6 +1675,15 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     const int t = atomicAdd(S.ticket, 1);
     sh.unit = (int)S.order[t];
     if (t == 0) *S.next_ticket = 0;  // the other pass's counter
+  }
+  if constexpr (UPD) {
+    // s . (A s), while the ticket is drawn
+    double d = 0.0;
+    if (wave < 4)
+      for (int i = threadIdx.x; i < S.ndpart; i += kSubThreads) d += S.dpart[i];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o, 64);
+    if (lane == 0 && wave < 4) sh.red[wave] = d;
   }
   __syncthreads();
   const int unit = __builtin_amdgcn_readfirstlane(sh.unit);
@@ -1644,16 +1748,20 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
         }
       stream(S.in, &rr[r][0][0], n, EV{});
       stream(S.code, &rk[r][0][0], n, E4{});
-      if constexpr (BWD) stream(S.dot_r, &rq[r][0][0], n, EV{});
+      if constexpr (BWD || UPD) stream(BWD ? S.dot_r : S.y, &rq[r][0][0], n, EV{});
     };
-    constexpr int kLoads = BWD ? Ring::kBwdLoads : Ring::kFwdLoads;
+    constexpr int kLoads = BWD || UPD ? Ring::kBwdLoads : Ring::kFwdLoads;
+    // with r's update a batch is complete one barrier earlier: wave 4
+    // updates its r in between
+    constexpr int kEarly = UPD ? 1 : 0;
     for (int n = 0; n < kLA; ++n) issue(n);
-    wait_vmcnt<(kLA - 1) * kLoads>();
+    wait_vmcnt<(kLA - 1 - kEarly) * kLoads>();
+    if constexpr (UPD) __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_s_barrier();  // batch 0's records
     for (int n = 0; n < nb; ++n) {
-      // batch n + 1 complete; the loads of the kLA - 2 batches after it may
-      // still be in flight
-      wait_vmcnt<(kLA - 2) * kLoads>();
+      // batch n + 1 (n + 2) complete; the loads of the batches after
+      // it may still be in flight
+      wait_vmcnt<(kLA - 2 - kEarly) * kLoads>();
       __builtin_amdgcn_s_barrier();
       issue(n + kLA);
     }
@@ -1711,6 +1819,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     };
     // batch 0 is due at the first batch's barrier
     fetch(0);
+    if constexpr (UPD) __syncthreads();
     __syncthreads();
     publish(0);
     if (1 < nb) fetch(1);
@@ -1722,6 +1831,66 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
       }
     }
     __syncthreads();
+    return;
+  }
+  // the cell of compute lane l in an exchange plane
+  auto cell = [&](int l) -> uint32_t {
+    return (uint32_t)((kS * sb + (l >> 3) + 1) * (kT + 1) + kS * sa + (l & 7) + 1);
+  };
+  if (PCG && wave == 4) {
+    // the PCG form's wave: forward, r of batch n is updated in the ring, one
+    // barrier before the compute wave reads it, and stored; backward, the
+    // x-face column the unit holds (k_face_cols' layout) is stored by lanes
+    // (step, row), a batch after the compute wave.  (By the store wave: 32.0
+    // / 32.6 us a sweep at 64^3 FP64; plain sweeps 27.6 / 29.5.)
+    if constexpr (UPD) {
+      double m = 0.0;
+      const double sz = ((sh.red[0] + sh.red[1]) + sh.red[2]) + sh.red[3];
+      const double alpha = S.scal[S.rho] / sz;  // PCGSolver.h:291
+      if (unit == 0 && lane == 0) S.scal[S.alpha] = alpha;
+      const double nalpha = -alpha;
+      auto upd = [&](int n) {
+#pragma unroll
+        for (int st = 0; st < kNB; ++st) {
+          const int w = n * kNB + st, rg = n & (kRB - 1);
+          const V v = (V)((double)rr[rg][st][lane] + (double)rq[rg][st][lane] * nalpha);
+          if (w < wend) {
+            rr[rg][st][lane] = v;
+            *at(S.r, slot(w, lane)) = v;
+            m = fmax(m, fabs((double)v));
+          }
+        }
+      };
+      __syncthreads();  // batches 0 and 1
+      upd(0);
+      if (1 < nb) upd(1);
+      __syncthreads();
+      for (int n = 0; n < nb; ++n) {
+        __syncthreads();
+        if (n + 2 < nb) upd(n + 2);
+      }
+      __syncthreads();
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+      // (the host polls these; -2 tells it of an earlier pass's abort)
+      if (lane == 0) S.rpart[ub * S.nua + ua] = unit == 0 && load_flag(S.abort_flag) ? -2.0 : m;
+    } else {
+      V* const col =
+          (psa ? S.col15 : S.col0) + ((tile0 >> 4) + (uint32_t)(kS * psb + lane % kS));
+      const uint32_t from = cell(63 - (lane % kS * kS + (psa ? kS - 1 : 0)));
+      auto put = [&](int n) {
+        const int w = n * kNB + lane / kS;
+        if (lane < kNB * kS && w < wend)
+          *at(col, (uint32_t)(nsteps - 1 - w0 - w) * kT) = pl[PL(w) + from];
+      };
+      __syncthreads();
+      for (int n = 0; n < nb; ++n) {
+        __syncthreads();
+        if (n > 0) put(n - 1);
+      }
+      __syncthreads();
+      put(nb - 1);
+    }
     return;
   }
   if (wave == 3) {
@@ -1738,9 +1907,6 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
     constexpr int kOps = kNB * kPer / 64;     // stores per batch
     struct alignas(16) Quad {
       V v[kVec];
-    };
-    auto cell = [&](int l) -> uint32_t {
-      return (uint32_t)((kS * sb + (l >> 3) + 1) * (kT + 1) + kS * sa + (l & 7) + 1);
     };
     auto put = [&](int n) {
 #pragma unroll
@@ -1779,6 +1945,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
         if (w < wend) dot += (double)pl[PL(w) + cown] * (double)rsave[st];
       }
     };
+    if constexpr (UPD) __syncthreads();
     __syncthreads();
     for (int n = 0; n < nb; ++n) {
       __syncthreads();  // batch n - 1 computed, batch n handed over
@@ -1865,6 +2032,7 @@ __global__ __launch_bounds__(kSubThreads) void k_sweep_sub(SweepArgs<V> S) {
   };
   Rec r0, r1;
   wait_lgkmcnt0();
+  if constexpr (UPD) __syncthreads();
   __syncthreads();  // batch 0's records
 #pragma unroll
   for (int st = 0; st < kNB; ++st) read(r0, 0, st);
@@ -2013,6 +2181,11 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const doub
   P.xf15.ensure(P.ncell / 16);
   P.xf0.ensure(P.ncell / 16);
   face_cols<double>(st, P.ncell, P.coef.p + 4 * P.ncell, P.cf15.p, nullptr);
+  if (pcg_in_passes(P)) {
+    // both columns of the preconditioned vector: zero where no unit runs, as zb
+    P.zc.ensure(P.ncell / 8);
+    WC_HIP(hipMemsetAsync(P.zc.p, 0, sizeof(double) * (P.ncell / 8), st));
+  }
   WC_HIP(hipStreamSynchronize(st));  // 'order' and 'order_sub' must outlive their copies
   P.valid = true;
 }
@@ -2114,7 +2287,8 @@ static V* ready_mail(hipStream_t st, SweepPlan& P) {
 
 template <class V>
 static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, const V* cb,
-                       V* zf, V* zb, KTimer* timer, int64_t ndof, bool cleared) {
+                       V* zf, V* zb, V* zc, KTimer* timer, int64_t ndof, bool cleared,
+                       const ResidualUpdate<V>* U = nullptr) {
   // Two ticket counters; the outputs start as the sentinel.  Each pass zeroes
   // the other pass's counter, and the forward pass's rhs loader sets every
   // slot of zb to the sentinel as it goes, so an apply clears only zf (just
@@ -2145,9 +2319,23 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
     S.mail_reset = mail + mail_values(P);
   }
   P.ndot = S.ntiles;
+  if (U) {
+    S.y = U->y;
+    S.r = U->r;
+    S.dpart = U->d.p;
+    S.ndpart = U->d.n;
+    S.scal = U->scal;
+    S.rho = U->rho;
+    S.alpha = U->alpha;
+    S.rpart = U->rpart;
+  }
   hipEvent_t e0 = timer ? timer->mark(st) : nullptr;
-  if (sub)
-    hipLaunchKernelGGL((k_sweep_sub<K_FWD, V>), dim3(S.ntiles), dim3(kSubThreads), 0, st, S);
+  if (U)
+    hipLaunchKernelGGL((k_sweep_sub<K_FWD, V, true>), dim3(S.ntiles), dim3(kSubThreads + 64), 0,
+                       st, S);
+  else if (sub)
+    hipLaunchKernelGGL((k_sweep_sub<K_FWD, V, false>), dim3(S.ntiles), dim3(kSubThreads), 0, st,
+                       S);
   else
     hipLaunchKernelGGL((k_sweep<K_FWD, V>), dim3(P.ntiles), dim3(SweepBlock<K_FWD>::value), 0, st, S);
   WC_LAUNCH_CHECK();
@@ -2158,13 +2346,21 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   S.reset = nullptr;
   S.dot_r = r;
   S.dot_out = P.tdot.p;
+  if (U) {
+    S.col15 = zc;
+    S.col0 = zc + P.ncell / 16;
+  }
   S.code = P.opb.p;
   S.ticket = tick + 1;
   S.next_ticket = tick;
   std::swap(S.mail, S.mail_reset);
   hipEvent_t e2 = timer ? timer->mark(st) : nullptr;
-  if (sub)
-    hipLaunchKernelGGL((k_sweep_sub<K_BWD, V>), dim3(S.ntiles), dim3(kSubThreads), 0, st, S);
+  if (U)
+    hipLaunchKernelGGL((k_sweep_sub<K_BWD, V, true>), dim3(S.ntiles), dim3(kSubThreads + 64), 0,
+                       st, S);
+  else if (sub)
+    hipLaunchKernelGGL((k_sweep_sub<K_BWD, V, false>), dim3(S.ntiles), dim3(kSubThreads), 0, st,
+                       S);
   else
     hipLaunchKernelGGL((k_sweep<K_BWD, V>), dim3(P.ntiles), dim3(SweepBlock<K_BWD>::value), 0, st, S);
   WC_LAUNCH_CHECK();
@@ -2175,14 +2371,27 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   }
 }
 
+// (the columns are for box_spmv_pcg only)
 void sweep_apply(hipStream_t st, SweepPlan& P, const double* r, KTimer* timer,
                  int64_t ndof, bool cleared) {
-  apply_impl<double>(st, P, r, P.cf.p, P.cb.p, P.zf.p, P.zb.p, timer, ndof, cleared);
+  apply_impl<double>(st, P, r, P.cf.p, P.cb.p, P.zf.p, P.zb.p, nullptr, timer, ndof, cleared);
 }
 
 void sweep_apply32(hipStream_t st, SweepPlan& P, const float* r, KTimer* timer,
                    int64_t ndof, bool cleared) {
-  apply_impl<float>(st, P, r, P.cf32.p, P.cb32.p, P.zf32.p, P.zb32.p, timer, ndof, cleared);
+  apply_impl<float>(st, P, r, P.cf32.p, P.cb32.p, P.zf32.p, P.zb32.p, nullptr, timer, ndof,
+                    cleared);
+}
+
+void sweep_apply_pcg(hipStream_t st, SweepPlan& P, double* r, KTimer* timer, int64_t ndof,
+                     const ResidualUpdate<double>& U) {
+  apply_impl<double>(st, P, r, P.cf.p, P.cb.p, P.zf.p, P.zb.p, P.zc.p, timer, ndof, false, &U);
+}
+
+void sweep_apply_pcg(hipStream_t st, SweepPlan& P, float* r, KTimer* timer, int64_t ndof,
+                     const ResidualUpdate<float>& U) {
+  apply_impl<float>(st, P, r, P.cf32.p, P.cb32.p, P.zf32.p, P.zb32.p,
+                    reinterpret_cast<float*>(P.zc.p), timer, ndof, false, &U);
 }
 
 static unsigned spmv_blocks(const SweepPlan& P) {
@@ -2201,6 +2410,19 @@ static int spmv_run_of(const SweepPlan& P) {
   return steps < 1024 ? 1 : steps < 2048 ? 2 : steps < 8192 ? 4 : 8;
 }
 
+// Whether the PCG iteration's vector updates run inside the SpMV and the
+// sweeps: three launches instead of five.  That pays while launches and
+// latency bound the iteration; on large systems the updates' traffic costs the
+// sweeps as much as it saves.  us per iteration, five launches / three (FP64,
+// then mixed): 16^3 41.5 / 35.2, 43.7 / 38.5; 32^3 50.6 / 45.5, 50.8 / 45.7;
+// 64^3 78.1 / 72.9, 75.2 / 69.8; 96^3 102.9 / 97.4, 96.2 / 92.4; 128^3 (4000
+// tile steps) 135.4 / 127.7, 125.2 / 118.7; 192^3 (12000) 275 / 282, 203 / 206;
+// 256^3 468 / 472, 351 / 346.
+bool pcg_in_passes(const SweepPlan& P) {
+  return P.sub && P.spmv_win && (int64_t)P.ntiles * P.nsteps < 8192 &&
+         P.nua * P.nub <= kHostParts;
+}
+
 // faces_ready: the columns of x are already in f15 / f0 (the s update
 // writes them); else they are extracted first
 template <class V, bool DOT>
@@ -2211,11 +2433,45 @@ static DotParts spmv_win(hipStream_t st, SweepPlan& P, const V* coef, const V* c
   const int nb = P.ntiles * nrun;
   if (DOT) P.spart.ensure(nb);
   if (!faces_ready) face_cols<V>(st, P.ncell, x, f15, f0);
-  hipLaunchKernelGGL((k_box_spmv_win<V, DOT>), dim3(nb), dim3(kThreads), 0, st,
+  hipLaunchKernelGGL((k_box_spmv_win<V, DOT, false>), dim3(nb), dim3(kThreads), 0, st,
                      (uint32_t)P.ncell, skew_of(P), run, nrun, P.sflag.p, coef, x, f15,
-                     f0, c15, y, DOT ? P.spart.p : nullptr);
+                     f0, c15, y, DOT ? P.spart.p : nullptr, PcgUpdate<V>{});
   WC_LAUNCH_CHECK();
   return DotParts{P.spart.p, nb};
+}
+
+template <class V>
+static DotParts spmv_pcg(hipStream_t st, SweepPlan& P, const V* coef, const V* c15,
+                         const PcgUpdate<V>& U, V* y) {
+  const int run = spmv_run_of(P);
+  const int nrun = (P.nsteps + run - 1) / run;
+  const int nb = P.ntiles * nrun;
+  P.spart.ensure(nb);
+  hipLaunchKernelGGL((k_box_spmv_win<V, true, true>), dim3(nb), dim3(kThreads), 0, st,
+                     (uint32_t)P.ncell, skew_of(P), run, nrun, P.sflag.p, coef, nullptr, nullptr,
+                     nullptr, c15, y, P.spart.p, U);
+  WC_LAUNCH_CHECK();
+  return DotParts{P.spart.p, nb};
+}
+
+template <class V>
+static PcgUpdate<V> pcg_update(SweepPlan& P, const V* z, const Direction<V>& s, const Direction<V>& sn, double* scal,
+                               int rho_old, int rho_new, int alpha) {
+  const V* zc = reinterpret_cast<const V*>(P.zc.p);
+  return {z, zc, zc + P.ncell / 16, s.v, s.c15, s.c0, sn.v, sn.c15, sn.c0, P.xb.p, P.tdot.p, P.ndot,
+          scal, rho_old, rho_new, alpha};
+}
+DotParts box_spmv_pcg(hipStream_t st, SweepPlan& P, const Direction<double>& s,
+                      const Direction<double>& sn, double* y, double* scal, int rho_old,
+                      int rho_new, int alpha) {
+  return spmv_pcg<double>(st, P, P.coef.p, P.cf15.p,
+                          pcg_update<double>(P, P.zb.p, s, sn, scal, rho_old, rho_new, alpha), y);
+}
+DotParts box_spmv_pcg(hipStream_t st, SweepPlan& P, const Direction<float>& s,
+                      const Direction<float>& sn, float* y, double* scal, int rho_old,
+                      int rho_new, int alpha) {
+  return spmv_pcg<float>(st, P, P.coef32.p, P.cf15_32.p,
+                         pcg_update<float>(P, P.zb32.p, s, sn, scal, rho_old, rho_new, alpha), y);
 }
 
 void box_spmv(hipStream_t st, SweepPlan& P, const double* x, double* y) {
@@ -2311,6 +2567,9 @@ void SweepPlan::release() {
   cf15.release();
   xf15.release();
   xf0.release();
+  zc.release();
+  s2.release();
+  sc2.release();
   cf15_32.release();
   xf15_32.release();
   xf0_32.release();

@@ -235,3 +235,36 @@ def test_box_without_empty_rows(oracle, wc, n, block_hi):
         s.set_option("sweep_subtiles", sub)
         assert np.array_equal(s.apply_preconditioner(r), want), sub
     assert np.array_equal(s.multiply(r), oracle.spmv(rs, col, val, r))
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("n,block_hi,run", [(16, (0.4, 0.6, 1.0), 0), (24, (1.0, 0.15, 0.2), 3),
+                                             (40, (0.9, 0.3, 0.55), 7), (64, (0.4, 0.6, 1.0), 0)])
+def test_iteration_in_passes(wc, n, block_hi, run, mixed):
+    """The PCG iteration with its vector updates inside the SpMV and the sweeps
+    against the one with a launch for each (chosen by the slot-parallel SpMV),
+    on one system, stopped after 1, 2, 3 and 8 iterations.  Both evaluate the
+    same expressions; only the order of the inner products' sums differs.  In
+    FP64 that moves alpha and beta by ~n eps (1e-13 here at most), grown by
+    less than 1e3 over the iterations; in the mixed form a vector's FP32
+    rounding (6e-8) may flip, grown the same way."""
+    s = wc.Scene((n, n, n), 1.0 / n, precision=wc.WC_MIXED if mixed else wc.WC_FP64)
+    s.seed_block((0.0, 0.0, 0.0), block_hi, seed=3, sigma=0.5)
+    s.rebucketizeParticles()
+    s.mapParticleNodesAPIC()
+    s.stepVelocity(1.0 / 480)
+    if run:
+        s.set_option("spmv_run", run)
+    for maxit in (1, 2, 3, 8):
+        out = []
+        for win in (1, 0):
+            s.set_option("spmv_window", win)
+            ok, it, res = s.projectFine(1.0 / 480, 1e-12, maxit)
+            out.append((ok, it, res, s.system()[4].copy()))
+        (oka, ita, resa, pa), (okb, itb, resb, pb) = out
+        assert not oka and not okb and ita == itb == maxit
+        assert np.abs(pb).max() > 0
+        assert np.abs(pa - pb).max() <= (6e-5 if mixed else 1e-10) * np.abs(pb).max(), maxit
+        if not mixed:
+            assert abs(resa - resb) <= 1e-8 * resb
+    s.close()
