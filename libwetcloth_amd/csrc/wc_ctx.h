@@ -2,6 +2,7 @@
 // kernel module exports to the C ABI layer (wc_capi.cpp).
 #pragma once
 
+#include <initializer_list>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -412,6 +413,14 @@ namespace wc {
 // In-place exclusive scan of n uint32 values; returns the total.
 uint32_t exclusive_scan(wc_ctx* ctx, uint32_t* data, int64_t n);
 uint32_t exclusive_scan(hipStream_t st, DevBuf<uint32_t>& scratch, uint32_t* data, int64_t n);
+// Byte fills (0 or 0xFF) of several ranges in one launch (wc_scan.hip); every
+// range starts at a 16-byte boundary.
+struct Fill {
+  void* p;
+  int64_t bytes;
+  int value;
+};
+void fill_ranges(hipStream_t st, std::initializer_list<Fill> list);
 // the same without reading the total back (no host wait); the scratch must
 // not be reused before the scan has run
 void exclusive_scan_async(hipStream_t st, DevBuf<uint32_t>& scratch, uint32_t* data, int64_t n);

@@ -188,7 +188,7 @@ struct DofArgs {
   const uint8_t* act;
   const double* lphi;
   const double* w[3];
-  uint32_t* isdof;
+  uint32_t *isdof, *dofscan;  // both: nnode flags and a zero
   FrozenView F;
 };
 
@@ -197,6 +197,7 @@ struct DofArgs {
 __global__ void k_dof_flags(DofArgs A) {
   const int64_t n = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
   const Grid& g = A.g;
+  if (n == g.nnode) A.isdof[n] = A.dofscan[n] = 0;
   if (n >= g.nnode) return;
   uint32_t f = 0;
   if (A.act[n >> 6] && fz_liquid(A.F, A.lphi, n)) {
@@ -211,6 +212,7 @@ __global__ void k_dof_flags(DofArgs A) {
     }
   }
   A.isdof[n] = f;
+  A.dofscan[n] = f;
 }
 
 struct AsmArgs {
@@ -545,12 +547,10 @@ int64_t grid_assemble(wc_ctx* ctx, double dt) {
   D.lphi = ctx->lphi.p;
   for (int d = 0; d < 3; ++d) D.w[d] = ctx->w[d].p;
   D.isdof = ctx->isdof.p;
+  D.dofscan = ctx->dofscan.p;
   D.F = frozen_view(ctx);
-  hipLaunchKernelGGL(k_dof_flags, dim3(blocks(g.nnode, 256)), dim3(256), 0, st, D);
+  hipLaunchKernelGGL(k_dof_flags, dim3(blocks(g.nnode + 1, 256)), dim3(256), 0, st, D);
   WC_LAUNCH_CHECK();
-  WC_HIP(hipMemsetAsync(ctx->isdof.p + g.nnode, 0, sizeof(uint32_t), st));
-  WC_HIP(hipMemcpyAsync(ctx->dofscan.p, ctx->isdof.p,
-                        sizeof(uint32_t) * (g.nnode + 1), hipMemcpyDeviceToDevice, st));
   const int64_t ndof = exclusive_scan(ctx, ctx->dofscan.p, g.nnode + 1);
   ctx->ndof = ndof;
   ctx->rowlen.ensure(ndof);

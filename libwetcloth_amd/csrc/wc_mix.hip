@@ -421,21 +421,17 @@ void mix_set(wc_ctx* ctx, int64_t ne, const double* x, const double* m, const do
     M.sat[d].ensure(nn);
     M.Q[d].ensure(nn);
     M.hdv[d].ensure(nn);
-    WC_HIP(hipMemsetAsync(M.sat[d].p, 0, sizeof(double) * nn, st));
-    WC_HIP(hipMemsetAsync(M.Q[d].p, 0, sizeof(double) * nn, st));
-    WC_HIP(hipMemsetAsync(M.hdv[d].p, 0, sizeof(double) * nn, st));
   }
   M.psi_p.ensure(nn);
   M.sat_p.ensure(nn);
   M.pp.ensure(nn);
-  WC_HIP(hipMemsetAsync(M.acc.p, 0, sizeof(double) * 3 * kPlanes * nn, st));
-  WC_HIP(hipMemsetAsync(M.cvs.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.cvf.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.cvl.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.psi_p.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.sat_p.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.pp.p, 0, sizeof(double) * nn, st));
-  WC_HIP(hipMemsetAsync(M.touch.p, 0, g.nbucket, st));
+  const int64_t bytes = sizeof(double) * nn;
+  fill_ranges(st, {{M.sat[0].p, bytes, 0}, {M.sat[1].p, bytes, 0}, {M.sat[2].p, bytes, 0},
+                   {M.Q[0].p, bytes, 0}, {M.Q[1].p, bytes, 0}, {M.Q[2].p, bytes, 0},
+                   {M.hdv[0].p, bytes, 0}, {M.hdv[1].p, bytes, 0}, {M.hdv[2].p, bytes, 0},
+                   {M.acc.p, 3 * kPlanes * bytes, 0}, {M.cvs.p, bytes, 0}, {M.cvf.p, bytes, 0},
+                   {M.cvl.p, bytes, 0}, {M.psi_p.p, bytes, 0}, {M.sat_p.p, bytes, 0},
+                   {M.pp.p, bytes, 0}, {M.touch.p, g.nbucket, 0}});
   SolidArgs A;
   A.g = g;
   A.ne = ne;

@@ -924,14 +924,15 @@ void sort_impl(wc_ctx* ctx, Planes<R> P) {
   ctx->adj.ready = false;
   ctx->bcount.ensure(g.nbucket + 1);
   ctx->bcursor.ensure(g.nbucket + 1);
-  WC_HIP(hipMemsetAsync(ctx->bcount.p, 0, sizeof(uint32_t) * (g.nbucket + 1), st));
-  WC_HIP(hipMemsetAsync(ctx->bcursor.p, 0, sizeof(uint32_t) * (g.nbucket + 1), st));
+  const int64_t bytes = sizeof(uint32_t) * (g.nbucket + 1);
+  fill_ranges(st, {{ctx->bcount.p, bytes, 0}, {ctx->bcursor.p, bytes, 0}});
   if (n > 0) {
     hipLaunchKernelGGL(k_sort_keys<R>, dim3(blocks(n, 256)), dim3(256), 0, st, g,
                        P.x->p, n, cap, ctx->pkey.p, ctx->bcount.p);
     WC_LAUNCH_CHECK();
   }
-  exclusive_scan(ctx, ctx->bcount.p, g.nbucket + 1);  // bcount becomes bstart
+  // bcount becomes bstart (the total is n: not read back)
+  exclusive_scan_async(st, ctx->scan_tmp, ctx->bcount.p, g.nbucket + 1);
   std::swap(ctx->bcount, ctx->bstart);
   ctx->bcount.ensure(g.nbucket + 1);
   if (n > 0) {
@@ -1188,12 +1189,11 @@ void particles_p2g(wc_ctx* ctx) {
   const Grid& g = ctx->g;
   hipStream_t st = ctx->stream;
   const int64_t nn = g.nnode;
-  for (int d = 0; d < 3; ++d) {
-    WC_HIP(hipMemsetAsync(ctx->mass[d].p, 0, sizeof(double) * nn, st));
-    WC_HIP(hipMemsetAsync(ctx->mom[d].p, 0, sizeof(double) * nn, st));
-  }
-  WC_HIP(hipMemsetAsync(ctx->phikey.p, 0xFF, sizeof(unsigned long long) * nn, st));
-  WC_HIP(hipMemsetAsync(ctx->touched.p, 0, g.nbucket, st));
+  const int64_t bytes = sizeof(double) * nn;
+  fill_ranges(st, {{ctx->mass[0].p, bytes, 0}, {ctx->mom[0].p, bytes, 0},
+                   {ctx->mass[1].p, bytes, 0}, {ctx->mom[1].p, bytes, 0},
+                   {ctx->mass[2].p, bytes, 0}, {ctx->mom[2].p, bytes, 0},
+                   {ctx->phikey.p, bytes, 0xFF}, {ctx->touched.p, g.nbucket, 0}});
   if (ctx->np == 0) return;
   if (ctx->mixed)
     p2g_launch(ctx, planes(ctx, 0.0f));

@@ -4,6 +4,8 @@
 // std::partial_sum of Pressure.cpp:421) and seeding compaction.
 #include "wc_ctx.h"
 
+#include <algorithm>
+
 namespace wc {
 namespace {
 
@@ -98,6 +100,47 @@ uint32_t exclusive_scan(hipStream_t st, DevBuf<uint32_t>& scratch, uint32_t* dat
 
 uint32_t exclusive_scan(wc_ctx* ctx, uint32_t* data, int64_t n) {
   return exclusive_scan(ctx->stream, ctx->scan_tmp, data, n);
+}
+
+namespace {
+constexpr int kMaxFills = 20;
+struct FillArgs {
+  Fill f[kMaxFills];
+  int n;
+};
+// A substep of a small grid clears some twenty arrays of a few KB: a launch
+// each, 5 us apart, was 60 us of it.  16 bytes per lane; the remainder of a
+// range by its first lanes.
+__global__ __launch_bounds__(256) void k_fill_ranges(FillArgs A) {
+  const int64_t t0 = blockIdx.x * 256ll + threadIdx.x, stride = gridDim.x * 256ll;
+  for (int r = 0; r < A.n; ++r) {
+    const uint32_t v = A.f[r].value ? ~0u : 0u;
+    const int64_t n16 = A.f[r].bytes / 16, left = A.f[r].bytes % 16;
+    uint4* const p = reinterpret_cast<uint4*>(A.f[r].p);
+    for (int64_t t = t0; t < n16; t += stride) p[t] = make_uint4(v, v, v, v);
+    if (t0 < left) reinterpret_cast<uint8_t*>(p + n16)[t0] = (uint8_t)v;
+  }
+}
+}  // namespace
+
+void fill_ranges(hipStream_t st, std::initializer_list<Fill> list) {
+  FillArgs A = {};
+  int64_t most = 0;
+  auto launch = [&] {
+    if (A.n == 0) return;
+    const int64_t nb = std::max<int64_t>(1, std::min<int64_t>(4096, (most / 16 + 255) / 256));
+    hipLaunchKernelGGL(k_fill_ranges, dim3((unsigned)nb), dim3(256), 0, st, A);
+    WC_LAUNCH_CHECK();
+    A.n = 0;
+    most = 0;
+  };
+  for (const Fill& f : list) {
+    if (f.bytes <= 0) continue;
+    A.f[A.n++] = f;
+    most = std::max(most, f.bytes);
+    if (A.n == kMaxFills) launch();
+  }
+  launch();
 }
 
 }  // namespace wc

@@ -2133,12 +2133,18 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const doub
                         hipMemcpyHostToDevice, st));
   // (the sub-tile sweeps write no slot outside their units' steps: those
   // keep this zero, and the factor's in zf)
-  WC_HIP(hipMemsetAsync(P.zb.p, 0, sizeof(double) * P.ncell, st));
   P.progress.ensure(8);
   P.tdot.ensure(4 * P.ntiles);
+  P.rsum.ensure(P.ncell * sizeof(RowSum) / sizeof(double));
+  const int64_t vec = sizeof(double) * P.ncell;
+  if (pcg_in_passes(P)) P.zc.ensure(P.ncell / 8);  // likewise zero where no unit runs
   // tickets and the abort flag start at zero (the abort flag is cleared
-  // again by each factor, not by the applies: once set it stays set)
-  WC_HIP(hipMemsetAsync(P.progress.p, 0, sizeof(int) * 8, st));
+  // again by each factor, not by the applies: once set it stays set); the
+  // row summaries are written at the DOFs' slots only
+  fill_ranges(st, {{P.zb.p, vec, 0},
+                   {P.progress.p, sizeof(int) * 8, 0},
+                   {P.rsum.p, (int64_t)sizeof(RowSum) * P.ncell, 0},
+                   {P.zc.p, pcg_in_passes(P) ? vec / 8 : 0, 0}});
   P.ticks_zero = true;
   P.mail_word = 0;
   BoxArgs A;
@@ -2165,10 +2171,8 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const doub
   A.cb = reinterpret_cast<Cell*>(P.cb.p);
   A.coef = P.coef.p;
   A.fin = reinterpret_cast<FacIn*>(P.fin.p);
-  // row summaries at the DOFs' slots (zeros elsewhere), then the fill
-  P.rsum.ensure(P.ncell * sizeof(RowSum) / sizeof(double));
+  // row summaries at the DOFs' slots, then the fill
   RowSum* rs = reinterpret_cast<RowSum*>(P.rsum.p);
-  WC_HIP(hipMemsetAsync(rs, 0, sizeof(RowSum) * P.ncell, st));
   hipLaunchKernelGGL(k_row_sums, dim3((unsigned)std::min<int64_t>(4096, blocks(g.nnode, 256))),
                      dim3(256), 0, st, A, rs);
   WC_LAUNCH_CHECK();
@@ -2181,11 +2185,6 @@ void sweep_prepare(hipStream_t st, SweepPlan& P, const GridSystem& G, const doub
   P.xf15.ensure(P.ncell / 16);
   P.xf0.ensure(P.ncell / 16);
   face_cols<double>(st, P.ncell, P.coef.p + 4 * P.ncell, P.cf15.p, nullptr);
-  if (pcg_in_passes(P)) {
-    // both columns of the preconditioned vector: zero where no unit runs, as zb
-    P.zc.ensure(P.ncell / 8);
-    WC_HIP(hipMemsetAsync(P.zc.p, 0, sizeof(double) * (P.ncell / 8), st));
-  }
   WC_HIP(hipStreamSynchronize(st));  // 'order' and 'order_sub' must outlive their copies
   P.valid = true;
 }
@@ -2205,8 +2204,8 @@ static SweepArgs<V> sweep_args(SweepPlan& P) {
 
 void sweep_factor(hipStream_t st, SweepPlan& P, double tau, double mdr) {
   int* tick = P.progress.p;
-  WC_HIP(hipMemsetAsync(tick, 0, sizeof(int) * 8, st));
-  WC_HIP(hipMemsetAsync(P.zf.p, 0xFF, sizeof(double) * P.ncell, st));
+  fill_ranges(st, {{tick, sizeof(int) * 8, 0},
+                   {P.zf.p, (int64_t)sizeof(double) * P.ncell, 0xFF}});
   SweepArgs<double> S = sweep_args<double>(P);
   S.fin = reinterpret_cast<const FacIn*>(P.fin.p);
   S.cf = reinterpret_cast<Cell*>(P.cf.p);
@@ -2234,8 +2233,8 @@ void sweep_narrow(hipStream_t st, SweepPlan& P) {
   P.rb32.ensure(P.ncell);
   P.sb32.ensure(P.ncell);
   P.bb.ensure(P.ncell);
-  WC_HIP(hipMemsetAsync(P.zf32.p, 0, sizeof(float) * P.ncell, st));  // as in sweep_prepare
-  WC_HIP(hipMemsetAsync(P.zb32.p, 0, sizeof(float) * P.ncell, st));
+  const int64_t vec = sizeof(float) * P.ncell;
+  fill_ranges(st, {{P.zf32.p, vec, 0}, {P.zb32.p, vec, 0}});  // as in sweep_prepare
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cf.p,
                      P.cf32.p, nrec);
   hipLaunchKernelGGL(k_narrow_box, dim3(blocks(nrec, 256)), dim3(256), 0, st, P.cb.p,
