@@ -7,8 +7,10 @@
 // k-pencils; a workgroup walks its tile's local hyperplanes i'+j'+k = w, one
 // step per w, passing the newest value of each pencil to its +x/+y
 // neighbours through LDS.  Values on a tile's low faces come from the
-// upstream tiles (a-1, b) and (a, b-1), which run ahead.  The output array is
-// filled with a NaN sentinel before the sweep and every cell is written
+// upstream tiles (a-1, b) and (a, b-1), which run ahead.  (The default form,
+// k_sweep_sub, has one wave per 8x8 quarter of a tile, and its units exchange
+// face values through mail records instead of the output; the factor and
+// k_sweep use the output.)  The output array is filled with a NaN sentinel before the sweep and every cell is written
 // exactly once with a single device-coherent (agent-scope atomic) store, so
 // a consumer knows a value is final when it no longer reads the sentinel.
 // A dedicated face wave per workgroup reads the upstream face values a batch
@@ -1583,8 +1585,10 @@ __global__ __launch_bounds__(SweepBlock<KIND>::value) void k_sweep(SweepArgs<V> 
 // cache lines instead of 4.)
 // Forward / backward sweep, us: 256^3 FP32 159 / 169 -> 128 / 129, FP64
 // 212 / 199 -> 162 / 171; 128^3 FP32 63 / 70 -> 56 / 58; 32^3 FP64 30 / 32 ->
-// 25 / 27.  A unit without upstream runs a step in 0.072 us (0.117 before the
-// records were read a batch ahead); a hop between units costs 1.8-2.4 us.
+// 25 / 27; with units running their own steps over a box without empty rows
+// 256^3 112 / 117 and 143 / 153, 128^3 46 / 47, 32^3 16 / 18.  A unit without
+// upstream runs a step in 0.072 us (0.117 before the records were read a batch
+// ahead); a hop between units costs 1.8-2.4 us.
 constexpr int kS = 8;             // sub-tile edge (pencils)
 constexpr int kNB = 4;            // steps per batch
 constexpr int kSubPlanes = 8;     // exchange planes (step % 8), two batches
