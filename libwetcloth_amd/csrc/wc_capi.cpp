@@ -1604,7 +1604,9 @@ namespace {
 wc_status check_ijk(int64_t n, const int32_t* ijk, int32_t ni, int32_t nj, int32_t nk) {
   if (n > 0 && !ijk) return WC_ERR_ARG;
   if (ni <= 0 || nj <= 0 || nk <= 0) return n > 0 ? WC_ERR_ARG : WC_OK;
-  if ((int64_t)ni * nj * nk >= 0x7FFFFFFFll) return WC_ERR_ARG;
+  // (divided, not multiplied: the product of three extents may pass 2^63)
+  const int64_t most = 0x7FFFFFFEll;  // cells of the grid
+  if (ni > most / nj || (int64_t)ni * nj > most / nk) return WC_ERR_ARG;
   for (int64_t f = 0; f < n; ++f)
     if (ijk[3 * f] < 0 || ijk[3 * f] >= ni || ijk[3 * f + 1] < 0 || ijk[3 * f + 1] >= nj ||
         ijk[3 * f + 2] < 0 || ijk[3 * f + 2] >= nk)
