@@ -369,6 +369,16 @@ wc_status wc_kernel_stats(const wc_ctx* ctx, int32_t kernel, double* ms,
 
 /* ---- robertbridson::PCGSolver<double> on a host CSR matrix ---- */
 
+/* Memory that outlives a call (no reference counterpart): a *_csr call below
+ * (the noalloc form apart) leaves its stream and device buffers, with 9 KB of
+ * pinned host memory, for the next one instead of creating them again: at most
+ * two idle workspaces per GPU of at most 256 MiB of device memory each, none
+ * of a larger call or of one that failed.  They are freed by this function, or
+ * when an allocation of this library fails, and hold nothing of a call's data
+ * that a later one reads.  Calls in progress in other threads keep theirs.
+ * A program whose other allocators need that memory calls it first. */
+wc_status wc_release_workspaces(void);
+
 /* Literal drop-in for PCGSolver<double>::solve(matrix, rhs, result,
  * residual_out, iterations_out) (PCGSolver/PCGSolver.h:260-308) after
  * set_solver_parameters(tol, maxit) (:249).  The CSR is

@@ -140,6 +140,7 @@ def lib():
             getattr(L, nm).argtypes = [vp, C.c_char_p]
         L.wc_apply_preconditioner.argtypes = [vp, _dp, _dp]
         L.wc_system_multiply.argtypes = [vp, _dp, _dp]
+        L.wc_release_workspaces.argtypes = []
         L.wc_pcg_solve_csr.argtypes = [C.c_int64, _u32p, _u32p, _dp, _dp, _dp, C.c_double,
                                        C.c_int32, _dp, _i32p]
         L.wc_pcg_solve_csr_noalloc.argtypes = L.wc_pcg_solve_csr.argtypes
@@ -510,6 +511,12 @@ class Scene:
 
 def _csr(rs, col):
     return (np.ascontiguousarray(rs, dtype=np.uint32), np.ascontiguousarray(col, dtype=np.uint32))
+
+
+def release_workspaces():
+    """Frees the idle workspaces that the *_csr calls keep for the next one (at
+    most two of 256 MiB per GPU)."""
+    _check(lib().wc_release_workspaces())
 
 
 def pcg_solve_csr(rs, col, val, rhs, tol=1e-8, maxit=500, no_alloc=False):

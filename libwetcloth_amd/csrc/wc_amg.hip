@@ -586,34 +586,10 @@ void smooth(hipStream_t st, const AmgHier& H, const AmgLevel& L, const double* b
 }  // namespace
 
 void AmgHier::release() {
-  for (int l = 0; l < kAmgMaxLevels; ++l) {
-    AmgLevel& L = this->L[l];
-    L.col.release();
-    L.len.release();
-    L.val.release();
-    L.ijk.release();
-    L.red.release();
-    L.parent.release();
-    L.kids.release();
-    L.x.release();
-    L.b.release();
-    L.r.release();
-    L.crow.release();
-    L.cpos.release();
-    L.cdiag.release();
-    L.ccol.release();
-    L.cval.release();
-    L.clen.release();
-    L.n = 0;
-    L.nred = 0;
-  }
+  each([](auto& b) { b.release(); });
+  for (AmgLevel& l : L) l.n = l.nred = 0;
   nl = 0;
   compact = false;
-  cmin.release();
-  flag.release();
-  scan_tmp.release();
-  nred.release();
-  err.release();
 }
 
 // GeometricLevelGen.h:186-249

@@ -1233,10 +1233,9 @@ struct CsrUpload {
     A.val = val.p;
     A.nnz_slots = nnz;
   }
-  void release() {
-    rowptr.release();
-    col.release();
-    val.release();
+  template <class F>
+  void each(F&& f) {
+    f(rowptr), f(col), f(val);
   }
 };
 
@@ -1244,10 +1243,11 @@ struct CsrUpload {
 // and freeing them took half of a call on 245,666 rows (72 allocations and
 // frees 5 ms, the stream 0.8 ms of 11 ms), so a call hands its session back to
 // a pool, at most kIdleSessions of at most kIdleBytes each per device; a
-// larger one is freed with its call, and the idle ones when an allocation of
-// any context or call fails (drop_idle_sessions, then tried once more).  A
-// session is used by one call at a time, with every array written by the call
-// itself; one whose call failed is not kept.
+// larger one is freed with its call, and the idle ones by
+// wc_release_workspaces or when an allocation of any context or call fails
+// (drop_idle_sessions, then tried once more).  A session is used by one call
+// at a time, with every array written by the call itself; one whose call
+// failed is not kept.
 struct FreeSession {
   hipStream_t st = nullptr;
   int device = 0;
@@ -1256,31 +1256,43 @@ struct FreeSession {
   wc::AmgHier amg;
   wc::DevBuf<int32_t> ijk;
   wc::DevBuf<double> in, out;
+  unsigned long long id = 0;  // of an idle one: the number of csr.rowptr's allocation
   FreeSession() { WC_HIP(hipStreamCreateWithFlags(&st, hipStreamNonBlocking)); }
   ~FreeSession() {
     if (st) (void)hipStreamSynchronize(st);
-    csr.release();
+    each([](auto& b) { b.release(); });
     work.release();
-    amg.release();
-    ijk.release();
-    in.release();
-    out.release();
     if (st) (void)hipStreamDestroy(st);
   }
-  // upper bound of the device bytes held: the arrays are sized by rows or by
-  // stored entries, and no call allocates others
-  size_t held() const {
-    size_t b = 4 * (csr.rowptr.cap + csr.col.cap + work.tpos.cap + work.level.cap +
-                    work.lvl_count.cap + work.lvl_cursor.cap + work.lvl_list.cap + ijk.cap +
-                    amg.cmin.cap + amg.flag.cap) +
-               8 * (csr.val.cap + work.invdiag.cap + work.adiag.cap + work.lv.cap + work.r.cap +
-                    work.z.cap + work.s.cap + work.x.cap + in.cap + out.cap);
-    for (const wc::AmgLevel& L : amg.L)
-      b += 4 * (L.col.cap + L.len.cap + L.ijk.cap + L.parent.cap + L.kids.cap + L.crow.cap +
-                L.cpos.cap + L.ccol.cap) +
-           8 * (L.val.cap + L.x.cap + L.b.cap + L.r.cap + L.cval.cap + L.cdiag.cap) +
-           L.red.cap + L.clen.cap;
+  template <class F>
+  void each(F&& f) {  // every device buffer
+    csr.each(f);
+    work.each(f);
+    amg.each(f);
+    f(ijk), f(in), f(out);
+  }
+  size_t held() {  // device bytes
+    size_t b = 0;
+    each([&](auto& d) { b += d.bytes(); });
     return b;
+  }
+  // The runtime numbers allocations and does not use a number twice, so an
+  // idle session whose buffer no longer has its number was ended from outside
+  // (hipDeviceReset), its stream and pinned memory with it.
+  static unsigned long long allocation(const void* p) {
+    unsigned long long v = 0;
+    if (hipPointerGetAttribute(&v, HIP_POINTER_ATTRIBUTE_BUFFER_ID,
+                               (hipDeviceptr_t) const_cast<void*>(p)) == hipSuccess)
+      return v;
+    (void)hipGetLastError();
+    return 0;
+  }
+  bool alive() const { return id != 0 && allocation(csr.rowptr.p) == id; }
+  // gives everything up without a call to the runtime
+  void forget() {
+    each([](auto& b) { b.forget(); });
+    work.host_scal = work.host_part = work.host_part_dev = nullptr;
+    st = nullptr;
   }
 };
 
@@ -1305,7 +1317,10 @@ void drop_idle_sessions() {
     std::lock_guard<std::mutex> lock(P.mu);
     idle.swap(P.idle);
   }
-  for (FreeSession* f : idle) delete f;
+  for (FreeSession* f : idle) {
+    if (!f->alive()) f->forget();
+    delete f;
+  }
 }
 }  // namespace wc
 
@@ -1320,12 +1335,19 @@ class Session {
     {
       SessionPool& P = session_pool();
       std::lock_guard<std::mutex> lock(P.mu);
-      for (size_t k = 0; k < P.idle.size(); ++k)
-        if (P.idle[k]->device == dev) {
-          s_ = P.idle[k];
-          P.idle.erase(P.idle.begin() + (ptrdiff_t)k);
-          break;
+      for (size_t k = 0; k < P.idle.size() && !s_;) {
+        if (P.idle[k]->device != dev) {
+          ++k;
+          continue;
         }
+        s_ = P.idle[k];
+        P.idle.erase(P.idle.begin() + (ptrdiff_t)k);
+        if (!s_->alive()) {
+          s_->forget();
+          delete s_;
+          s_ = nullptr;
+        }
+      }
     }
     if (!s_) {
       s_ = new FreeSession;
@@ -1333,7 +1355,8 @@ class Session {
     }
   }
   ~Session() {
-    if (keep_ && s_->held() <= kIdleBytes) {
+    if (keep_ && s_->held() <= kIdleBytes &&
+        (s_->id = FreeSession::allocation(s_->csr.rowptr.p)) != 0) {
       SessionPool& P = session_pool();
       std::lock_guard<std::mutex> lock(P.mu);
       size_t here = 0;
@@ -1405,6 +1428,11 @@ wc_status check_csr(int64_t n, const uint32_t* rs, const uint32_t* col) {
 }  // namespace
 
 extern "C" {
+
+wc_status wc_release_workspaces(void) {
+  wc::drop_idle_sessions();
+  return WC_OK;
+}
 
 wc_status wc_pcg_solve_csr(int64_t n, const uint32_t* rowstart,
                            const uint32_t* col, const double* val,

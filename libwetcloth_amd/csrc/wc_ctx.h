@@ -67,10 +67,15 @@ struct DevBuf {
   }
   void release() {
     if (p && !lent) (void)hipFree(p);
+    forget();
+  }
+  // the buffer is given up without a call to the runtime
+  void forget() {
     p = nullptr;
     cap = 0;
     lent = false;
   }
+  size_t bytes() const { return lent ? 0 : cap * sizeof(T); }
 };
 
 // Matrix in "padded CSR": row i holds len[i] sorted entries starting at
@@ -224,6 +229,12 @@ struct PcgWork {
   double host_scal_own[8] = {};
   double* host_part = nullptr;  // mapped host memory, kHostParts |r| partials
   double* host_part_dev = nullptr;  // its device address
+  // every buffer of its own (the sweep plan's apart)
+  template <class F>
+  void each(F&& f) {
+    f(invdiag), f(adiag), f(lv), f(r), f(z), f(s), f(x), f(partial), f(scal);
+    f(tpos), f(flags), f(level), f(lvl_count), f(lvl_cursor), f(lvl_list);
+  }
   void release();
 };
 
@@ -250,6 +261,11 @@ struct AmgLevel {
   DevBuf<uint32_t> ccol;        // [s * n + p]
   DevBuf<double> cval;
   DevBuf<uint8_t> clen;
+  template <class F>
+  void each(F&& f) {  // every buffer
+    f(col), f(len), f(val), f(ijk), f(red), f(parent), f(kids), f(x), f(b), f(r);
+    f(crow), f(cpos), f(cdiag), f(ccol), f(cval), f(clen);
+  }
 };
 constexpr int kAmgMaxLevels = 16;
 struct AmgHier {
@@ -259,6 +275,11 @@ struct AmgHier {
   DevBuf<uint32_t> cmin, flag, scan_tmp;
   DevBuf<uint32_t> nred;        // red rows of each level, on the device
   DevBuf<int> err;
+  template <class F>
+  void each(F&& f) {  // every buffer, the levels' included
+    for (AmgLevel& l : L) l.each(f);
+    f(cmin), f(flag), f(scan_tmp), f(nred), f(err);
+  }
   void release();
 };
 // builds the levels of A (level 0 rows as given, DOF cell coordinates ijk

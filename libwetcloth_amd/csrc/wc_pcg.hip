@@ -832,21 +832,7 @@ void KTimer::release() {
 void PcgWork::release() {
   timer.release();
   sweep.release();
-  invdiag.release();
-  adiag.release();
-  flags.release();
-  lv.release();
-  r.release();
-  z.release();
-  s.release();
-  x.release();
-  partial.release();
-  scal.release();
-  tpos.release();
-  level.release();
-  lvl_count.release();
-  lvl_cursor.release();
-  lvl_list.release();
+  each([](auto& b) { b.release(); });
   if (host_scal && host_scal != host_scal_own) (void)hipHostFree(host_scal);
   host_scal = nullptr;
   if (host_part) (void)hipHostFree(host_part);
