@@ -1620,6 +1620,9 @@ wc_status wc_pcg_solve_csr_noalloc(int64_t n, const uint32_t* rowstart, const ui
   } catch (const HipError& e) {
     if (d && d->st) (void)hipStreamSynchronize(d->st);
     return hip_fail(nullptr, e);
+  } catch (const std::bad_alloc&) {  // (of the level schedule's host lists)
+    if (d && d->st) (void)hipStreamSynchronize(d->st);
+    return fail(nullptr, WC_ERR_NOMEM, "host allocation failed");
   }
   if (residual_out) *residual_out = res;
   if (iters_out) *iters_out = it;
