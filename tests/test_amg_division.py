@@ -1,6 +1,8 @@
 """The coarsest AMG solve divides by a row's diagonal from its reciprocal: two
-fma refinements of a * RN(1 / d).  Restated with exact rational arithmetic for
-the fmas, the quotient is the correctly rounded one."""
+fma refinements of a * RN(1 / d).  This checks the method, not the kernel: restated
+with exact rational arithmetic for the fmas, the quotient is the correctly
+rounded one.  The device's quotients are compared with true ones, inside and
+outside the method's range, in test_gpu_amg.py (test_coarsest_quotients)."""
 import random
 import struct
 from fractions import Fraction

@@ -191,3 +191,120 @@ def test_amgpcg_not_converged_after_maxit(oracle, wc):
     assert not ok_r and not ok and it == it_r == 1
     assert np.abs(x - x_r).max() <= 1e-10 * np.abs(x_r).max()
     assert abs(res - res_r) <= 1e-8 * res_r
+
+
+def cells_system(blocks, tank, seed):
+    """Isolated blocks of cells (lists of cells, coupled to face neighbours of
+    the same block only) and a tank[0] x tank[1] x tank[2] tank beside them: CSR,
+    cells and grid."""
+    rng = np.random.default_rng(seed)
+    groups = list(blocks)
+    if tank:
+        x0 = max((c[0] for g in groups for c in g), default=-4) + 4
+        x0 += x0 % 2
+        groups.append([(x0 + i, j, k) for k in range(tank[2]) for j in range(tank[1])
+                       for i in range(tank[0])])
+    where, cells = {}, []
+    for q, g in enumerate(groups):
+        for c in g:
+            where[c] = (len(cells), q)
+            cells.append(c)
+    n = len(cells)
+    W = {}
+    for c, (a, q) in where.items():
+        for d in ((1, 0, 0), (0, 1, 0), (0, 0, 1)):
+            o = where.get(tuple(c[t] + d[t] for t in range(3)))
+            if o and o[1] == q:
+                W[(a, o[0])] = W[(o[0], a)] = -rng.uniform(0.1, 1.0)
+    diag = rng.uniform(0.1, 0.5, n)
+    for (a, _), w in W.items():
+        diag[a] -= w
+    for a in range(n):
+        W[(a, a)] = diag[a]
+    rows, cols = np.array(sorted(W)).T
+    val = np.array([W[k] for k in zip(rows.tolist(), cols.tolist())])
+    rs = np.zeros(n + 1, dtype=np.uint32)
+    np.cumsum(np.bincount(rows, minlength=n), out=rs[1:])
+    ijk = np.array(cells, dtype=np.int32)
+    return rs, cols.astype(np.uint32), val, ijk, tuple(int(v) for v in ijk.max(0) + 1)
+
+
+def lattice(count, parity, unit):
+    """count cells of an 18 x 18 x ... lattice of unit's multiples, of one parity
+    of i + j + k, no two of them neighbours."""
+    out = []
+    for t in range(10 ** 6):
+        c = (t % 18, t // 18 % 18, t // 324)
+        if sum(c) % 2 == parity:
+            out.append(tuple(unit * a for a in c))
+            if len(out) == count:
+                return out
+
+
+@pytest.mark.parametrize("levels", [1, 2])
+@pytest.mark.parametrize("red", [0, 1])
+@pytest.mark.parametrize("count", [1950, 2049, 3000])
+def test_coarsest_level_of_one_colour(oracle, wc, count, red, levels):
+    """A coarsest level most of whose rows are of one colour (up to 2048 of a
+    colour take the kernel with two rows of a colour per thread, more the other
+    one), as the only level and as the coarser of two."""
+    if levels == 1:
+        blocks, tank = [[c] for c in lattice(count, red, 1)], (6, 5, 4)
+    else:  # two cells per coarse cell, and a coarse parity
+        blocks = [[c, (c[0] + 1, c[1], c[2])] for c in lattice(count, red, 2)]
+        tank = (12, 10, 8)
+    rs, col, val, ijk, dims = cells_system(blocks, tank, seed=count)
+    sizes = oracle.amg_levels(rs, col, val, ijk, dims)
+    assert len(sizes) == levels and sizes[-1] == count + 120 <= 4096
+    r = np.random.default_rng(count + 1).standard_normal(len(rs) - 1)
+    assert np.array_equal(wc.amg_apply_csr(rs, col, val, ijk, dims, r),
+                          oracle.amg_vcycle(rs, col, val, ijk, dims, r))
+
+
+@pytest.mark.parametrize("span", [390, 398, 402, 500])
+def test_coarsest_quotients(wc, span):
+    """Rows of a diagonal alone: one V-cycle is b / d, correctly rounded, for
+    exponents inside, across and far outside the range in which the kernel
+    divides by a reciprocal, and with zeros among them."""
+    rng = np.random.default_rng(span)
+    n = 4096
+    ijk = np.array([(i, j, k) for k in range(16) for j in range(16) for i in range(16)],
+                   dtype=np.int32)
+    for zeros in (False, True):
+        b, d = (rng.uniform(1, 2, n) * 2.0 ** rng.integers(-span, span + 1, n) *
+                rng.choice((-1, 1), n) for _ in range(2))
+        ones = rng.integers(0, n, n // 3)  # mantissas of ones: the hardest reciprocals
+        bits = d.view(np.uint64)
+        bits[ones] |= np.uint64((1 << 52) - 1) - (np.uint64(1) << rng.integers(0, 6, n // 3).astype(np.uint64))
+        if zeros:
+            b[rng.integers(0, n, 200)] = 0.0
+            b[rng.integers(0, n, 20)] = -0.0
+            b[rng.integers(0, n, 20)] = 5e-324
+            d[rng.integers(0, n, 100)] = 0.0  # the value of such a row is 0
+        q = np.divide(b, d, out=np.zeros(n), where=d != 0)
+        z = wc.amg_apply_csr(np.arange(n + 1), np.arange(n), d, ijk, (16, 16, 16), b)
+        assert np.isfinite(q).all()
+        assert np.array_equal(z, q), np.flatnonzero(z != q)[:8]
+
+
+def test_coarsest_rows_out_of_range(oracle, wc):
+    """A coupled system whose waves mix rows inside and outside that range, rows
+    whose diagonal is zero and rows that store none."""
+    rs, col, val, ijk, dims = cells_system([], (16, 16, 12), seed=3)
+    rng = np.random.default_rng(4)
+    n = len(rs) - 1
+    rows = np.repeat(np.arange(n), np.diff(rs.astype(np.int64)))
+    scale = np.ones(n)
+    scale[rng.integers(0, n, 300)] = 2.0 ** 450
+    scale[rng.integers(0, n, 300)] = 2.0 ** -450
+    val *= scale[rows]  # (row by row: the solution keeps its size)
+    b = rng.standard_normal(n) * scale
+    b[rng.integers(0, n, 300)] = 0.0
+    b[rng.integers(0, n, 50)] = 1e-310
+    val[(rows == col) & np.isin(rows, rng.integers(0, n, 40))] = 0.0
+    keep = ~((rows == col) & np.isin(rows, rng.integers(0, n, 40)))
+    rs = np.concatenate([[0], np.cumsum(np.bincount(rows[keep], minlength=n))])
+    z = wc.amg_apply_csr(rs, col[keep], val[keep], ijk, dims, b)
+    ref = oracle.amg_vcycle(rs, col[keep], val[keep], ijk, dims, b)
+    assert np.isfinite(ref).all() and (ref == 0).sum() >= 40
+    assert np.array_equal(z, ref)

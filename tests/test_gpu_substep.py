@@ -202,8 +202,10 @@ def test_cfl_substep_split(oracle, wc):
 @pytest.mark.parametrize("dims", [(4, 4, 4), (12, 4, 8), (20, 12, 8), (36, 16, 16)])
 def test_grid_cleared_between_substeps(wc, dims):
     """A context that has stepped particles elsewhere steps as a fresh one: no
-    array of the grid keeps values (1, 6, 30 and 144 buckets: flag arrays whose
-    length is no multiple of the clearing kernel's 16 bytes, and one that is).
+    array of the grid keeps values (125, 210, 378 and 832 buckets with the ghost
+    layers: flag arrays whose length is no multiple of the clearing kernel's 16
+    bytes, and one that is; the last bytes are ghost buckets that no particle
+    reaches, so test_gpu_fill.py covers the kernel's remainders).
     The order of the FP64 sums differs from run to run, so the velocities agree
     to rounding (1e-16 per sum, grown by less than 1e4 in the solve at 1e-12)."""
     h = 1.0 / max(dims)
