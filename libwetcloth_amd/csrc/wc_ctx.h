@@ -176,7 +176,8 @@ struct SweepPlan {
   // columns (li = 15, then li = 0), a second direction and its columns
   DevBuf<double> zc, s2, sc2;
   // The forward sweep's ticket counter is zero: the sweeps zero each
-  // other's counter, so only the first apply after the plan needs a clear.
+  // other's counter, so only the first apply after the plan (or after one
+  // that failed between its passes) needs a clear.
   bool ticks_zero = false;
   void release();
 };
@@ -545,7 +546,8 @@ struct DotParts {
 DotParts box_spmv_dot(hipStream_t st, SweepPlan& P, const double* x, double* y,
                       double* partial, int nblocks, bool faces_ready = false);
 DotParts box_spmv32_dot(hipStream_t st, SweepPlan& P, const float* x, float* y,
-                        double* partial, int nblocks, bool faces_ready = false);// PCG's residual update inside the forward sub-tile sweep that applies the
+                        double* partial, int nblocks, bool faces_ready = false);
+// PCG's residual update inside the forward sub-tile sweep that applies the
 // preconditioner to it: r -= y alpha, alpha = scal[rho] / (the sum of d) left
 // in scal[alpha], and each unit's |r|_inf in rpart (-2 for the first unit's
 // where the abort flag is set; P.nua * P.nub entries, mapped host memory).

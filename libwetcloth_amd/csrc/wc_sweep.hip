@@ -2300,10 +2300,14 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
   // kernel of its own: a runtime fill waited ~15 us longer to start.
   int* tick = P.progress.p;
   if (!P.ticks_zero) WC_HIP(hipMemsetAsync(tick, 0, sizeof(int) * 2, st));
+  // Until both passes are launched: the forward one alone leaves its counter at
+  // its units' number, from which a next apply would read past the order.
+  P.ticks_zero = false;
   static_assert(kThreads % 16 == 0, "slots come in whole 16-byte words");
   const bool sub = P.sub;
   // the sub-tile sweeps keep their own records as sentinels between passes
   V* const mail = sub ? ready_mail<V>(st, P) : nullptr;
+  if (sub) P.mail_word = 0;  // (likewise)
   if (!sub && !cleared)  // else the PCG update before this apply has filled zf
     fill_sentinel(st, zf, (int64_t)sizeof(V) * P.ncell / 16);
   SweepArgs<V> S = sweep_args<V>(P);
@@ -2368,6 +2372,7 @@ static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, co
     hipLaunchKernelGGL((k_sweep<K_BWD, V>), dim3(P.ntiles), dim3(SweepBlock<K_BWD>::value), 0, st, S);
   WC_LAUNCH_CHECK();
   P.ticks_zero = true;
+  if (sub) P.mail_word = (int)sizeof(V);
   if (timer) {
     timer->add(KTimer::SWEEP_FWD, ndof, e0, e1);
     timer->add(KTimer::SWEEP_BWD, ndof, e2, timer->mark(st));
