@@ -660,7 +660,6 @@ void amg_build(hipStream_t st, AmgHier& H, const DevCsr& A, const int32_t* ijk, 
       L.x.ensure((size_t)L.n);
       L.b.ensure((size_t)L.n);
     }
-    if (l + 1 < H.nl) L.r.ensure((size_t)L.n);
     // colour-ordered rows: red positions by a scan of the red flags
     H.flag.ensure((size_t)L.n + 1);
     hipLaunchKernelGGL(k_amg_redflag, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.n, L.red.p,
@@ -698,6 +697,8 @@ void amg_build(hipStream_t st, AmgHier& H, const DevCsr& A, const int32_t* ijk, 
     throw HipError{hipErrorInvalidValue, "AMG levels: two DOFs share a cell", __FILE__, __LINE__};
   for (int l = 0; l < H.nl; ++l) H.L[l].nred = nred[l];
   H.compact = (herr & 4) == 0;
+  // the residual as a vector of its own (k_amg_resid_restrict stores none)
+  for (int l = 0; l + 1 < H.nl && !H.compact; ++l) H.L[l].r.ensure((size_t)H.L[l].n);
 }
 
 bool amg_spmv(hipStream_t st, AmgHier& H, const double* x, double* y) {

@@ -252,7 +252,8 @@ struct AmgLevel {
   DevBuf<uint32_t> parent;      // the coarse DOF of each DOF (every level but the last)
   DevBuf<uint32_t> kids;        // 8 per DOF: its fine children ascending, ~0u after them
                                 // (every level but the first)
-  DevBuf<double> x, b, r;       // V-cycle vectors (x, b of level 0 are the caller's)
+  DevBuf<double> x, b;          // V-cycle vectors (those of level 0 are the caller's)
+  DevBuf<double> r;             // the residual, where the rows are not colour-ordered
   // the rows again, ordered by colour (red rows ascending, then black rows
   // ascending) with each row's entries in their order as 7 planes of n, so a
   // colour's smoothing reads only its own rows, coalesced
