@@ -7,11 +7,12 @@
 // earlier levels.  One launch runs all levels of a pass: its waves take 64
 // rows of one level at a time by ticket, in level order, and wait for the
 // values they read (a matrix whose pattern is not symmetric is run with one
-// launch per level).  Each row is computed in gather ("left-looking") form, applying exactly the updates the reference's
-// column-sweeping loops apply to it and in the same order (ascending column),
-// so the factor and the preconditioned vector are bitwise the sequential
-// ones.  Inner products are two-stage block reductions in FP64 with a fixed
-// order (deterministic, but not the reference's SIMD order).
+// launch per level).  Each row is computed in gather ("left-looking") form,
+// applying exactly the updates the reference's column-sweeping loops apply to
+// it and in the same order (ascending column), so the factor and the
+// preconditioned vector are bitwise the sequential ones.  Inner products are
+// two-stage block reductions in FP64 with a fixed order (deterministic, but
+// not the reference's SIMD order).
 #include <math.h>
 
 #include <algorithm>
@@ -1085,18 +1086,6 @@ static double read_scal(hipStream_t st, PcgWork& w, int slot) {
   return w.host_scal[slot];
 }
 
-// The residual of the last update: the max of its block partials, which
-// the update kernel wrote into mapped host memory with the sweeps' abort
-// flag, once the event recorded after it has completed (work enqueued after
-// the event may still be running).
-// The update kernel's |r|_inf partials arrive in mapped host memory, each
-// block's over the -1 the host left there: a max (>= 0), or -2 from block 0
-// when the sweeps' abort flag is set.  Polling them instead of waiting on
-// an event keeps the event's marker packet, ~5.6 us of idle GPU per
-// iteration, out of the stream.  After 10 ms (an iteration takes well
-// under one) the stream is queried as well, which enqueues a marker of its
-// own: a stream that failed, or finished without the partials, ends the
-// wait with an error.
 // Test hook ("debug_abort_sweeps"): the sweeps' abort flag set before the
 // loop, as a sweep whose bounded wait ran out would set it, so the solve
 // takes its error path (every kernel still runs to its end).
@@ -1108,7 +1097,16 @@ static void clear_residual(PcgWork& w) {
   for (int i = 0; i < kHostParts; ++i) w.host_part[i] = -1.0;
 }
 
-// nb: how many partials the update writes
+// The residual of the last update: the max of its nb |r|_inf partials (of
+// the update kernel's blocks, or of the units of the forward sweep that
+// updates r).  They arrive in mapped host memory, each over the -1 the host
+// left there: a max (>= 0), or -2 from the first when the abort flag of the
+// sweeps (or of the waiting passes) is set.  Polling them instead of waiting
+// on an event keeps the event's marker packet, ~5.6 us of idle GPU per
+// iteration, out of the stream.  After 10 ms (an iteration takes well
+// under one) the stream is queried as well, which enqueues a marker of its
+// own: a stream that failed, or finished without the partials, ends the
+// wait with an error.
 static double box_residual_max(hipStream_t st, PcgWork& w, int nb,
                                const char* abort_text = "pipelined MIC(0) sweep: a tile wait "
                                                         "exceeded its bound") {
@@ -1212,13 +1210,14 @@ struct FusedIter {
 
 // The PCG loop of PCGSolver::solve (PCGSolver.h:280-304) on box vectors: the
 // pipelined sweeps apply MIC(0) in place and the SpMV is the box stencil.
-// b is gathered into the box once and x scattered back once.  Each iteration
-// is the SpMV with the s . z partials, one update kernel (alpha, x, r and the
-// |r|_inf partials), then -- enqueued before the host has read the residual,
-// since they touch only s and the sweep outputs, which are dead once the
-// residual meets the tolerance -- the MIC(0) apply (whose backward sweep
-// also leaves the z . r partials, one per tile) and the update of s with
-// beta.
+// b is gathered into the box once and x scattered back once.  Small plans
+// (pcg_in_passes) run FusedIter's three launches per iteration.  Else an
+// iteration is the SpMV with the s . z partials, one update kernel (alpha, x,
+// r and the |r|_inf partials), then -- enqueued before the host has read the
+// residual, since they touch only s and the sweep outputs, which are dead
+// once the residual meets the tolerance -- the MIC(0) apply (whose backward
+// sweep also leaves the z . r partials, one per unit) and the update of s
+// with beta.
 static bool pcg_loop_box(hipStream_t st, PcgWork& w, int64_t ndof, const double* b,
                          double* x_dof, double tolr, int maxit, double* residual_out,
                          int* iters_out) {

@@ -10,9 +10,10 @@
 // upstream tiles (a-1, b) and (a, b-1), which run ahead.  (The default form,
 // k_sweep_sub, has one wave per 8x8 quarter of a tile, and its units exchange
 // face values through mail records instead of the output; the factor and
-// k_sweep use the output.)  The output array is filled with a NaN sentinel before the sweep and every cell is written
-// exactly once with a single device-coherent (agent-scope atomic) store, so
-// a consumer knows a value is final when it no longer reads the sentinel.
+// k_sweep use the output.)  The output array is filled with a NaN sentinel
+// before the sweep and every cell is written exactly once with a single
+// device-coherent (agent-scope atomic) store, so a consumer knows a value is
+// final when it no longer reads the sentinel.
 // A dedicated face wave per workgroup reads the upstream face values a batch
 // of steps ahead and re-reads only those that were not final yet.  Tiles are
 // claimed with a ticket counter in (a+b, a) order, so a tile only waits for
@@ -2292,12 +2293,17 @@ template <class V>
 static void apply_impl(hipStream_t st, SweepPlan& P, const V* r, const V* cf, const V* cb,
                        V* zf, V* zb, V* zc, KTimer* timer, int64_t ndof, bool cleared,
                        const ResidualUpdate<V>* U = nullptr) {
-  // Two ticket counters; the outputs start as the sentinel.  Each pass zeroes
-  // the other pass's counter, and the forward pass's rhs loader sets every
-  // slot of zb to the sentinel as it goes, so an apply clears only zf (just
-  // before the forward pass, which leaves it cache-resident for the face
-  // reads) and, after the plan or the factor, the counters.  The clear is a
-  // kernel of its own: a runtime fill waited ~15 us longer to start.
+  // Two ticket counters; each pass zeroes the other pass's.
+  // Sub-tile sweeps: the sentinels are the mail records', which each pass
+  // resets for the other, so an apply clears nothing.  zf and zb are written
+  // at the units' own steps only and must hold zeros at every other slot (the
+  // plan's, the factor's or sweep_narrow's; box vectors that borrow zf write
+  // zeros there too): the loaders and the SpMV read those slots.
+  // Tile sweeps: zf and zb are the sentinels.  The forward pass's rhs loader
+  // sets every slot of zb as it goes, so an apply clears only zf (just before
+  // the forward pass, which leaves it cache-resident for the face reads),
+  // unless the PCG update before it has.  The clear is a kernel of its own: a
+  // runtime fill waited ~15 us longer to start.
   int* tick = P.progress.p;
   if (!P.ticks_zero) WC_HIP(hipMemsetAsync(tick, 0, sizeof(int) * 2, st));
   // Until both passes are launched: the forward one alone leaves its counter at
@@ -2421,11 +2427,13 @@ static int spmv_run_of(const SweepPlan& P) {
 // Whether the PCG iteration's vector updates run inside the SpMV and the
 // sweeps: three launches instead of five.  That pays while launches and
 // latency bound the iteration; on large systems the updates' traffic costs the
-// sweeps as much as it saves.  us per iteration, five launches / three (FP64,
-// then mixed): 16^3 41.5 / 35.2, 43.7 / 38.5; 32^3 50.6 / 45.5, 50.8 / 45.7;
-// 64^3 78.1 / 72.9, 75.2 / 69.8; 96^3 102.9 / 97.4, 96.2 / 92.4; 128^3 (4000
-// tile steps) 135.4 / 127.7, 125.2 / 118.7; 192^3 (12000) 275 / 282, 203 / 206;
-// 256^3 468 / 472, 351 / 346.
+// sweeps about as much as it saves.  The line is drawn for both value types at
+// once, below the first size at which either was slower with three; what that
+// leaves is 5 us of 351 (mixed at 256^3).  us per iteration, five launches /
+// three (FP64, then mixed): 16^3 41.5 / 35.2, 43.7 / 38.5; 32^3 50.6 / 45.5,
+// 50.8 / 45.7; 64^3 78.1 / 72.9, 75.2 / 69.8; 96^3 102.9 / 97.4, 96.2 / 92.4;
+// 128^3 (4000 tile steps) 135.4 / 127.7, 125.2 / 118.7; 192^3 (12000) 275 /
+// 282, 203 / 206; 256^3 468 / 472, 351 / 346.
 bool pcg_in_passes(const SweepPlan& P) {
   return P.sub && P.spmv_win && (int64_t)P.ntiles * P.nsteps < 8192 &&
          P.nua * P.nub <= kHostParts;
@@ -2463,12 +2471,14 @@ static DotParts spmv_pcg(hipStream_t st, SweepPlan& P, const V* coef, const V* c
 }
 
 template <class V>
-static PcgUpdate<V> pcg_update(SweepPlan& P, const V* z, const Direction<V>& s, const Direction<V>& sn, double* scal,
-                               int rho_old, int rho_new, int alpha) {
+static PcgUpdate<V> pcg_update(SweepPlan& P, const V* z, const Direction<V>& s,
+                               const Direction<V>& sn, double* scal, int rho_old, int rho_new,
+                               int alpha) {
   const V* zc = reinterpret_cast<const V*>(P.zc.p);
-  return {z, zc, zc + P.ncell / 16, s.v, s.c15, s.c0, sn.v, sn.c15, sn.c0, P.xb.p, P.tdot.p, P.ndot,
-          scal, rho_old, rho_new, alpha};
+  return {z,     zc,      zc + P.ncell / 16, s.v,    s.c15, s.c0,    sn.v,    sn.c15,
+          sn.c0, P.xb.p, P.tdot.p,           P.ndot, scal,  rho_old, rho_new, alpha};
 }
+
 DotParts box_spmv_pcg(hipStream_t st, SweepPlan& P, const Direction<double>& s,
                       const Direction<double>& sn, double* y, double* scal, int rho_old,
                       int rho_new, int alpha) {
